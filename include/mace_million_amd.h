@@ -54,6 +54,16 @@ int mm_nl_scan_noalloc(const int* NN, long* rowptr, long N, mm_stream_t stream);
 int mm_nl_fill(const double* pos_sorted, const int* cell_sorted, long N, const double* box /* HOST [3] */,
                const int* ncell /* HOST [3] */, const int* cell_start, const int* cell_count, double r_cut2,
                int brute, const long* rowptr, int* send, mm_stream_t stream);
+/* mm_nl_count and mm_nl_fill with the count pass's decisions kept for the fill pass: masks holds cap 64-bit words per
+ * atom, the bit of each candidate of a receiver in candidate order; a receiver with more than 64 cap candidates is
+ * tested again by the fill pass.  The two calls take the same arguments otherwise (cap 0: no masks). */
+int mm_nl_count_masked(const double* pos_sorted, const int* cell_sorted, long N, const double* box /* HOST [3] */,
+                       const int* ncell /* HOST [3] */, const int* cell_start, const int* cell_count, double r_cut2,
+                       int brute, int* NN, unsigned long long* masks /* nullable */, int cap, mm_stream_t stream);
+int mm_nl_fill_masked(const double* pos_sorted, const int* cell_sorted, long N, const double* box /* HOST [3] */,
+                      const int* ncell /* HOST [3] */, const int* cell_start, const int* cell_count, double r_cut2,
+                      int brute, const long* rowptr, int* send, const unsigned long long* masks /* nullable */, int cap,
+                      mm_stream_t stream);
 /* per-step pair list of an MD run: pairs of a skin list within r_max (LAMMPS' ML-IAP pair list within the
  * cutoff, inputs/in.water_scan.lmp:44-52) */
 int mm_nl_filter_count(const double* pos, long N, const double* box /* HOST [3] */, const long* skin_rowptr,

@@ -10,6 +10,7 @@
 // over the 8 channel blocks of the convolution backward and the density term g_rho[recv] * d'(r) added.
 #include "common.h"
 #include "gen/sh.h"
+#include "mic.h"
 
 #define MM_MAX_BESSEL 16
 
@@ -117,14 +118,6 @@ __global__ void mm_edge_geom_rij_kernel(int E, const double* __restrict__ rij, c
                  e_pk, e_recv, e_dd);
 }
 
-// x_i - x_j - L * rint((x_i - x_j) / L), every operation rounded separately (no FMA contraction), as torch's
-// System.min_image on the CPU
-__device__ __forceinline__ double mm_mic_f64(double xi, double xj, double L) {
-#pragma clang fp contract(off)
-  const double x = xi - xj;
-  return x - L * rint(x / L);
-}
-
 // standalone path: v = minimum image of x_recv - x_send in fp64 (receiver_chunk_mace.py:110-111, 194)
 __global__ void mm_edge_geom_pos_kernel(int E, const double* __restrict__ pos, double bx, double by, double bz,
                                         const int* __restrict__ recv_local, int a, const int* __restrict__ ls,
@@ -140,7 +133,7 @@ __global__ void mm_edge_geom_pos_kernel(int E, const double* __restrict__ pos, d
   double v[3];
   const double b[3] = {bx, by, bz};
 #pragma unroll
-  for (int k = 0; k < 3; ++k) v[k] = mm_mic_f64(pos[3 * gi + k], pos[3 * gj + k], b[k]);
+  for (int k = 0; k < 3; ++k) v[k] = mm_mic(pos[3 * gi + k] - pos[3 * gj + k], b[k], 0.5 * b[k]);
   (void)a;
   mm_geom_common(e, (float)v[0], (float)v[1], (float)v[2], rl, sl, node_spec, S, pair_map, dp, sp, x_from_spec,
                  e_u, e_Y, e_pk, e_recv, e_dd);

@@ -11,6 +11,7 @@
 // the arithmetic scopes carry "#pragma clang fp contract(off)" (HIP's __dmul_rn / __dadd_rn are plain * and +,
 // which clang would otherwise fuse into FMAs and so change dd at the last bit).  Output: CSR (rowptr int64 [N+1], senders int32 [E]) in the sorted index space.
 #include "common.h"
+#include "mic.h"
 
 #include <hipcub/hipcub.hpp>
 
@@ -87,50 +88,189 @@ __global__ void mm_fill_i32_kernel_nl(int* __restrict__ p, int n, int v) {
   if (i < n) p[i] = v;
 }
 
-__device__ __forceinline__ double mm_mic(double v, double L) {
-#pragma clang fp contract(off)
-  return __dsub_rn(v, __dmul_rn(L, rint(__ddiv_rn(v, L))));
-}
+// Candidate test of the cell list, one workgroup of 4 waves per cell: all receivers of a cell share their candidates
+// (the 27 cells around it), which are staged in LDS MM_NL_CH at a time in candidate order; a wave tests 64 of them
+// against four receivers at once and compacts the kept ones with ballots.  blockIdx.y shares a cell's receivers out
+// when there are too few cells to fill the GPU.  brute != 0: every atom is a candidate of every receiver, 16 receivers
+// per workgroup.
+// Bound by the fp64 arithmetic of the tests (27 / 4.2 candidates per kept pair).  196,608 water atoms, 8 A (302 M
+// candidates, 42 M pairs): count 945 -> 487 us, fill 1,041 -> 250 us against one thread per receiver with its
+// candidates in global memory, three fp64 divisions per test and every test made twice.
+//
+// FILL = false: NN[i] = kept candidates of receiver i; with masks != nullptr also the ballots, one word per 64
+// candidates (masks[i * cap + word], if the cell's candidates fit cap words).
+// FILL = true: the kept candidates in order, send[rowptr[i] + k]; from the ballots where the count pass left them,
+// otherwise by testing again.
+#define MM_NL_CH 1024
+#define MM_NL_R 4
 
 template <bool FILL>
-__global__ void mm_nl_pairs_kernel(const double* __restrict__ pos, const int* __restrict__ cell, long N, double bx,
-                                   double by, double bz, int nx, int ny, int nz, const int* __restrict__ start,
-                                   const int* __restrict__ count, double r2, int brute, int* __restrict__ NN,
-                                   const long* __restrict__ rowptr, int* __restrict__ send) {
-  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (i >= N) return;
-  const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
-  long n = 0;
-  const long base = FILL ? rowptr[i] : 0;
-  auto test = [&](long j) {
-#pragma clang fp contract(off)
-    const double dx = mm_mic(__dsub_rn(xi, pos[3 * j]), bx);
-    const double dy = mm_mic(__dsub_rn(yi, pos[3 * j + 1]), by);
-    const double dz = mm_mic(__dsub_rn(zi, pos[3 * j + 2]), bz);
-    const double dd = __dadd_rn(__dadd_rn(__dmul_rn(dx, dx), __dmul_rn(dy, dy)), __dmul_rn(dz, dz));
-    if (dd < r2 && j != i) {
-      if (FILL) send[base + n] = (int)j;
-      ++n;
-    }
-  };
+__global__ void __launch_bounds__(256) mm_nl_pairs_kernel(const double* __restrict__ pos, long N, double bx, double by,
+                                                          double bz, int nx, int ny, int nz,
+                                                          const int* __restrict__ start,
+                                                          const int* __restrict__ count, double r2, int brute,
+                                                          int* __restrict__ NN, const long* __restrict__ rowptr,
+                                                          int* __restrict__ send,
+                                                          unsigned long long* __restrict__ masks, int cap) {
+  __shared__ double sx[MM_NL_CH], sy[MM_NL_CH], sz[MM_NL_CH];
+  __shared__ int sj[MM_NL_CH];
+  __shared__ int cs[27], cp[28];   // first atom of each candidate cell; candidates before it (cp[27]: all)
+  __shared__ int out_of_box;       // a coordinate outside [0, L] (or NaN): the tests take the general minimum image
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  long r0, nr, T;
   if (brute) {
-    for (long j = 0; j < N; ++j) test(j);
+    r0 = (long)blockIdx.x * (4 * MM_NL_R);
+    nr = min((long)(4 * MM_NL_R), N - r0);
+    T = N;
   } else {
-    const int cx = cell[3 * i], cy = cell[3 * i + 1], cz = cell[3 * i + 2];
-    for (int ox = -1; ox <= 1; ++ox) {
-      const int ax = ((cx + ox) % nx + nx) % nx;
-      for (int oy = -1; oy <= 1; ++oy) {
-        const int ay = ((cy + oy) % ny + ny) % ny;
-        for (int oz = -1; oz <= 1; ++oz) {
-          const int az = ((cz + oz) % nz + nz) % nz;
-          const int cl = (ax * ny + ay) * nz + az;
-          const int st = start[cl], ct = count[cl];
-          for (int k = 0; k < ct; ++k) test((long)st + k);
-        }
+    const int cl = blockIdx.x;
+    r0 = start[cl];
+    nr = count[cl];
+    if (nr == 0) return;
+    if (tid < 27) {
+      const int cx = cl / (ny * nz), cy = (cl / nz) % ny, cz = cl % nz;
+      const int ax = (cx + tid / 9 - 1 + nx) % nx, ay = (cy + (tid / 3) % 3 - 1 + ny) % ny,
+                az = (cz + tid % 3 - 1 + nz) % nz;
+      const int q = (ax * ny + ay) * nz + az;
+      cs[tid] = start[q];
+      cp[tid + 1] = count[q];
+    }
+    __syncthreads();
+    if (tid == 0) {
+      cp[0] = 0;
+      for (int k = 0; k < 27; ++k) cp[k + 1] += cp[k];
+    }
+    __syncthreads();
+    T = cp[27];
+  }
+  if (tid == 0) out_of_box = 0;
+  const bool masked = masks != nullptr && T <= 64L * cap;
+  auto inside = [&](double x, double y, double z) {
+    return x >= 0 && x <= bx && y >= 0 && y <= by && z >= 0 && z <= bz;
+  };
+  const double hx = 0.5 * bx, hy = 0.5 * by, hz = 0.5 * bz;
+  const int n_ch = (int)((T + MM_NL_CH - 1) / MM_NL_CH);
+  for (long rb = (long)blockIdx.y * (4 * MM_NL_R); rb < nr; rb += (long)gridDim.y * (4 * MM_NL_R)) {
+    long id[MM_NL_R], base[MM_NL_R];
+    double xi[MM_NL_R], yi[MM_NL_R], zi[MM_NL_R];
+    int n[MM_NL_R];
+    bool on[MM_NL_R];
+#pragma unroll
+    for (int r = 0; r < MM_NL_R; ++r) {
+      const long k = rb + MM_NL_R * wave + r;
+      on[r] = k < nr;
+      id[r] = r0 + (on[r] ? k : 0);
+      n[r] = 0;
+      base[r] = FILL ? rowptr[id[r]] : 0;
+      if (!(FILL && masked)) {
+        xi[r] = pos[3 * id[r]];
+        yi[r] = pos[3 * id[r] + 1];
+        zi[r] = pos[3 * id[r] + 2];
       }
     }
+    for (int ch = 0; ch < n_ch; ++ch) {
+      const long c0 = (long)ch * MM_NL_CH;
+      const int m = (int)min((long)MM_NL_CH, T - c0);
+      if (n_ch > 1 || rb == (long)blockIdx.y * (4 * MM_NL_R)) {   // a single chunk stays staged
+        __syncthreads();
+        for (int k = tid; k < m; k += 256) {
+          long j;
+          if (brute) {
+            j = c0 + k;
+          } else {
+            const int g = (int)c0 + k;
+            int lo = 0, hi = 26;   // last cell with cp <= g
+            while (lo < hi) {
+              const int mid = (lo + hi + 1) >> 1;
+              if (cp[mid] <= g) lo = mid;
+              else hi = mid - 1;
+            }
+            j = (long)cs[lo] + (g - cp[lo]);
+          }
+          sj[k] = (int)j;
+          if (!(FILL && masked)) {
+            const double x = pos[3 * j], y = pos[3 * j + 1], z = pos[3 * j + 2];
+            sx[k] = x;
+            sy[k] = y;
+            sz[k] = z;
+            if (!inside(x, y, z)) out_of_box = 1;
+          }
+        }
+        __syncthreads();
+      }
+      // receivers are candidates of their own cell: every coordinate of the tests has been looked at, the receivers'
+      // possibly in another stage of the candidates
+      bool general = out_of_box != 0;
+      if (!(FILL && masked)) {
+#pragma unroll
+        for (int r = 0; r < MM_NL_R; ++r) general |= !inside(xi[r], yi[r], zi[r]);
+      }
+      unsigned long long mine[MM_NL_R];   // lane s: the ballot of step s of this chunk
+#pragma unroll
+      for (int r = 0; r < MM_NL_R; ++r) {
+        mine[r] = 0;
+        if (FILL && masked && 64 * lane < m) mine[r] = masks[id[r] * cap + c0 / 64 + lane];
+      }
+      for (int s = 0; 64 * s < m; ++s) {
+        const int k = 64 * s + lane;
+        const bool in = k < m;
+        const int j = sj[in ? k : 0];
+        unsigned long long b[MM_NL_R];
+        if (FILL && masked) {
+#pragma unroll
+          for (int r = 0; r < MM_NL_R; ++r)   // s is uniform: the word goes to scalar registers
+            b[r] = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)mine[r], s) |
+                   (unsigned long long)(unsigned)__builtin_amdgcn_readlane((int)(mine[r] >> 32), s) << 32;
+        } else {
+          const double xj = sx[in ? k : 0], yj = sy[in ? k : 0], zj = sz[in ? k : 0];
+          auto test = [&](auto mic) {
+#pragma unroll
+            for (int r = 0; r < MM_NL_R; ++r) {
+#pragma clang fp contract(off)
+              const double dx = mic(xi[r] - xj, bx, hx);
+              const double dy = mic(yi[r] - yj, by, hy);
+              const double dz = mic(zi[r] - zj, bz, hz);
+              const double dd = (dx * dx + dy * dy) + dz * dz;
+              b[r] = __ballot(in & (dd < r2) & (j != (int)id[r]));
+            }
+          };
+          if (general) test([](double v, double L, double h) { return mm_mic(v, L, h); });
+          else test([](double v, double L, double h) { return mm_mic_in_box(v, L, h); });
+        }
+#pragma unroll
+        for (int r = 0; r < MM_NL_R; ++r) {
+          if (FILL) {
+            if (on[r] & (int)((b[r] >> lane) & 1ull))
+              send[base[r] + n[r] + __builtin_amdgcn_mbcnt_hi((unsigned)(b[r] >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo((unsigned)b[r], 0))] = j;
+          } else {
+            mine[r] = lane == s ? b[r] : mine[r];
+          }
+          n[r] += __popcll(b[r]);
+        }
+      }
+      if (!FILL && masked) {
+#pragma unroll
+        for (int r = 0; r < MM_NL_R; ++r)
+          if (on[r] && 64 * lane < m) masks[id[r] * cap + c0 / 64 + lane] = mine[r];
+      }
+    }
+    if (!FILL && lane == 0) {
+#pragma unroll
+      for (int r = 0; r < MM_NL_R; ++r)
+        if (on[r]) NN[id[r]] = n[r];
+    }
   }
-  if (!FILL) NN[i] = (int)n;
+}
+
+// Grid of mm_nl_pairs_kernel: a workgroup per cell (16 receivers per workgroup when brute), a cell's receivers shared
+// by up to 8 workgroups while the cells alone give the GPU fewer than 4 workgroups per CU.
+static dim3 nl_pairs_grid(long N, const int* ncell, int brute) {
+  if (brute) return dim3((unsigned)((N + 4 * MM_NL_R - 1) / (4 * MM_NL_R)));
+  const long cells = (long)ncell[0] * ncell[1] * ncell[2];
+  long y = 1;
+  while (y < 8 && cells * y < 1024) y *= 2;
+  return dim3((unsigned)cells, (unsigned)y);
 }
 
 extern "C" int mm_nl_workspace_bytes(long N, size_t* bytes) {
@@ -188,14 +328,22 @@ extern "C" int mm_nl_cell_ranges(const int* cell_s, long N, const int* ncell, in
   return mm::launch_status("mm_nl_cell_ranges");
 }
 
+extern "C" int mm_nl_count_masked(const double* pos_s, const int* cell_s, long N, const double* box, const int* ncell,
+                                  const int* start, const int* count, double r2, int brute, int* NN,
+                                  unsigned long long* masks, int cap, hipStream_t stream) {
+  MM_CHECK_ARG(N >= 0 && N < (1L << 31) && box && ncell, "bad arguments");
+  MM_CHECK_ARG(cap >= 0 && (cap == 0 || masks), "cap words per atom need the mask buffer");
+  (void)cell_s;   // the cells' ranges say which atoms they hold
+  if (N == 0) return MM_OK;
+  hipLaunchKernelGGL(mm_nl_pairs_kernel<false>, nl_pairs_grid(N, ncell, brute), dim3(256), 0, stream, pos_s, N, box[0],
+                     box[1], box[2], ncell[0], ncell[1], ncell[2], start, count, r2, brute, NN, (const long*)nullptr,
+                     (int*)nullptr, cap ? masks : nullptr, cap);
+  return mm::launch_status("mm_nl_count");
+}
+
 extern "C" int mm_nl_count(const double* pos_s, const int* cell_s, long N, const double* box, const int* ncell,
                            const int* start, const int* count, double r2, int brute, int* NN, hipStream_t stream) {
-  MM_CHECK_ARG(N >= 0 && box && ncell, "bad arguments");
-  if (N == 0) return MM_OK;
-  hipLaunchKernelGGL(mm_nl_pairs_kernel<false>, dim3((unsigned)((N + 127) / 128)), dim3(128), 0, stream, pos_s,
-                     cell_s, N, box[0], box[1], box[2], ncell[0], ncell[1], ncell[2], start, count, r2, brute, NN,
-                     (const long*)nullptr, (int*)nullptr);
-  return mm::launch_status("mm_nl_count");
+  return mm_nl_count_masked(pos_s, cell_s, N, box, ncell, start, count, r2, brute, NN, nullptr, 0, stream);
 }
 
 extern "C" int mm_nl_scan(const int* NN, long* rowptr, long N, void* ws, size_t ws_bytes, hipStream_t stream) {
@@ -347,15 +495,23 @@ extern "C" int mm_nl_scan_noalloc(const int* NN, long* rowptr, long N, hipStream
   return mm::launch_status("mm_nl_scan_noalloc");
 }
 
+extern "C" int mm_nl_fill_masked(const double* pos_s, const int* cell_s, long N, const double* box, const int* ncell,
+                                 const int* start, const int* count, double r2, int brute, const long* rowptr,
+                                 int* send, const unsigned long long* masks, int cap, hipStream_t stream) {
+  MM_CHECK_ARG(N >= 0 && N < (1L << 31) && box && ncell, "bad arguments");
+  MM_CHECK_ARG(cap >= 0 && (cap == 0 || masks), "cap words per atom need the mask buffer");
+  (void)cell_s;
+  if (N == 0) return MM_OK;
+  hipLaunchKernelGGL(mm_nl_pairs_kernel<true>, nl_pairs_grid(N, ncell, brute), dim3(256), 0, stream, pos_s, N, box[0],
+                     box[1], box[2], ncell[0], ncell[1], ncell[2], start, count, r2, brute, (int*)nullptr, rowptr,
+                     send, cap ? (unsigned long long*)masks : nullptr, cap);
+  return mm::launch_status("mm_nl_fill");
+}
+
 extern "C" int mm_nl_fill(const double* pos_s, const int* cell_s, long N, const double* box, const int* ncell,
                           const int* start, const int* count, double r2, int brute, const long* rowptr, int* send,
                           hipStream_t stream) {
-  MM_CHECK_ARG(N >= 0 && box && ncell, "bad arguments");
-  if (N == 0) return MM_OK;
-  hipLaunchKernelGGL(mm_nl_pairs_kernel<true>, dim3((unsigned)((N + 127) / 128)), dim3(128), 0, stream, pos_s,
-                     cell_s, N, box[0], box[1], box[2], ncell[0], ncell[1], ncell[2], start, count, r2, brute,
-                     (int*)nullptr, rowptr, send);
-  return mm::launch_status("mm_nl_fill");
+  return mm_nl_fill_masked(pos_s, cell_s, N, box, ncell, start, count, r2, brute, rowptr, send, nullptr, 0, stream);
 }
 
 // Per-step pair list of an MD run: the pairs of a skin list (built with r_cut = r_max + skin) whose current
@@ -407,9 +563,9 @@ __global__ void __launch_bounds__(256) mm_nl_filter_kernel(const double* __restr
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
 #pragma clang fp contract(off)
-        const double dx = mm_mic(xi - px[k], bx);
-        const double dy = mm_mic(yi - py[k], by);
-        const double dz = mm_mic(zi - pz[k], bz);
+        const double dx = mm_mic(xi - px[k], bx, 0.5 * bx);
+        const double dy = mm_mic(yi - py[k], by, 0.5 * by);
+        const double dz = mm_mic(zi - pz[k], bz, 0.5 * bz);
         const double dd = (dx * dx + dy * dy) + dz * dz;
         keep[k] = (e0 + lane + 64 * k < end) & (dd < r2) & (j[k] != i);
       }

@@ -32,9 +32,11 @@ SIGNATURES = {
     "mm_nl_gather": [P, L, P, P, P, P, P, P, P],
     "mm_nl_cell_ranges": [P, L, P, P, P, P],
     "mm_nl_count": [P, P, L, P, P, P, P, D, I, P, P],
+    "mm_nl_count_masked": [P, P, L, P, P, P, P, D, I, P, P, I, P],
     "mm_nl_scan": [P, P, L, P, SZ, P],
     "mm_nl_scan_noalloc": [P, P, L, P],
     "mm_nl_fill": [P, P, L, P, P, P, P, D, I, P, P, P],
+    "mm_nl_fill_masked": [P, P, L, P, P, P, P, D, I, P, P, P, I, P],
     "mm_nl_filter_count": [P, L, P, P, P, D, P, P, P],
     "mm_nl_filter_fill": [P, L, P, P, P, D, P, P, P, I, P],
     "mm_nl_reverse": [P, P, L, L, P, P],

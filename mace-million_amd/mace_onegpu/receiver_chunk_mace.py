@@ -67,6 +67,14 @@ class System:
         box = torch.as_tensor(self.box, dtype=v.dtype, device=v.device)
         return v - box * torch.round(v / box)
 
+    def _mask_words(self, brute, ncells):
+        """Mask words per atom in which the count pass leaves its decisions to the fill pass: half as many again as
+        the mean number of candidates needs (denser cells are tested twice).  None beyond 2 GB: there the masks would
+        rival the pair list itself."""
+        T = self.N if brute else 27 * self.N / ncells
+        cap = int(1.5 * T / 64) + 2
+        return cap if 8 * cap * self.N <= 2 << 30 else 0
+
     def build_neighbors(self, r_cut=None):
         """CSR neighbour list within r_cut (default r_max) in the reference's candidate order.  The cell grid
         is the one of r_max (as System.__init__ fixes it), so r_cut must not exceed r_max unless the System was
@@ -83,13 +91,17 @@ class System:
         K.mm_nl_cell_ranges(self.cell, N, self._nc_h, start, count, stream())
         NN = torch.empty(N, dtype=torch.int32, device=dev)
         r2 = r_cut ** 2
-        K.mm_nl_count(self.pos, self.cell, N, self._box_h, self._nc_h, start, count, r2, brute, NN, stream())
+        cap, masks = self._mask_words(brute, ncells), None
+        if cap:
+            masks = torch.empty(N * cap, dtype=torch.int64, device=dev)
+        K.mm_nl_count_masked(self.pos, self.cell, N, self._box_h, self._nc_h, start, count, r2, brute, NN, masks, cap,
+                             stream())
         rowptr = torch.empty(N + 1, dtype=torch.int64, device=dev)
         K.mm_nl_scan(NN, rowptr, N, self._ws, self._ws.numel(), stream())
         E = int(rowptr[-1])
         send = torch.empty(max(E, 1), dtype=torch.int32, device=dev)
-        K.mm_nl_fill(self.pos, self.cell, N, self._box_h, self._nc_h, start, count, r2, brute, rowptr, send,
-                     stream())
+        K.mm_nl_fill_masked(self.pos, self.cell, N, self._box_h, self._nc_h, start, count, r2, brute, rowptr, send,
+                            masks, cap, stream())
         self.NN, self.rowptr, self.send = NN, rowptr, send[:E]
         self.MN = int(NN.max()) if N else 0
         return self.MN
