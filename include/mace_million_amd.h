@@ -170,6 +170,12 @@ int mm_spline_coeffs_flat(const double* samples, int M, int D, double eps, doubl
  * Other tables (harmonics up to l = 3): the same two entry points, named mm_tpw_j<hash>_fwd / _bwd, are exported
  * by lib/jit/tpw_j<hash>.so, which mace_onegpu.tp_jit generates and compiles for the table on first use (P from
  * codegen.tpw_layout(table)["parts"]). */
+/* Index preparation of the above for an edge list: rowptr [n + 1] = first edge with receiver >= k (the CSR when the
+ * receivers are sorted), send32 [E] = the senders as int32, and violation counts added to bad [3] (zeroed by the
+ * caller): senders outside [0, n_send), receivers outside [0, n), receivers smaller than their predecessor.  send and
+ * recv are int32, or int64 with index64 != 0; strides in elements; send and send32 may both be null. */
+int mm_edge_csr(const void* send, long send_stride, const void* recv, long recv_stride, int index64, int E, int n,
+                int n_send, int* send32, int* rowptr, int* bad, mm_stream_t stream);
 int mm_tpw_l1_fwd(const int* rowptr, int nR, const int* eid, const int* send, const float* Y, long y_stride,
                   const float* W, long w_stride, const float* X, long x_stride, float* out, long out_stride,
                   mm_stream_t stream);
@@ -191,6 +197,29 @@ int mm_tpw_l0123_bwd(const int* rowptr, int nR, const int* eid, const int* send,
                      const float* W, long w_stride, const float* X, long x_stride, const float* gO, long g_stride,
                      float* gW, long gw_stride, float* gYp, long gy_cb_stride, float* gX, long gx_stride,
                      mm_stream_t stream);
+/* The same with the edge count E of the list, by which the launch shares long receivers' edges between waves (-1:
+ * unknown, as the calls above). */
+int mm_tpw_l1_fwd_n(long E, const int* rowptr, int nR, const int* eid, const int* send, const float* Y,
+                    long y_stride, const float* W, long w_stride, const float* X, long x_stride, float* out,
+                    long out_stride, mm_stream_t stream);
+int mm_tpw_l2_fwd_n(long E, const int* rowptr, int nR, const int* eid, const int* send, const float* Y,
+                    long y_stride, const float* W, long w_stride, const float* X, long x_stride, float* out,
+                    long out_stride, mm_stream_t stream);
+int mm_tpw_l0123_fwd_n(long E, const int* rowptr, int nR, const int* eid, const int* send, const float* Y,
+                       long y_stride, const float* W, long w_stride, const float* X, long x_stride, float* out,
+                       long out_stride, mm_stream_t stream);
+int mm_tpw_l1_bwd_n(long E, const int* rowptr, int nR, const int* eid, const int* send, const float* Y,
+                    long y_stride, const float* W, long w_stride, const float* X, long x_stride, const float* gO,
+                    long g_stride, float* gW, long gw_stride, float* gYp, long gy_cb_stride, float* gX,
+                    long gx_stride, mm_stream_t stream);
+int mm_tpw_l2_bwd_n(long E, const int* rowptr, int nR, const int* eid, const int* send, const float* Y,
+                    long y_stride, const float* W, long w_stride, const float* X, long x_stride, const float* gO,
+                    long g_stride, float* gW, long gw_stride, float* gYp, long gy_cb_stride, float* gX,
+                    long gx_stride, mm_stream_t stream);
+int mm_tpw_l0123_bwd_n(long E, const int* rowptr, int nR, const int* eid, const int* send, const float* Y,
+                       long y_stride, const float* W, long w_stride, const float* X, long x_stride, const float* gO,
+                       long g_stride, float* gW, long gw_stride, float* gYp, long gy_cb_stride, float* gX,
+                       long gx_stride, mm_stream_t stream);
 
 /* ---------------------------------------------------------------------------------------------- (4) node level
  * Symmetric contraction (correlation 3, per species) forward / backward: replaces model.products[k]

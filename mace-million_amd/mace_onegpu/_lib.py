@@ -57,9 +57,12 @@ SIGNATURES = {
     "mm_conv0123_fwd": [P, I, P, P, P, I, P, I, I, P, P, P],
     "mm_conv0123_bwd": [P, I, P, P, P, I, P, I, I, F, P, P, L, P, P],
     "mm_gather_rows_csr": [P, P, P, L, I, P, L, I, P],
+    "mm_edge_csr": [P, L, P, L, I, I, I, I, P, P, P, P],
     # explicit-weight channelwise TP (generated; FusedConvTP)
     **{f"mm_tpw_{n}_fwd": [P, I, P, P, P, L, P, L, P, L, P, L, P] for n in ("l1", "l2", "l0123")},
     **{f"mm_tpw_{n}_bwd": [P, I, P, P, P, L, P, L, P, L, P, L, P, L, P, L, P, L, P] for n in ("l1", "l2", "l0123")},
+    **{f"mm_tpw_{n}_fwd_n": [L, P, I, P, P, P, L, P, L, P, L, P, L, P] for n in ("l1", "l2", "l0123")},
+    **{f"mm_tpw_{n}_bwd_n": [L, P, I, P, P, P, L, P, L, P, L, P, L, P, L, P, L, P, L, P] for n in ("l1", "l2", "l0123")},
     # symmetric contraction (generated)
     "mm_symc1_fwd": [I, P, L, P, P, P, L, P],
     "mm_symc2_fwd": [I, P, L, P, P, P, L, P],

@@ -584,6 +584,23 @@ def conv_source(tab, layer, need_gx, opts=None):
 TPW_TABLES = o3.COMPILED_TP_TABLES
 
 
+# When the four waves of a workgroup of the explicit-weight kernels share one receiver's edges instead of taking a
+# receiver each.  With few receivers it is the parallelism that pays (501 receivers of 37 edges, shared against not:
+# forward l1 34 -> 14 us, l2 68 -> 26; backward l1 83 -> 27, l2 106 -> 62); with many, a wave streams contiguous rows of
+# W next to its neighbours' (16,384 receivers of 90 edges: forward l2 1,651 -> 1,559 us, backward 4,121 -> 4,015), but
+# each pays for its part of the reduction or its own receiver constants, so short receivers stay whole.
+# Mean edges per receiver from which they are shared, by the accumulators (forward) or constants (backward) per lane:
+# at 16,384 receivers forward l1 (32) 3 edges 39 -> 39 us, 7 83 -> 72; l2 (80) 7 199 -> 198, 13 306 -> 287; l0123 (99) 13
+# 718 -> 732, 20 1,037 -> 1,019; backward l1 (32) 3 85 -> 83, l2 (76) 7 407 -> 417, 13 689 -> 680.  A backward in path
+# groups (l0123) has several waves per receiver already: shared up to SHARE_WAVES of them (37 edges: 1,500 waves 139 ->
+# 94 us, 9,000 633 -> 619, 12,000 799 -> 817).
+SHARE_WAVES = 8192
+
+
+def _share_edges(state):
+    return 4 if state <= 40 else 10 if state <= 88 else 18
+
+
 def tpw_layout(tab):
     """Lane layout of the explicit-weight kernels of one path table.  A wave serves one receiver and a row of 64
     or 128 channels: cpl channels per lane (c = 64 h + lane + 64 j, j < cpl), nh = 2 / cpl waves per receiver
@@ -695,15 +712,24 @@ def tpw_source(tab, name):
     L = []
     A = L.append
 
-    def head(kind, nh, npg=1):
+    def head(kind, nh, npg=1, shared=False):
         """Wave -> (receiver i, sub-wave h): h = channel half * npg + path group; c = first channel of the lane
-        (channel half * 64 + lane), always < 128."""
-        A(f"  const int gw = blockIdx.x * 4 + (threadIdx.x >> 6);   // global wave: receiver i, sub-wave h")
+        (channel half * 64 + lane), always < 128.  shared: one (i, h) per workgroup, a quarter of the receiver's edges
+        per wave."""
+        if shared:
+            A("  const int wave = threadIdx.x >> 6;")
+            A("  const int gw = blockIdx.x;   // receiver i, sub-wave h")
+        else:
+            A(f"  const int gw = blockIdx.x * 4 + (threadIdx.x >> 6);   // global wave: receiver i, sub-wave h")
         A(f"  const int i = gw / {nh}, h = gw % {nh};" if nh > 1 else "  const int i = gw, h = 0;")
         A("  if (i >= nR) return;")
         A("  const int lane = threadIdx.x & 63;")
         A(f"  const int c = (h / {npg}) * 64 + lane;" if npg > 1 else "  const int c = h * 64 + lane;")
-        A("  const int p0 = rowptr[i], p1 = rowptr[i + 1];")
+        if shared:
+            A("  const int r0 = rowptr[i], nr = rowptr[i + 1] - r0;")
+            A("  const int p0 = r0 + (int)((long)nr * wave / 4), p1 = r0 + (int)((long)nr * (wave + 1) / 4);")
+        else:
+            A("  const int p0 = rowptr[i], p1 = rowptr[i + 1];")
 
     def edge_loads(t, cpl, pidx, guard=None, ws=None, ks=None):
         ws = used_w if ws is None else ws
@@ -742,176 +768,204 @@ def tpw_source(tab, name):
     A('#include "../common.h"')
     A("")
     # ------------------------------------------------------------------ forward
-    cpl, nh, un = lay["cpl_fwd"], lay["nh_fwd"], lay["unroll_fwd"]
-    A("extern \"C\" __global__ void __launch_bounds__(256)")
-    A(f"mm_{kn}_fwd_kernel(const int* __restrict__ rowptr, int nR, const int* __restrict__ eid,")
-    A("    const int* __restrict__ send, const float* __restrict__ Y, long y_stride, const float* __restrict__ W,")
-    A("    long w_stride, const float* __restrict__ X, long x_stride, float* __restrict__ out, long out_stride) {")
-    head("fwd", nh)
-    for o in used_o:
-        for j in range(cpl):
-            A(f"  float acc{o}_{j} = 0.f;")
-
-    def fwd_body(t):
-        # per (w, k) group: q = W X, one product q |coef| per distinct |coef| of the group, then one FMA per term
-        # with the edge's (wave-uniform) harmonic
-        for (w, k), lst in groups.items():
-            mags = OrderedDict()
-            for (m, o, c) in lst:
-                if abs(abs(c) - 1.0) > 1e-12:
-                    mags.setdefault(round(abs(c), 12), (len(mags), abs(c)))
+    def forward(shared):
+        cpl, nh, un = lay["cpl_fwd"], lay["nh_fwd"], lay["unroll_fwd"]
+        A("extern \"C\" __global__ void __launch_bounds__(256)")
+        A(f"mm_{kn}_fwd{'_shared' if shared else ''}_kernel(const int* __restrict__ rowptr, int nR, const int* __restrict__ eid,")
+        A("    const int* __restrict__ send, const float* __restrict__ Y, long y_stride, const float* __restrict__ W,")
+        A("    long w_stride, const float* __restrict__ X, long x_stride, float* __restrict__ out, long out_stride) {")
+        accs = [f"acc{o}_{j}" for o in used_o for j in range(cpl)]
+        if shared:
+            A(f"  __shared__ float red[{len(accs)} * 64];   // one wave's sums [accumulator][lane]")
+        head("fwd", nh, shared=shared)
+        for o in used_o:
             for j in range(cpl):
-                A(f"    {{ const float q = W{w}_{j}_{t} * X{k}_{j}_{t};")
-                for key, (idx, ac) in mags.items():
-                    A(f"      const float q{idx} = {_f(ac)} * q;")
+                A(f"  float acc{o}_{j} = 0.f;")
+
+        def fwd_body(t):
+            # per (w, k) group: q = W X, one product q |coef| per distinct |coef| of the group, then one FMA per term
+            # with the edge's (wave-uniform) harmonic
+            for (w, k), lst in groups.items():
+                mags = OrderedDict()
                 for (m, o, c) in lst:
-                    key = round(abs(c), 12)
-                    qv = f"q{mags[key][0]}" if key in mags else "q"
-                    A(f"      acc{o}_{j} = fmaf({'-' if c < 0 else ''}{qv}, Y{m}_{t}, acc{o}_{j});")
-                A("    }")
-
-    if un == 2:
-        A("  for (int p = p0; p < p1; p += 2) {")
-        A("    const bool two = p + 1 < p1;   // wave-uniform")
-        edge_loads("a", cpl, "p")
-        edge_loads("b", cpl, "p + 1", guard="two")
-        fwd_body("a")
-        A("    if (two) {")
-        fwd_body("b")
-        A("    }")
-        A("  }")
-    else:
-        A("  for (int p = p0; p < p1; ++p) {")
-        edge_loads("a", cpl, "p")
-        fwd_body("a")
-        A("  }")
-    A("  float* __restrict__ op = out + (size_t)i * out_stride + c;")
-    for o in range(nO):
-        for j in range(cpl):
-            v = f"acc{o}_{j}" if o in used_o else "0.f"
-            A(f"  op[{o * C + 64 * j}] = {v};")
-    A("}")
-    A("")
-    # ------------------------------------------------------------------ backward
-    cpl, nh, un, npg = lay["cpl_bwd"], lay["nh_bwd"], lay["unroll_bwd"], lay["npg"]
-    pgroups = _path_groups(tab)
-    A("// Backward from gO = dL/dout: gW[e, w, c] (written), gYp[part][e][m] = partial sums of dL/dY[e, m] over")
-    A(f"// the channels and paths of one wave ({lay['parts']} partial(s): channel half h x path group g, part")
-    A(f"// h * {npg} + g; summed by the caller), gX[send, k, c] (atomic adds).  Null outputs are skipped.")
-    if npg > 1:
-        A(f"// Path groups (one wave each): {pgroups}.")
-    A("extern \"C\" __global__ void __launch_bounds__(256)")
-    A(f"mm_{kn}_bwd_kernel(const int* __restrict__ rowptr, int nR, const int* __restrict__ eid,")
-    A("    const int* __restrict__ send, const float* __restrict__ Y, long y_stride, const float* __restrict__ W,")
-    A("    long w_stride, const float* __restrict__ X, long x_stride, const float* __restrict__ gO, long g_stride,")
-    A("    float* __restrict__ gW, long gw_stride, float* __restrict__ gYp, long gy_cb_stride,")
-    A("    float* __restrict__ gX, long gx_stride) {")
-    head("bwd", nh * npg, npg)
-    if npg > 1:
-        A(f"  const int pg = h % {npg};   // path group; channel half h / {npg}")
-    A("  const int part = h;")
-    A("  const int cl = lane & 15;")
-    A("  const bool b3 = cl & 8, b2 = cl & 4, b1 = cl & 2, b0 = cl & 1;")
-
-    def bwd_group(gi, wsel):
-        gsel = [(wk, lst) for wk, lst in groups.items() if wk[0] in wsel]
-        ksel = sorted({k for (w, k), _ in gsel})
-        osel = sorted({o for _, lst in gsel for (m, o, cf) in lst})
-        A("  const float* __restrict__ gp = gO + (size_t)i * g_stride + c;")
-        for o in osel:
-            for j in range(cpl):
-                A(f"  const float g{o}_{j} = gp[{o * C + 64 * j}];")
-        tid, gm, sums = _bwd_constants(gsel)
-        for n, ocs in enumerate(sums):
-            for j in range(cpl):
-                A(f"  const float G{n}_{j} = {_const_expr(ocs, lambda o: f'g{o}_{j}')};")
-
-        def bwd_body(t):
-            for m in range(16):
-                A(f"    float gy{m} = 0.f;")
-            for k in ksel:
+                    if abs(abs(c) - 1.0) > 1e-12:
+                        mags.setdefault(round(abs(c), 12), (len(mags), abs(c)))
                 for j in range(cpl):
-                    A(f"    float gx{k}_{j} = 0.f;")
-            A(f"    float* __restrict__ gwp = gW ? gW + (size_t)e{t} * gw_stride + c : nullptr;")
-            for w in wsel:
-                A("    {")
-                for j in range(cpl):
-                    A(f"      float gw{j} = 0.f;")
-                for (ww, k), lst in gsel:
-                    if ww != w:
-                        continue
-                    for j in range(cpl):
-                        A(f"      {{ const float q = W{w}_{j}_{t} * X{k}_{j}_{t}; float u = 0.f;")
-                        for m in gm[(w, k)]:
-                            G = f"G{tid[(w, k, m)]}_{j}"
-                            A(f"        u = fmaf(Y{m}_{t}, {G}, u); gy{m} = fmaf(q, {G}, gy{m});")
-                        A(f"        gw{j} = fmaf(X{k}_{j}_{t}, u, gw{j}); gx{k}_{j} = fmaf(W{w}_{j}_{t}, u, gx{k}_{j});")
-                        A("      }")
-                for j in range(cpl):
-                    A(f"      if (gwp) gwp[{w * C + 64 * j}] = gw{j};")
-                A("    }")
-            if gi == 0:
-                for w in range(nW):
-                    if w not in used_w:
-                        for j in range(cpl):
-                            A(f"    if (gwp) gwp[{w * C + 64 * j}] = 0.f;")
-            A("    if (gYp) {")
-            A("      // transpose-reduction over each 16-lane row (lane cl ends with the row's sum of gy_cl), then the"
-              " 4 rows")
-            for j in range(8):
-                A(f"      const float s8_{j} = (b3 ? gy{8 + j} : gy{j}) + mm_dpp<0x140>(b3 ? gy{j} : gy{8 + j});")
-            for j in range(4):
-                A(f"      const float s4_{j} = (b2 ? s8_{4 + j} : s8_{j}) + mm_dpp<0x141>(b2 ? s8_{j} : s8_{4 + j});")
-            for j in range(2):
-                A(f"      const float s2_{j} = (b1 ? s4_{2 + j} : s4_{j}) + mm_dpp<0x1B>(b1 ? s4_{j} : s4_{2 + j});")
-            A("      float gyl = (b0 ? s2_1 : s2_0) + mm_dpp<0xB1>(b0 ? s2_0 : s2_1);")
-            A("      gyl += __shfl_xor(gyl, 16);")
-            A("      gyl += __shfl_xor(gyl, 32);")
-            A(f"      if (lane < 16) gYp[(size_t)part * gy_cb_stride + (size_t)e{t} * 16 + lane] = gyl;")
-            A("    }")
-            A("    if (gX) {")
-            A(f"      float* __restrict__ gxp = gX + (size_t)s{t} * gx_stride + c;")
-            for k in ksel:
-                for j in range(cpl):
-                    A(f"      atomicAdd(gxp + {k * C + 64 * j}, gx{k}_{j});")
-            A("    }")
+                    A(f"    {{ const float q = W{w}_{j}_{t} * X{k}_{j}_{t};")
+                    for key, (idx, ac) in mags.items():
+                        A(f"      const float q{idx} = {_f(ac)} * q;")
+                    for (m, o, c) in lst:
+                        key = round(abs(c), 12)
+                        qv = f"q{mags[key][0]}" if key in mags else "q"
+                        A(f"      acc{o}_{j} = fmaf({'-' if c < 0 else ''}{qv}, Y{m}_{t}, acc{o}_{j});")
+                    A("    }")
 
         if un == 2:
             A("  for (int p = p0; p < p1; p += 2) {")
             A("    const bool two = p + 1 < p1;   // wave-uniform")
-            edge_loads("a", cpl, "p", ws=wsel, ks=ksel)
-            edge_loads("b", cpl, "p + 1", guard="two", ws=wsel, ks=ksel)
-            bwd_body("a")
+            edge_loads("a", cpl, "p")
+            edge_loads("b", cpl, "p + 1", guard="two")
+            fwd_body("a")
             A("    if (two) {")
-            bwd_body("b")
+            fwd_body("b")
             A("    }")
             A("  }")
         else:
             A("  for (int p = p0; p < p1; ++p) {")
-            edge_loads("a", cpl, "p", ws=wsel, ks=ksel)
-            bwd_body("a")
+            edge_loads("a", cpl, "p")
+            fwd_body("a")
             A("  }")
+        if shared:
+            A("  for (int s = 1; s < 4; ++s) {   // the waves' sums in wave order")
+            A("    if (wave == s) {")
+            for q, v in enumerate(accs):
+                A(f"      red[{64 * q} + lane] = {v};")
+            A("    }")
+            A("    __syncthreads();")
+            A("    if (wave == 0) {")
+            for q, v in enumerate(accs):
+                A(f"      {v} += red[{64 * q} + lane];")
+            A("    }")
+            A("    __syncthreads();")
+            A("  }")
+            A("  if (wave) return;")
+        A("  float* __restrict__ op = out + (size_t)i * out_stride + c;")
+        for o in range(nO):
+            for j in range(cpl):
+                v = f"acc{o}_{j}" if o in used_o else "0.f"
+                A(f"  op[{o * C + 64 * j}] = {v};")
+        A("}")
+        A("")
 
-    if npg == 1:
-        bwd_group(0, pgroups[0])
-    else:
-        for gi, wsel in enumerate(pgroups):
-            A(f"  {'if' if gi == 0 else 'else if'} (pg == {gi}) {{")
-            bwd_group(gi, wsel)
-            A("  }")
-    A("}")
-    A("")
+    forward(False)
+    forward(True)
+    # ------------------------------------------------------------------ backward
+    def backward(shared):
+        cpl, nh, un, npg = lay["cpl_bwd"], lay["nh_bwd"], lay["unroll_bwd"], lay["npg"]
+        pgroups = _path_groups(tab)
+        A("// Backward from gO = dL/dout: gW[e, w, c] (written), gYp[part][e][m] = partial sums of dL/dY[e, m] over")
+        A(f"// the channels and paths of one wave ({lay['parts']} partial(s): channel half h x path group g, part")
+        A(f"// h * {npg} + g; summed by the caller), gX[send, k, c] (atomic adds).  Null outputs are skipped.")
+        if npg > 1:
+            A(f"// Path groups (one wave each): {pgroups}.")
+        A("extern \"C\" __global__ void __launch_bounds__(256)")
+        A(f"mm_{kn}_bwd{'_shared' if shared else ''}_kernel(const int* __restrict__ rowptr, int nR, const int* __restrict__ eid,")
+        A("    const int* __restrict__ send, const float* __restrict__ Y, long y_stride, const float* __restrict__ W,")
+        A("    long w_stride, const float* __restrict__ X, long x_stride, const float* __restrict__ gO, long g_stride,")
+        A("    float* __restrict__ gW, long gw_stride, float* __restrict__ gYp, long gy_cb_stride,")
+        A("    float* __restrict__ gX, long gx_stride) {")
+        head("bwd", nh * npg, npg, shared)
+        if npg > 1:
+            A(f"  const int pg = h % {npg};   // path group; channel half h / {npg}")
+        A("  const int part = h;")
+        A("  const int cl = lane & 15;")
+        A("  const bool b3 = cl & 8, b2 = cl & 4, b1 = cl & 2, b0 = cl & 1;")
+
+        def bwd_group(gi, wsel):
+            gsel = [(wk, lst) for wk, lst in groups.items() if wk[0] in wsel]
+            ksel = sorted({k for (w, k), _ in gsel})
+            osel = sorted({o for _, lst in gsel for (m, o, cf) in lst})
+            A("  const float* __restrict__ gp = gO + (size_t)i * g_stride + c;")
+            for o in osel:
+                for j in range(cpl):
+                    A(f"  const float g{o}_{j} = gp[{o * C + 64 * j}];")
+            tid, gm, sums = _bwd_constants(gsel)
+            for n, ocs in enumerate(sums):
+                for j in range(cpl):
+                    A(f"  const float G{n}_{j} = {_const_expr(ocs, lambda o: f'g{o}_{j}')};")
+
+            def bwd_body(t):
+                for m in range(16):
+                    A(f"    float gy{m} = 0.f;")
+                for k in ksel:
+                    for j in range(cpl):
+                        A(f"    float gx{k}_{j} = 0.f;")
+                A(f"    float* __restrict__ gwp = gW ? gW + (size_t)e{t} * gw_stride + c : nullptr;")
+                for w in wsel:
+                    A("    {")
+                    for j in range(cpl):
+                        A(f"      float gw{j} = 0.f;")
+                    for (ww, k), lst in gsel:
+                        if ww != w:
+                            continue
+                        for j in range(cpl):
+                            A(f"      {{ const float q = W{w}_{j}_{t} * X{k}_{j}_{t}; float u = 0.f;")
+                            for m in gm[(w, k)]:
+                                G = f"G{tid[(w, k, m)]}_{j}"
+                                A(f"        u = fmaf(Y{m}_{t}, {G}, u); gy{m} = fmaf(q, {G}, gy{m});")
+                            A(f"        gw{j} = fmaf(X{k}_{j}_{t}, u, gw{j}); gx{k}_{j} = fmaf(W{w}_{j}_{t}, u, gx{k}_{j});")
+                            A("      }")
+                    for j in range(cpl):
+                        A(f"      if (gwp) gwp[{w * C + 64 * j}] = gw{j};")
+                    A("    }")
+                if gi == 0:
+                    for w in range(nW):
+                        if w not in used_w:
+                            for j in range(cpl):
+                                A(f"    if (gwp) gwp[{w * C + 64 * j}] = 0.f;")
+                A("    if (gYp) {")
+                A("      // transpose-reduction over each 16-lane row (lane cl ends with the row's sum of gy_cl), then the"
+                  " 4 rows")
+                for j in range(8):
+                    A(f"      const float s8_{j} = (b3 ? gy{8 + j} : gy{j}) + mm_dpp<0x140>(b3 ? gy{j} : gy{8 + j});")
+                for j in range(4):
+                    A(f"      const float s4_{j} = (b2 ? s8_{4 + j} : s8_{j}) + mm_dpp<0x141>(b2 ? s8_{j} : s8_{4 + j});")
+                for j in range(2):
+                    A(f"      const float s2_{j} = (b1 ? s4_{2 + j} : s4_{j}) + mm_dpp<0x1B>(b1 ? s4_{j} : s4_{2 + j});")
+                A("      float gyl = (b0 ? s2_1 : s2_0) + mm_dpp<0xB1>(b0 ? s2_0 : s2_1);")
+                A("      gyl += __shfl_xor(gyl, 16);")
+                A("      gyl += __shfl_xor(gyl, 32);")
+                A(f"      if (lane < 16) gYp[(size_t)part * gy_cb_stride + (size_t)e{t} * 16 + lane] = gyl;")
+                A("    }")
+                A("    if (gX) {")
+                A(f"      float* __restrict__ gxp = gX + (size_t)s{t} * gx_stride + c;")
+                for k in ksel:
+                    for j in range(cpl):
+                        A(f"      atomicAdd(gxp + {k * C + 64 * j}, gx{k}_{j});")
+                A("    }")
+
+            if un == 2:
+                A("  for (int p = p0; p < p1; p += 2) {")
+                A("    const bool two = p + 1 < p1;   // wave-uniform")
+                edge_loads("a", cpl, "p", ws=wsel, ks=ksel)
+                edge_loads("b", cpl, "p + 1", guard="two", ws=wsel, ks=ksel)
+                bwd_body("a")
+                A("    if (two) {")
+                bwd_body("b")
+                A("    }")
+                A("  }")
+            else:
+                A("  for (int p = p0; p < p1; ++p) {")
+                edge_loads("a", cpl, "p", ws=wsel, ks=ksel)
+                bwd_body("a")
+                A("  }")
+
+        if npg == 1:
+            bwd_group(0, pgroups[0])
+        else:
+            for gi, wsel in enumerate(pgroups):
+                A(f"  {'if' if gi == 0 else 'else if'} (pg == {gi}) {{")
+                bwd_group(gi, wsel)
+                A("  }")
+        A("}")
+        A("")
+
+    backward(False)
+    backward(True)
     # ------------------------------------------------------------------ entry points
     for kind, nh_k in (("fwd", lay["nh_fwd"]), ("bwd", lay["nh_bwd"] * lay["npg"])):
+        state = (lay["cpl_fwd"] * len(used_o) if kind == "fwd" else
+                 lay["cpl_bwd"] * len(_bwd_constants(list(groups.items()))[2]))
+        few = f"waves <= {SHARE_WAVES}" if kind == "bwd" and lay["npg"] > 1 else "true"
         if kind == "fwd":
-            A(f"extern \"C\" int mm_{kn}_fwd(const int* rowptr, int nR, const int* eid, const int* send, const float* Y,")
+            A(f"extern \"C\" int mm_{kn}_fwd_n(long E, const int* rowptr, int nR, const int* eid, const int* send, const float* Y,")
             A("    long y_stride, const float* W, long w_stride, const float* X, long x_stride, float* out, long out_stride,")
             A("    hipStream_t stream) {")
             A("  MM_CHECK_ARG(nR >= 0, \"bad sizes\");")
             A(f"  MM_CHECK_ARG(y_stride >= 16 && w_stride >= {nW * C} && x_stride >= {nX * C} && out_stride >= {nO * C},")
             A("               \"row strides smaller than the path table's widths\");")
         else:
-            A(f"extern \"C\" int mm_{kn}_bwd(const int* rowptr, int nR, const int* eid, const int* send, const float* Y,")
+            A(f"extern \"C\" int mm_{kn}_bwd_n(long E, const int* rowptr, int nR, const int* eid, const int* send, const float* Y,")
             A("    long y_stride, const float* W, long w_stride, const float* X, long x_stride, const float* gO, long g_stride,")
             A("    float* gW, long gw_stride, float* gYp, long gy_cb_stride, float* gX, long gx_stride, hipStream_t stream) {")
             A("  MM_CHECK_ARG(nR >= 0, \"bad sizes\");")
@@ -920,14 +974,27 @@ def tpw_source(tab, name):
             A(f"  MM_CHECK_ARG(!gW || gw_stride >= {nW * C}, \"gW row stride\");")
             A(f"  MM_CHECK_ARG(!gX || gx_stride >= {nX * C}, \"gX row stride\");")
         A("  if (nR == 0) return MM_OK;")
-        A(f"  dim3 grid((unsigned)(((long)nR * {nh_k} + 3) / 4)), block(256);")
+        A(f"  const long waves = (long)nR * {nh_k};")
+        A("  // E < 0: unknown, shared where the receivers alone leave most of the chip idle")
+        A(f"  const bool shared = E < 0 ? waves <= 2048 : {few} && E >= {_share_edges(state)}L * nR;")
+        A("  dim3 grid((unsigned)(shared ? waves : (waves + 3) / 4)), block(256);")
         if kind == "fwd":
-            A(f"  hipLaunchKernelGGL(mm_{kn}_fwd_kernel, grid, block, 0, stream, rowptr, nR, eid, send, Y, y_stride, W,")
+            A(f"  hipLaunchKernelGGL(shared ? mm_{kn}_fwd_shared_kernel : mm_{kn}_fwd_kernel, grid, block, 0, stream, rowptr, nR, eid, send, Y, y_stride, W,")
             A("                     w_stride, X, x_stride, out, out_stride);")
         else:
-            A(f"  hipLaunchKernelGGL(mm_{kn}_bwd_kernel, grid, block, 0, stream, rowptr, nR, eid, send, Y, y_stride, W,")
+            A(f"  hipLaunchKernelGGL(shared ? mm_{kn}_bwd_shared_kernel : mm_{kn}_bwd_kernel, grid, block, 0, stream, rowptr, nR, eid, send, Y, y_stride, W,")
             A("                     w_stride, X, x_stride, gO, g_stride, gW, gw_stride, gYp, gy_cb_stride, gX, gx_stride);")
         A(f"  return mm::launch_status(\"mm_{kn}_{kind}\");")
+        A("}")
+        A("")
+        args = ("rowptr, nR, eid, send, Y, y_stride, W, w_stride, X, x_stride, " +
+                ("out, out_stride" if kind == "fwd" else "gO, g_stride, gW, gw_stride, gYp, gy_cb_stride, gX, gx_stride"))
+        A(f"extern \"C\" int mm_{kn}_{kind}(const int* rowptr, int nR, const int* eid, const int* send, const float* Y,")
+        A("    long y_stride, const float* W, long w_stride, const float* X, long x_stride,")
+        A("    float* out, long out_stride, hipStream_t stream) {" if kind == "fwd" else
+          "    const float* gO, long g_stride, float* gW, long gw_stride, float* gYp, long gy_cb_stride, float* gX,\n"
+          "    long gx_stride, hipStream_t stream) {")
+        A(f"  return mm_{kn}_{kind}_n(-1, {args}, stream);")
         A("}")
         A("")
     return "\n".join(L)

@@ -64,16 +64,18 @@ class ChannelwiseTP:
             raise ValueError(f"edge_attrs_irreps must be the harmonics l = 0 .. L in order, not {edge_attrs_irreps!r}")
         return cls([l for (_, l, _) in node], len(ls) - 1, tuple(l for (_, l, _) in target))
 
-    def kernels(self):
-        """(forward, backward) entry points of this table (arguments of mm_tpw_l1_fwd / _bwd): the library's for a
-        compiled table, else those built for the table (tp_jit; the first use builds them)."""
+    def kernels(self, edge_count=False):
+        """(forward, backward) entry points of this table (arguments of mm_tpw_l1_fwd / _bwd; with edge_count those
+        of mm_tpw_l1_fwd_n / _bwd_n): the library's for a compiled table, else those built for the table (tp_jit; the
+        first use builds them)."""
         if self.nY > 16:
             raise NotImplementedError("the kernels take spherical harmonics up to l = 3 (16 components), "
                                       f"not {self.nY} (sh_lmax = {self.sh_lmax})")
         if self.name is not None:
-            return getattr(K, f"mm_tpw_{self.name}_fwd"), getattr(K, f"mm_tpw_{self.name}_bwd")
+            n = "_n" if edge_count else ""
+            return getattr(K, f"mm_tpw_{self.name}_fwd{n}"), getattr(K, f"mm_tpw_{self.name}_bwd{n}")
         from . import tp_jit
-        return tp_jit.kernels(self.table)
+        return tp_jit.kernels(self.table, edge_count)
 
     def __repr__(self):
         kern = self.name if self.name is not None else "built on first use"
@@ -101,23 +103,27 @@ def receiver_csr(edge_index, n_nodes, n_send_rows):
     if E >= 2 ** 31:
         raise ValueError("more than 2^31 - 1 edges")
     dev = edge_index.device
-    send = edge_index[0].to(torch.int32).contiguous()
-    recv = edge_index[1].long()
     if E == 0:
-        return torch.zeros(n_nodes + 1, dtype=torch.int32, device=dev), None, send
-    stats = torch.stack([send.min().long(), send.max().long(), recv.min(), recv.max(),
-                         (recv[1:] >= recv[:-1]).all().long() if E > 1 else torch.ones((), dtype=torch.long,
-                                                                                        device=dev)]).tolist()
-    smin, smax, rmin, rmax, is_sorted = stats
-    if smin < 0 or smax >= n_send_rows:
-        raise IndexError(f"sender index out of range [0, {n_send_rows}): min {smin}, max {smax}")
-    if rmin < 0 or rmax >= n_nodes:
-        raise IndexError(f"receiver index out of range [0, {n_nodes}): min {rmin}, max {rmax}")
-    counts = torch.bincount(recv, minlength=n_nodes)
-    rowptr = torch.zeros(n_nodes + 1, dtype=torch.int64, device=dev)
-    torch.cumsum(counts, 0, out=rowptr[1:])
-    eid = None if is_sorted else torch.argsort(recv, stable=True).to(torch.int32)
-    return rowptr.to(torch.int32), eid, send
+        return (torch.zeros(n_nodes + 1, dtype=torch.int32, device=dev), None,
+                edge_index[0].to(torch.int32).contiguous())
+    if edge_index.dtype not in (torch.int32, torch.int64):
+        edge_index = edge_index.long()
+    send, recv = edge_index[0], edge_index[1]
+    out = torch.empty(E + n_nodes + 1, dtype=torch.int32, device=dev)
+    send32, rowptr = out[:E], out[E:]
+    bad = torch.zeros(3, dtype=torch.int32, device=dev)
+    K.mm_edge_csr(send, send.stride(0), recv, recv.stride(0), recv.dtype == torch.int64, E, n_nodes, n_send_rows,
+                  send32, rowptr, bad, stream())
+    bad_send, bad_recv, unsorted = bad.tolist()
+    if bad_send:
+        raise IndexError(f"sender index out of range [0, {n_send_rows}): min {int(send.min())}, max {int(send.max())}")
+    if bad_recv:
+        raise IndexError(f"receiver index out of range [0, {n_nodes}): min {int(recv.min())}, max {int(recv.max())}")
+    if not unsorted:
+        return rowptr, None, send32
+    recv, eid = torch.sort(recv.to(torch.int32), stable=True)
+    K.mm_edge_csr(None, 0, recv, 1, 0, E, n_nodes, n_send_rows, None, rowptr, bad, stream())
+    return rowptr, eid.to(torch.int32), send32
 
 
 def _check(t, name, cols):
@@ -133,7 +139,7 @@ def _check(t, name, cols):
 class _FusedConvFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, X, Y, W, edge_index, desc):
-        fwd, bwd = desc.kernels()
+        fwd, bwd = desc.kernels(edge_count=True)
         X = _check(X, "node_feats", desc.nX * C)
         Y = _check(Y, "edge_attrs", desc.nY)
         W = _check(W, "tp_weights", desc.nW * C)
@@ -145,7 +151,7 @@ class _FusedConvFn(torch.autograd.Function):
         n = X.shape[0]
         rowptr, eid, send = receiver_csr(edge_index, n, n)
         out = torch.empty(n, desc.nO * C, dtype=torch.float32, device=X.device)
-        fwd(rowptr, n, eid, send, Y, Y.stride(0), W, W.stride(0), X, X.stride(0), out, out.stride(0), stream())
+        fwd(E, rowptr, n, eid, send, Y, Y.stride(0), W, W.stride(0), X, X.stride(0), out, out.stride(0), stream())
         ctx.save_for_backward(X, Y, W, rowptr, send, eid if eid is not None else torch.empty(0))
         ctx.has_eid = eid is not None
         ctx.desc, ctx.bwd = desc, bwd
@@ -164,11 +170,11 @@ class _FusedConvFn(torch.autograd.Function):
         gYp = torch.empty(desc.gy_parts, E, 16, dtype=torch.float32, device=X.device) if (ny and E) else None
         gW = torch.empty_like(W) if nw else None
         if E and (nx or ny or nw):
-            ctx.bwd(rowptr, n, eid, send, Y, Y.stride(0), W, W.stride(0), X, X.stride(0), gO, gO.stride(0), gW,
+            ctx.bwd(E, rowptr, n, eid, send, Y, Y.stride(0), W, W.stride(0), X, X.stride(0), gO, gO.stride(0), gW,
                     W.stride(0), gYp, E * 16, gX, X.stride(0), stream())
         gY = None
         if ny:
-            gY = gYp.sum(0)[:, :desc.nY] if E else torch.zeros(0, desc.nY, dtype=Y.dtype, device=Y.device)
+            gY = (gYp.sum(0) if desc.gy_parts > 1 else gYp[0])[:, :desc.nY] if E else torch.zeros(0, desc.nY, dtype=Y.dtype, device=Y.device)
         if nw and not E:
             gW = torch.zeros_like(W)
         return gX, gY, gW, None, None

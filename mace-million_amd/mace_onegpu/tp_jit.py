@@ -108,9 +108,9 @@ def build(table, force=False):
     return so
 
 
-def kernels(table):
-    """(forward, backward) entry points of the table's kernels, with the arguments of mm_tpw_l1_fwd / _bwd; built
-    first when needed."""
+def kernels(table, edge_count=False):
+    """(forward, backward) entry points of the table's kernels, with the arguments of mm_tpw_l1_fwd / _bwd (with
+    edge_count: of mm_tpw_l1_fwd_n / _bwd_n); built first when needed."""
     key = table_key(table)
     with _lock:
         if key not in _loaded:
@@ -123,9 +123,11 @@ def kernels(table):
                 return so.mm_last_error().decode()
 
             fns = []
-            for kind, sig in (("fwd", SIG_FWD), ("bwd", SIG_BWD)):
+            for kind, sig in (("fwd", SIG_FWD), ("bwd", SIG_BWD), ("fwd_n", [ctypes.c_long] + SIG_FWD),
+                              ("bwd_n", [ctypes.c_long] + SIG_BWD)):
                 f = getattr(so, f"mm_tpw_{name}_{kind}")
                 f.argtypes, f.restype = sig, ctypes.c_int
                 fns.append(_Fn(f"mm_tpw_{name}_{kind}", f, err))
-            _loaded[key] = (so, fns[0], fns[1])
-    return _loaded[key][1], _loaded[key][2]
+            _loaded[key] = (so, fns)
+    fns = _loaded[key][1]
+    return tuple(fns[2:]) if edge_count else tuple(fns[:2])
