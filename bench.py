@@ -92,7 +92,7 @@ def conv_algorithmic(name, E, nC, N, tab, Kp=128):
 
 # the HIP sources that define each profiled kernel (a measurement stays valid while these are unchanged)
 KERNEL_SOURCES = {
-    "mm_conv2_bwd_kernel": ("gen/conv_l2.hip", "gen/sh.h", "common.h"),
+    "mm_conv2_bwd_vec_kernel": ("gen/conv_l2v.hip", "gen/polar.h", "common.h"),
     "mm_conv2_fwd_kernel": ("gen/conv_l2.hip", "gen/sh.h", "common.h"),
     "mm_ace1_fwd_kernel": ("ace.hip", "gen/sh.h", "common.h"),
     "mm_ace1_bwd_kernel": ("ace.hip", "gen/sh.h", "common.h"),
@@ -105,6 +105,7 @@ KERNEL_SOURCES = {
     "mm_fill_f32_kernel": ("node.hip", "common.h"),
     "mm_fill_i32_kernel_nl": ("nlist.hip", "common.h"),
 }
+KERNEL_NAMES = {"conv2_bwd": "conv2_bwd_vec"}      # the device kernel where it is not named as the stage
 
 
 def kernel_digest(kernel, read=None):
@@ -219,7 +220,8 @@ def summarize(name, launches, ms_total, B, F, steps):
 
 def engine(name):
     """The unit a kernel's arithmetic runs on: the edge convolutions and the symmetric contractions are fp32 VALU
-    code (v_fma_f32), the layer-1 ACE kernels fp32 MFMA, the linears bf16 MFMA."""
+    code (v_fma_f32; the layer-2 backward takes one of its contractions on fp16 MFMA and is bound by the VALU),
+    the layer-1 ACE kernels fp32 MFMA, the linears bf16 MFMA."""
     if name.startswith("ace1"):
         return "mfma_f32"
     if name == "linear":
@@ -252,7 +254,8 @@ def roofline_of(kernels, workload=None):
     peak = {"valu": VALU_F32_PEAK_TFLOPS, "mfma_f32": MFMA_F32_PEAK_TFLOPS,
             "mfma_bf16": MFMA_F32_PEAK_TFLOPS}[eng]
     compute = intensity > peak * 1e12 / (HBM_PEAK_GBS * 1e9)
-    out = {"kernel": f"mm_{dom}_kernel"}
+    kernel = f"mm_{KERNEL_NAMES.get(dom, dom)}_kernel"
+    out = {"kernel": kernel}
     if compute:
         out.update({"bound": "valu" if eng == "valu" else "mfma", "achieved": round(k["TFLOPs"], 3), "peak": peak,
                     "unit": "TFLOP/s", "frac": round(k["TFLOPs"] / peak, 4),
@@ -260,7 +263,7 @@ def roofline_of(kernels, workload=None):
     else:
         out.update({"bound": "hbm", "achieved": round(k["GBps"], 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                     "frac": round(k["hbm_frac"], 5)})
-    out.update({"traffic": measured_traffic(f"mm_{dom}_kernel", workload) if workload else None,
+    out.update({"traffic": measured_traffic(kernel, workload) if workload else None,
                 "intensity_flop_per_byte": round(intensity, 1),
                 "hbm_achieved_GBps": round(k["GBps"], 2), "hbm_frac": round(k["hbm_frac"], 5),
                 "flop_rate_TFLOPs": round(k["TFLOPs"], 3),
@@ -268,7 +271,9 @@ def roofline_of(kernels, workload=None):
                 "bytes_per_launch": int(k["bytes_per_launch"]), "flops_per_launch": int(k["flops_per_launch"]),
                 "ms_per_launch": round(k["ms_per_launch"], 4), "launches": k["launches"]})
     if compute and eng == "valu":
-        out["note"] = ("the kernel runs on the vector ALUs (v_fma_f32, no packed FP32): 157.3 TFLOP/s needs two VALU "
+        out["note"] = (("the contraction over the harmonics runs on fp16 matrix instructions, the rest " if
+                        dom == "conv2_bwd" else "the kernel runs ") +
+                       "on the vector ALUs (v_fma_f32, no packed FP32): 157.3 TFLOP/s needs two VALU "
                        "instructions from two waves per SIMD issued per quad-cycle (gfx950 dual issue; 151.6 TFLOP/s "
                        "measured for VGPR-operand FMAs); DPP, v_cndmask and SGPR-operand instructions cannot pair")
     return out
@@ -684,6 +689,8 @@ def run_conv(a):
     part = torch.empty(8 * E * 17, device="cuda")
     gX = torch.zeros(nN, 4 * C, device="cuda")
     st = stream()
+    slots = (ws["e_slot"], ws["g_send"], ws["g_n"])
+    K.mm_sender_slots(g.rowptr, nC, g.ls, *slots, st)
     calls = {
         "conv1_fwd": (lambda: K.mm_conv1_fwd(g.rowptr, nC, pk1, eu1, fl.Xs1, C, fl.tab[0], fl.n_tab, fl.M, out1, rho,
                                              st), fl.tables.tp1),
@@ -691,8 +698,8 @@ def run_conv(a):
                                              gA1, part, E * 17, None, st), fl.tables.tp1),
         "conv2_fwd": (lambda: K.mm_conv2_fwd(g.rowptr, nC, pk2, eu2, X2, 4 * C, fl.tab[1], fl.n_tab, fl.M, out2, rho,
                                              st), fl.tables.tp2),
-        "conv2_bwd": (lambda: K.mm_conv2_bwd(g.rowptr, nC, pk2, eu2, X2, 4 * C, fl.tab[1], fl.n_tab, fl.M, fl.inv_h,
-                                             gA2, part, E * 17, gX, st), fl.tables.tp2),
+        "conv2_bwd": (lambda: K.mm_conv2_bwd_vec(g.rowptr, nC, pk2, eu2, X2, 4 * C, fl.tab[1], fl.n_tab, fl.M,
+                                                 fl.inv_h, gA2, part, E * 3, gX, *slots, st), fl.tables.tp2),
     }
     if fl.ace:
         calls["ace1_fwd"] = (lambda: K.mm_ace1_fwd(g.rowptr, nC, pk1, eu1, fl.tab_h, fl.S, fl.S_pad, Bace, rho, st),
@@ -789,16 +796,16 @@ def run_conv(a):
             g.rij.cpu().numpy(), g.recv_local.cpu().numpy(), g.ls.cpu().numpy(), rp_h, E, nC, nN, X2.cpu(),
             gA2.cpu())
         # the same receivers through the GPU kernels: forward output, and the backward of L = gA . out restricted
-        # to them (gA zero elsewhere) -> dL/dX (G1 path) and per-edge dL/dvec (mm_edge_grad, no density term)
+        # to them (gA zero elsewhere) -> dL/dX (G1 path) and per-edge dL/dvec (mm_edge_grad_vec, no density term)
         gAm = gA2.clone()
         gAm[nr_c:] = 0
         gXm = torch.zeros_like(X2)
         partm = torch.empty_like(part)
         PFm = torch.empty(E, 3, device="cuda")
-        K.mm_conv2_bwd(g.rowptr, nC, pk2, eu2, X2, 4 * C, fl.tab[1], fl.n_tab, fl.M, fl.inv_h, gAm, partm, E * 17,
-                       gXm, st)
-        K.mm_edge_grad(E, None, partm, E * 17, 8, torch.zeros(nC, device="cuda"), ws["e_recv"], ws["e_dd"], eu2,
-                       PFm, 0, st)
+        K.mm_conv2_bwd_vec(g.rowptr, nC, pk2, eu2, X2, 4 * C, fl.tab[1], fl.n_tab, fl.M, fl.inv_h, gAm, partm, E * 3,
+                           gXm, *slots, st)
+        K.mm_edge_grad_vec(E, None, partm, E * 3, 8, torch.zeros(nC, device="cuda"), ws["e_recv"], ws["e_dd"], eu2,
+                           PFm, 0, st)
         calls["conv2_fwd"][0]()
         torch.cuda.synchronize()
 
@@ -807,7 +814,7 @@ def run_conv(a):
         oracle_check = {"receivers": nr_c, "edges": ne_c, "tolerance": 1e-4,
                         "out_max_rel": rel(out2[:nr_c].view(nr_c, 40, C), o_out),
                         "dL_dvec_max_rel": rel(PFm[:ne_c], o_gv),
-                        # mm_conv2_bwd's dL/dX rows are 16-channel-block-major: gX[s][cb][k][16]
+                        # mm_conv2_bwd_vec's dL/dX rows are 16-channel-block-major: gX[s][cb][k][16]
                         "dL_dX_max_rel": rel(gXm[:nn_c].view(nn_c, 8, 4, 16).permute(0, 2, 1, 3).reshape(nn_c, 4, C),
                                              o_gx)}
         oracle_check["pass"] = all(oracle_check[k] < 1e-4 for k in ("out_max_rel", "dL_dvec_max_rel",

@@ -105,6 +105,11 @@ int mm_edge_geom_pos(int E, const int* E_dev /* nullable */, const double* pos, 
 int mm_edge_grad(int E, const int* E_dev /* nullable */, const float* part, long part_stride, int n_part,
                  const float* g_rho, const int* e_recv, const float* e_dd, const float* e_u, float* pair_force,
                  int accumulate, mm_stream_t stream);
+/* the same from the partials of mm_conv2_bwd_vec: part[cb][e][3] = (dL/dr, dL/dtheta, (1 / sin theta) dL/dphi) in the
+ * polar frame of the edge direction (z axis; phi = 0 at the poles) */
+int mm_edge_grad_vec(int E, const int* E_dev /* nullable */, const float* part, long part_stride, int n_part,
+                     const float* g_rho, const int* e_recv, const float* e_dd, const float* e_u, float* pair_force,
+                     int accumulate, mm_stream_t stream);
 
 /* ---------------------------------------------------------------------------------------------- (2)+(3) edge conv
  * Replace conv_spline.ConvSpline.forward / gen_fwd (conv_spline.py:38-94, 294-301), spline_w._w_fwd
@@ -140,6 +145,19 @@ int mm_conv0123_bwd(const int* rowptr, int nC, const float* e_pk, const float* e
 int mm_conv2_bwd_det(const int* rowptr, int nC, const float* e_pk, const float* e_u, const float* X, int x_stride,
                      const float* tab, int n_tab, int M, float inv_h, const float* gA, float* part, long part_stride,
                      float* gXe, mm_stream_t stream);
+/* mm_conv2_bwd / mm_conv2_bwd_det with the angular derivative taken in the kernel, on the matrix cores: three numbers
+ * per edge and channel block, part[cb][e][3] (as mm_edge_grad_vec reads them), instead of dL/dr and 16 dL/dY_m; gX and
+ * gXe as above.  One channel block's tables (n_tab tables) must stay below 4 GiB.
+ * mm_sender_slots prepares mm_conv2_bwd_vec's accumulation of gX for each group of 4 consecutive receivers, once per
+ * edge list: send [E] = the senders of e_pk; e_slot [E + 64], g_send [ceil(nC / 4)][208], g_n [ceil(nC / 4)]. */
+int mm_sender_slots(const int* rowptr, int nC, const int* send, unsigned char* e_slot, int* g_send, int* g_n,
+                    mm_stream_t stream);
+int mm_conv2_bwd_vec(const int* rowptr, int nC, const float* e_pk, const float* e_u, const float* X, int x_stride,
+                     const float* tab, int n_tab, int M, float inv_h, const float* gA, float* part, long part_stride,
+                     float* gX, const unsigned char* e_slot, const int* g_send, const int* g_n, mm_stream_t stream);
+int mm_conv2_bwd_vec_det(const int* rowptr, int nC, const float* e_pk, const float* e_u, const float* X, int x_stride,
+                         const float* tab, int n_tab, int M, float inv_h, const float* gA, float* part,
+                         long part_stride, float* gXe, mm_stream_t stream);
 
 /* ---------------------------------------------------------------------------------------------- layer-1 ACE form
  * Replace ace_layer1.ACELayer1.message (ace_layer1.py:58-85) and its autograd backward: the exact density-projection

@@ -9,6 +9,7 @@
 // mm_edge_grad: dL/dv_e = dL/dr u + (I - u u^T) grad_u(sum_m dL/dY_m Y_m) / r, with dL/dr and dL/dY summed
 // over the 8 channel blocks of the convolution backward and the density term g_rho[recv] * d'(r) added.
 #include "common.h"
+#include "gen/polar.h"
 #include "gen/sh.h"
 #include "mic.h"
 
@@ -175,6 +176,44 @@ __global__ void mm_edge_grad_kernel(int E, const float* __restrict__ part, long 
   }
 }
 
+// The same assembly from the three-number partials of mm_conv2_bwd_vec: (dL/dr, dL/dtheta, (1/sin theta) dL/dphi) in
+// the polar frame of the edge direction, summed over the n_part channel blocks.
+__global__ void mm_edge_grad_vec_kernel(int E, const float* __restrict__ part, long part_stride, int n_part,
+                                        const float* __restrict__ g_rho, const int* __restrict__ e_recv,
+                                        const float* __restrict__ e_dd, const float4* __restrict__ e_u,
+                                        float* __restrict__ pf, int accumulate, const int* __restrict__ E_dev) {
+  const int e = blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= (E_dev ? *E_dev : E)) return;   // E_dev: the edge count in device memory (graph replays)
+  float gr = 0.f, gt = 0.f, gp = 0.f;
+  for (int cb = 0; cb < n_part; ++cb) {
+    const float* __restrict__ pp = part + (size_t)cb * part_stride + (size_t)e * 3;
+    gr += pp[0];
+    gt += pp[1];
+    gp += pp[2];
+  }
+  if (g_rho) gr += g_rho[e_recv[e]] * e_dd[e];
+  const float4 u = e_u[e];
+  float s, cp, sp;
+  mm_polar(u.x, u.y, s, cp, sp);
+  const float ir = 1.0f / u.w;
+  gt *= ir;
+  gp *= ir;
+  // v = r u: dL/dv = gr u + (gt theta + gp phi) / r, theta = (z cp, z sp, -s), phi = (-sp, cp, 0)
+  const float gx = fmaf(gr, u.x, fmaf(gt, u.z * cp, -gp * sp));
+  const float gy = fmaf(gr, u.y, fmaf(gt, u.z * sp, gp * cp));
+  const float gz = fmaf(gr, u.z, -gt * s);
+  float* __restrict__ o = pf + 3 * (size_t)e;
+  if (accumulate) {
+    o[0] += gx;
+    o[1] += gy;
+    o[2] += gz;
+  } else {
+    o[0] = gx;
+    o[1] = gy;
+    o[2] = gz;
+  }
+}
+
 static int make_density(MMDensity& dp, const float* w, int nb, float r_max, int p) {
   if (nb < 1 || nb > MM_MAX_BESSEL) return MM_EINVAL;
   for (int i = 0; i < MM_MAX_BESSEL; ++i) dp.w[i] = i < nb ? w[i] : 0.f;
@@ -223,4 +262,14 @@ extern "C" int mm_edge_grad(int E, const int* E_dev, const float* part, long par
   hipLaunchKernelGGL(mm_edge_grad_kernel, dim3((E + 255) / 256), dim3(256), 0, stream, E, part, part_stride, n_part,
                      g_rho, e_recv, e_dd, (const float4*)e_u, pf, accumulate, E_dev);
   return mm::launch_status("mm_edge_grad");
+}
+
+extern "C" int mm_edge_grad_vec(int E, const int* E_dev, const float* part, long part_stride, int n_part,
+                                const float* g_rho, const int* e_recv, const float* e_dd, const float* e_u, float* pf,
+                                int accumulate, hipStream_t stream) {
+  MM_CHECK_ARG(E >= 0 && n_part >= 0, "bad sizes");
+  if (E == 0) return MM_OK;
+  hipLaunchKernelGGL(mm_edge_grad_vec_kernel, dim3((E + 255) / 256), dim3(256), 0, stream, E, part, part_stride,
+                     n_part, g_rho, e_recv, e_dd, (const float4*)e_u, pf, accumulate, E_dev);
+  return mm::launch_status("mm_edge_grad_vec");
 }

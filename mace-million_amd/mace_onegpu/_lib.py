@@ -48,12 +48,16 @@ SIGNATURES = {
     "mm_ace1_bwd": [P, I, P, P, P, I, I, P, F, P, P],
     "mm_spline_coeffs_flat": [P, I, I, D, D, I, P, P],
     "mm_edge_grad": [I, P, P, L, I, P, P, P, P, P, I, P],
+    "mm_edge_grad_vec": [I, P, P, L, I, P, P, P, P, P, I, P],
     # convolutions (generated)
     "mm_conv1_fwd": [P, I, P, P, P, I, P, I, I, P, P, P],
     "mm_conv2_fwd": [P, I, P, P, P, I, P, I, I, P, P, P],
     "mm_conv1_bwd": [P, I, P, P, P, I, P, I, I, F, P, P, L, P, P],
     "mm_conv2_bwd": [P, I, P, P, P, I, P, I, I, F, P, P, L, P, P],
     "mm_conv2_bwd_det": [P, I, P, P, P, I, P, I, I, F, P, P, L, P, P],
+    "mm_sender_slots": [P, I, P, P, P, P, P],
+    "mm_conv2_bwd_vec": [P, I, P, P, P, I, P, I, I, F, P, P, L, P, P, P, P, P],
+    "mm_conv2_bwd_vec_det": [P, I, P, P, P, I, P, I, I, F, P, P, L, P, P],
     "mm_conv0123_fwd": [P, I, P, P, P, I, P, I, I, P, P, P],
     "mm_conv0123_bwd": [P, I, P, P, P, I, P, I, I, F, P, P, L, P, P],
     "mm_gather_rows_csr": [P, P, P, L, I, P, L, I, P],

@@ -10,6 +10,7 @@ HIP code once, at build time, with every coupling coefficient a compile-time con
                     (forward) and its backward (d r, d Y per edge, optional d X scattered to senders)
   gen/symc_l{1,2}.hip  per-species correlation-3 symmetric contraction, forward and backward
   gen/conv_l0123.hip   the same fused convolution for the literal 0e+1o+2e+3o node features (23 paths)
+  gen/conv_l2v.hip  the layer-2 backward on the matrix cores; gen/polar.h its harmonics
   gen/tpw_*.hip     channelwise TP with explicit per-edge weights (FusedConvTP), forward and backward
 
 Kernel/launch design is documented in the generated files' headers.
@@ -577,6 +578,482 @@ def conv_source(tab, layer, need_gx, opts=None):
         A("                     gA, part, part_stride, gXe);")
         A(f"  return mm::launch_status(\"mm_{name}_bwd_det\");")
         A("}")
+    return "\n".join(L) + "\n"
+
+
+# ----------------------------------------------------------------------------- layer-2 backward on the matrix cores
+# The layer-2 edge-convolution backward on the matrix cores.
+#
+# The backward of the fused edge convolution (conv_source) evaluates, per edge, channel c and (path w, input
+# component k), the sum u_wk = sum_m Y_m G[w, k, m, c] and contracts it with the sender features and the radial weights.
+# G is a constant of the receiver, Y of the edge, so over the edges of one receiver u is a matrix product: rows = 16
+# edges, columns = 16 channels, inner index = the harmonics m of the path's degree l2.  The same product with the
+# harmonics' polar and azimuthal derivatives in place of Y gives du/dtheta and du/dphi, from which the angular force
+# follows: the kernel returns three numbers per edge (dL/dr and two tangential derivatives) where the per-harmonic form
+# returns 17.
+#
+# Products at fp32 accuracy from fp16 matrix instructions: each operand is the sum of two fp16 values (h0 = fp16(x), h1 =
+# fp16(x - h0), |x - h0 - h1| <= 2^-24 |x|; G is scaled per channel into the fp16 range by a power of two, the harmonics are
+# below 6), and all four piece products are taken, side by side along the inner index: k-group 2 a + b of the instruction
+# holds piece a of Y and piece b of G.
+#
+# Measured (16,384 receivers x 90 edges, 1.47 M edges): 2.42 -> 2.20 ms, the edge gradient that reads its partials 0.149 ->
+# 0.028 ms, mm_sender_slots 9 us; the layer-2 pass of that chunk 4.50 -> 4.18 ms.  Errors against 64 bits 5.3e-7 -> 5.2e-7.
+# Bound by VALU issue (the spline evaluation, the two products with X and W, the operand split) at 2 waves per SIMD:
+# about 0.2 ms of the matrix time is exposed, 0.25 ms goes into each receiver's operand B, 0.15 ms into the LDS adds.
+# Why this form: fp32 matrix instructions (16x16x1) hold the SIMD's vector ALU while they run (2.64 ms), the fp16 ones
+# run beside it; a tile of 16 edges x 16 channels is one instruction's rows and columns, so lane (edge group, channel)
+# holds four edges of its channel and reads X, W and G rows of 64 contiguous bytes; a third wave per SIMD does not fit (252
+# registers, of which 64 hold B), deeper prefetch spills.
+def _polar_basis(u):
+    """[n, 16] B_m of unit vectors: z-polynomial x sin^|m| theta x {cos, sin}(|m| phi), the functions that
+    mm_polar_operands evaluates (value type)."""
+    x, y, z = u.T
+    s = np.hypot(x, y)
+    ph = np.arctan2(y, x)
+    f = {(1, 0): z, (1, 1): s, (2, 0): 3 * z * z - 1, (2, 1): z * s, (2, 2): s * s,
+         (3, 0): z * (5 * z * z - 3), (3, 1): s * (5 * z * z - 1), (3, 2): z * s * s, (3, 3): s ** 3}
+    out = np.ones((len(u), 16))
+    for (l, m), v in f.items():
+        out[:, l * l + l + m] = v * np.cos(m * ph)
+        if m:
+            out[:, l * l + l - m] = v * np.sin(m * ph)
+    return out
+
+
+def polar_norms():
+    """c_m with Y_m = c_m B_m, checked at random directions."""
+    rng = np.random.default_rng(0)
+    u = rng.normal(size=(64, 3))
+    u /= np.linalg.norm(u, axis=1, keepdims=True)
+    Y = np.stack(o3.sh_cartesian(u[:, 0], u[:, 1], u[:, 2]), 1)
+    B = _polar_basis(u)
+    j = np.argmax(np.abs(B), 0)
+    c = np.array([Y[j[m], m] / B[j[m], m] for m in range(16)])
+    if np.abs(B * c - Y).max() > 1e-12:
+        raise AssertionError("the polar basis is not proportional to the harmonics")
+    return c
+
+
+BWD_VEC_HEADER = """// generated by mace_onegpu/codegen.py -- layer-2 edge convolution, backward, on the matrix cores
+#include "../common.h"
+#include "polar.h"
+
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef _Float16 half4v __attribute__((ext_vector_type(4)));
+typedef _Float16 half8v __attribute__((ext_vector_type(8)));
+typedef float float2v __attribute__((ext_vector_type(2)));
+typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+
+// x = h0 + h1 (fp16, round to nearest even; the difference is exact in fp32): |x - h0 - h1| <= 2^-24 |x| for the
+// scaled operands below.  Two values at a time.
+__device__ __forceinline__ void mm_split2_f16(float x, float y, unsigned& h0, unsigned& h1) {
+  const half2v a = __builtin_convertvector(float2v{x, y}, half2v);
+  const float2v r = float2v{x, y} - __builtin_convertvector(a, float2v);
+  h0 = __builtin_bit_cast(unsigned, a);
+  h1 = __builtin_bit_cast(unsigned, __builtin_convertvector(r, half2v));
+}
+
+__device__ __forceinline__ unsigned mm_load_u32(const unsigned char* p) {
+  unsigned v;
+  __builtin_memcpy(&v, p, 4);
+  return v;
+}
+
+// Slots of the distinct senders of each group of GROUP consecutive receivers (spatially close in the Morton order, so
+// they share most senders): e_slot[e] = the slot of edge e's sender in its group (255: none, the sender found no slot or
+// the edge lies beyond the group's first SLOT_EDGES), g_send[group][slot] = the sender, g_n[group] = slots in use.
+// Once per chunk, for the 8 channel blocks of the backward (which hashed the senders 8 times before).
+#define MM_SLOT_HASH 2048
+extern "C" __global__ void __launch_bounds__(256)
+mm_sender_slots_kernel(const int* __restrict__ rowptr, int nC, const int* __restrict__ send,
+    unsigned char* __restrict__ e_slot, int* __restrict__ g_send, int* __restrict__ g_n) {
+  __shared__ int hkey[MM_SLOT_HASH];
+  __shared__ unsigned char hslot[MM_SLOT_HASH];
+  __shared__ int nslot;
+  const int i0 = blockIdx.x * GROUP, tid = threadIdx.x;
+  const int E0 = rowptr[i0], nE = rowptr[min(i0 + GROUP, nC)] - E0, nH = min(nE, SLOT_EDGES);
+  for (int h = tid; h < MM_SLOT_HASH; h += 256) hkey[h] = -1;
+  if (tid == 0) nslot = 0;
+  __syncthreads();
+  for (int j = tid; j < nH; j += 256) {   // at most SLOT_EDGES keys: the probing ends at a free entry
+    const int s = send[E0 + j];
+    unsigned h = ((unsigned)s * 2654435761u) >> 21;
+    while (true) {
+      const int prev = atomicCAS(&hkey[h], -1, s);
+      if (prev == -1) {
+        const int sl = atomicAdd(&nslot, 1);
+        hslot[h] = sl < SLOTS ? (unsigned char)sl : 255;
+        if (sl < SLOTS) g_send[(size_t)blockIdx.x * SLOTS + sl] = s;
+      }
+      if (prev == -1 || prev == s) break;
+      h = (h + 1) & (MM_SLOT_HASH - 1);
+    }
+  }
+  __syncthreads();
+  for (int j = tid; j < nE; j += 256) {
+    unsigned char sl = 255;
+    if (j < nH) {
+      const int s = send[E0 + j];
+      unsigned h = ((unsigned)s * 2654435761u) >> 21;
+      while (hkey[h] != s) h = (h + 1) & (MM_SLOT_HASH - 1);
+      sl = hslot[h];
+    }
+    e_slot[E0 + j] = sl;
+  }
+  if (tid == 0) g_n[blockIdx.x] = min(nslot, SLOTS);
+}
+
+extern "C" int mm_sender_slots(const int* rowptr, int nC, const int* send, unsigned char* e_slot, int* g_send, int* g_n,
+    hipStream_t stream) {
+  MM_CHECK_ARG(nC >= 0, "bad sizes");
+  if (nC == 0) return MM_OK;
+  hipLaunchKernelGGL(mm_sender_slots_kernel, dim3((nC + GROUP - 1) / GROUP), dim3(256), 0, stream, rowptr, nC, send,
+                     e_slot, g_send, g_n);
+  return mm::launch_status("mm_sender_slots");
+}
+"""
+
+POLAR_HEADER = """// generated by mace_onegpu/codegen.py -- harmonics of an edge direction and their tangential derivatives
+#pragma once
+
+// Polar frame of a unit vector (x, y, z): s = sin(theta), (cp, sp) = (cos, sin)(phi).  At the poles phi = 0.
+__device__ __forceinline__ void mm_polar(float x, float y, float& s, float& cp, float& sp) {
+  const float s2 = fmaf(x, x, y * y);
+  const bool pole = s2 < 1e-30f;
+  const float r0 = __builtin_amdgcn_rsqf(pole ? 1.f : s2);
+  const float r = r0 * fmaf(-0.5f * s2 * r0, r0, 1.5f);   // one Newton step
+  s = pole ? 0.f : s2 * r;
+  cp = pole ? 1.f : x * r;
+  sp = pole ? 0.f : y * r;
+}
+
+// A-operand values of one edge: P[m], m = 1..15, of the basis B_lm = F_lm(z, s) {cos, sin}(|m| phi) (Y_m = c_m B_m, the
+// c_m folded into the other operand): type 0 the value, type 1 d/dtheta, type 2 (1 / sin(theta)) d/dphi.  The three
+// types differ in one scalar factor per (l, |m|) and in the azimuthal pair, so a lane evaluates its own type only.
+__device__ __forceinline__ void mm_polar_operands(float z, float s, float cp, float sp, int type, float (&P)[16]) {
+  const bool t0 = type == 0, t1 = type == 1;
+  const float z2 = z * z, s2 = s * s, zs = z * s;
+  const float f5 = fmaf(5.f, z2, -1.f);
+  // F_lm | dF_lm/dtheta | |m| F_lm / s
+  const float f10 = t0 ? z : t1 ? -s : 0.f;
+  const float f11 = t0 ? s : t1 ? z : 1.f;
+  const float f20 = t0 ? fmaf(3.f, z2, -1.f) : t1 ? -6.f * zs : 0.f;
+  const float f21 = t0 ? zs : t1 ? z2 - s2 : z;
+  const float f22 = t0 ? s2 : t1 ? 2.f * zs : 2.f * s;
+  const float f30 = t0 ? z * fmaf(5.f, z2, -3.f) : t1 ? -s * fmaf(15.f, z2, -3.f) : 0.f;
+  const float f31 = t0 ? s * f5 : t1 ? z * fmaf(-10.f, s2, f5) : f5;
+  const float f32 = t0 ? z * s2 : t1 ? s * fmaf(2.f, z2, -s2) : 2.f * zs;
+  const float f33 = t0 ? s * s2 : t1 ? 3.f * z * s2 : 3.f * s2;
+  const float c2 = fmaf(cp, cp, -sp * sp), q2 = 2.f * cp * sp;
+  const float c3 = fmaf(cp, c2, -sp * q2), q3 = fmaf(sp, c2, cp * q2);
+  const bool t2 = type == 2;
+  // azimuthal pair (cos, sin)(m phi), or its derivative / m: (-sin, cos)
+  const float a1 = t2 ? -sp : cp, b1 = t2 ? cp : sp;
+  const float a2 = t2 ? -q2 : c2, b2 = t2 ? c2 : q2;
+  const float a3 = t2 ? -q3 : c3, b3 = t2 ? c3 : q3;
+  P[0] = t0 ? 1.f : 0.f;
+  P[1] = f11 * b1; P[2] = f10; P[3] = f11 * a1;
+  P[4] = f22 * b2; P[5] = f21 * b1; P[6] = f20; P[7] = f21 * a1; P[8] = f22 * a2;
+  P[9] = f33 * b3; P[10] = f32 * b2; P[11] = f31 * b1; P[12] = f30; P[13] = f31 * a1; P[14] = f32 * a2;
+  P[15] = f33 * a3;
+}
+"""
+
+GROUP = 4        # receivers per workgroup, one per wave
+SLOTS = 208      # LDS accumulators (64 floats) of a workgroup's distinct senders (at most a workgroup's threads)
+SLOT_EDGES = 1024   # edges of a group that take part in the slots
+
+
+def conv2_bwd_vec_source(tab, depth=2):
+    """Backward kernels mm_conv2_bwd_vec (dL/dX pooled per receiver group in LDS) and mm_conv2_bwd_vec_det (a row of
+    dL/dX per edge)."""
+    nX, nW, nO, terms = tab["nX"], tab["nW"], tab["nO"], tab["terms"]
+    norm = polar_norms()
+    G = OrderedDict()
+    for (w, k, m, o, cf) in terms:
+        G.setdefault((w, k, m), []).append((o, cf * norm[m]))
+    gmax = max(sum(abs(c) for _, c in lst) for lst in G.values())
+    # |G| <= gmax max|g|; the operand is scaled to at most 2^15
+    b_exp = 14 - int(np.ceil(np.log2(gmax)))
+    xoff = o3.Irreps(tab["in_ls"]).offsets
+    paths = []                                  # (w, l2, [k])
+    for w, (i1, l1, l2, l3) in enumerate(tab["paths"]):
+        paths.append((w, l2, [xoff[i1] + a for a in range(2 * l1 + 1)]))
+    steps = sorted([p for p in paths if p[1]], key=lambda p: (-p[1], p[0])) + [p for p in paths if not p[1]]
+    n = len(steps)
+    degrees = sorted({p[1] for p in paths if p[1]}, reverse=True)
+    L = [BWD_VEC_HEADER.replace("SLOT_EDGES", str(SLOT_EDGES)).replace("MM_SLOT_HASH", "@H@").replace("SLOTS", str(SLOTS))
+         .replace("GROUP", str(GROUP)).replace("@H@", "MM_SLOT_HASH")]
+    A = L.append
+
+    def gexpr(w, k, m):
+        e = None
+        for (o, cc) in G.get((w, k, m), []):
+            if e is None:
+                e = f"g{o}" if abs(cc - 1) < 1e-12 else f"{_f(cc)} * g{o}"
+            else:
+                e = f"fmaf({_f(cc)}, g{o}, {e})"
+        return e or "0.f"
+
+    def kernel(name, mode):
+        pool = mode == "pool"
+        A(f"extern \"C\" __global__ void __launch_bounds__({64 * GROUP}, 2)")
+        A(f"{name}(const int* __restrict__ rowptr, int nC, const floatx4* __restrict__ e_pk,")
+        A("    const floatx4* __restrict__ e_u, const float* __restrict__ X, int x_stride,")
+        A("    const floatx4* __restrict__ tab, int tab_cb_stride, float inv_h,")
+        A("    const float* __restrict__ gA, float* __restrict__ part, long part_stride, float* __restrict__ gX" +
+          (",\n    const unsigned char* __restrict__ e_slot, const int* __restrict__ g_send,\n"
+           "    const int* __restrict__ g_n) {" if pool else ") {"))
+        A("  const int cb = mm_xcd_channel_block();")
+        A(f"  __shared__ uint4v ya_all[{GROUP * 3 * len(degrees) * 32}];   // per wave: [type][degree][edge][piece] operand rows")
+        A(f"  const int grp = blockIdx.x >> 3, i = grp * {GROUP} + (threadIdx.x >> 6);")
+        if pool:
+            A(f"  __shared__ floatx4 gxs4[{SLOTS * 4 * nX}];   // [slot][component][16 channels]")
+            A(f"  __shared__ int ssend[{SLOTS}];")
+            A("  float* __restrict__ gxs = (float*)gxs4;")
+            A("  const int ns = g_n[grp];")
+            A("  const int ir = min(i, nC - 1);   // waves past the last receiver prepare for it and take no edges")
+        else:
+            A("  if (i >= nC) return;")
+            A("  const int ir = i;")
+        A("  const int lane = threadIdx.x & 63, cl = lane & 15, eg = lane >> 4;")
+        A(f"  uint4v* __restrict__ ya = ya_all + (threadIdx.x >> 6) * {3 * len(degrees) * 32};")
+        A("  const int c = cb * 16 + cl;")
+        A("  const int e0 = rowptr[ir], e1 = i < nC ? rowptr[ir + 1] : e0;")
+        A("  const char* __restrict__ tcb = (const char*)(tab + (size_t)cb * tab_cb_stride);")
+        A(f"  const float* __restrict__ gp = gA + (size_t)ir * {nO * C} + c;")
+        for o in range(nO):
+            A(f"  float g{o} = gp[{o * C}];")
+        A("  // power-of-two scale of this channel's constants into the fp16 range")
+        mx = "0.f"
+        for o in range(0, nO, 2):
+            mx = f"fmaxf(fmaxf(fabsf(g{o}), fabsf(g{o + 1})), {mx})" if o + 1 < nO else f"fmaxf(fabsf(g{o}), {mx})"
+            if o % 8 == 6 or o + 2 >= nO:
+                A(f"  {'const float mx0' if o == 6 else f'const float mx{o // 8}'} = {mx};")
+                mx = f"mx{o // 8}"
+        A(f"  const int gex = max(__float_as_int({mx}) >> 23, 40);")
+        A(f"  const float gsc = __int_as_float(({127 + 127 + b_exp} - gex) << 23);")
+        A(f"  const float gun = __int_as_float((gex - {b_exp}) << 23);   // 1 / gsc")
+        for w, l2, ks in paths:
+            if l2 == 0:
+                for k in ks:
+                    A(f"  const float U{w}_{k} = {gexpr(w, k, 0)} * gsc;   // l2 = 0: u does not depend on the edge")
+        for o in range(nO):
+            A(f"  g{o} *= gsc;")
+        A("  // B operands: lane (channel cl, k-group eg) holds fp16 piece eg & 1 of its channel's constants")
+        A("  const bool pb = eg & 1;")
+        for w, l2, ks in steps:
+            if not l2:
+                continue
+            for k in ks:
+                nm = 2 * l2 + 1
+                nr = 2 if l2 == 1 else 4
+                A(f"  uint{nr}v B{w}_{k};")
+                for j in range(nr):
+                    ms = [l2 * l2 + 2 * j + q for q in (0, 1)]
+                    ex = [gexpr(w, k, m) if m < l2 * l2 + nm else "0.f" for m in ms]
+                    if ex == ["0.f", "0.f"]:
+                        A(f"  B{w}_{k}[{j}] = 0;")
+                    else:
+                        A(f"  {{ unsigned h0, h1; mm_split2_f16({ex[0]}, {ex[1]}, h0, h1); B{w}_{k}[{j}] = pb ? h1 : h0; }}")
+
+        def rec_load(eb):
+            """Records of this lane's four edges of the tile at eb (clamped to the receiver's last edge)."""
+            for v in range(4):
+                A(f"    pkn{v} = e_pk[min({eb} + 4 * eg + {v}, e1 - 1)];")
+            A(f"    un = e_u[min({eb} + cl, e1 - 1)];")
+
+        def rec_rows():
+            for v in range(4):
+                A(f"    on{v} = (unsigned)__float_as_int(pkn{v}.y) * {nW * 256}u + cl * 16u;")
+
+        def qload(j, suffix, decl):
+            for v in range(4):
+                A(f"    {'floatx4 ' if decl else ''}q{j}_{v} = *(const floatx4*)(tcb + o{suffix}{v} + {steps[j][0] * 256});")
+
+        if pool:
+            A(f"  if ((int)threadIdx.x < ns) ssend[threadIdx.x] = g_send[(size_t)grp * {SLOTS} + threadIdx.x];")
+            A(f"  for (int j = threadIdx.x; j < ns * {4 * nX}; j += {64 * GROUP}) gxs4[j] = floatx4{{0.f, 0.f, 0.f, 0.f}};")
+            A("  __syncthreads();")
+        A("  if (e0 < e1) {")
+        A("  floatx4 pkn0, pkn1, pkn2, pkn3, un;   // records and edge vector of the next tile")
+        A("  unsigned on0, on1, on2, on3;           // its table rows")
+        rec_load("e0")
+        rec_rows()
+        for j in range(depth):
+            qload(j, "n", True)
+        A("  for (int eb = e0; eb < e1; eb += 16) {")
+        for v in range(4):
+            A(f"    const float t{v} = pkn{v}.x;")
+            A(f"    const unsigned o{v} = on{v};")
+            A(f"    const float* __restrict__ xp{v} = X + (size_t)__float_as_int(pkn{v}.z) * x_stride + c;")
+            for k in range(nX):
+                A(f"    const float X{k}_{v} = xp{v}[{k * C}];")
+        A("    const floatx4 ua = un;")
+        A("    // the next tile's records and edge vector are loaded one tile ahead (the last tile reloads its own end)")
+        rec_load("eb + 16")
+        if pool:
+            A("    const unsigned sl4 = mm_load_u32(e_slot + eb + 4 * eg);   // slots of four edges (the array is padded)")
+        A("    // A operands of edge eb + cl: lane group 0 the harmonics, 1 and 2 their two derivatives")
+        A("    {")
+        A("      float P[16], s, cp, sp;")
+        A("      mm_polar(ua.x, ua.y, s, cp, sp);")
+        A("      mm_polar_operands(ua.z, s, cp, sp, eg, P);")
+        A("      mm_wave_lds_sync();   // the previous tile's operands have been read")
+        A("      if (eg < 3) {")
+        for d, l2 in enumerate(degrees):
+            nm = 2 * l2 + 1
+            A(f"        {{ uint4v a = {{}}, b = {{}};")
+            for j in range((nm + 1) // 2):
+                v = [f"P[{l2 * l2 + 2 * j + q}]" if 2 * j + q < nm else "0.f" for q in (0, 1)]
+                A(f"          {{ unsigned h0, h1; mm_split2_f16({v[0]}, {v[1]}, h0, h1); a[{j}] = h0; b[{j}] = h1; }}")
+            A(f"          uint4v* __restrict__ d = ya + ((eg * {len(degrees)} + {d}) * 16 + cl) * 2;")
+            A("          d[0] = a; d[1] = b; }")
+        A("      }")
+        A("      mm_wave_lds_sync();")
+        A("    }")
+        for v in range(4):
+            A(f"    float gr{v} = 0.f, gt{v} = 0.f, gp{v} = 0.f;")
+            for k in range(nX):
+                A(f"    float gx{k}_{v} = 0.f;")
+
+        def path(j, ks, src):
+            """Contributions of a path; src(k, v) -> (u, dtheta, dphi) expressions for edge v (None: zero)."""
+            for v in range(4):
+                A("    {")
+                A(f"      const floatx4 q = q{j}_{v};")
+                A(f"      const float a = fmaf(q.w, t{v}, q.z);")
+                A(f"      const float b = fmaf(a, t{v}, q.y);")
+                A(f"      const float W = fmaf(b, t{v}, q.x);")
+                A(f"      const float D = fmaf(fmaf(q.w, t{v}, a), t{v}, b);")
+                for k in ks:
+                    A(f"      gx{k}_{v} = fmaf(W, {src(k, v)[0]}, gx{k}_{v});")
+                for ty, (g, f) in enumerate((("gr", "D"), ("gt", "W"), ("gp", "W"))):
+                    if src(ks[0], v)[ty] is None:
+                        continue
+                    e = None
+                    for k in ks:
+                        u = src(k, v)[ty]
+                        e = f"X{k}_{v} * {u}" if e is None else f"fmaf(X{k}_{v}, {u}, {e})"
+                    A(f"      {g}{v} = fmaf({e}, {f}, {g}{v});")
+                A("    }")
+        last = None
+        for j, (w, l2, ks) in enumerate(steps):
+            if l2:
+                ht = "half4v" if l2 == 1 else "half8v"
+                mf = "__builtin_amdgcn_mfma_f32_16x16x16f16" if l2 == 1 else "__builtin_amdgcn_mfma_f32_16x16x32_f16"
+                if l2 != last:
+                    d = degrees.index(l2)
+                    for ty in range(3):
+                        row = f"ya[(({ty * len(degrees) + d}) * 16 + cl) * 2 + (eg >> 1)]"
+                        if l2 == 1:
+                            A(f"    const half4v A{l2}_{ty} = __builtin_bit_cast(half4v, *(const uint2v*)&{row});")
+                        else:
+                            A(f"    const half8v A{l2}_{ty} = __builtin_bit_cast(half8v, {row});")
+                    last = l2
+                for k in ks:
+                    for ty in range(3):
+                        A(f"    const floatx4 D{ty}_{w}_{k} = {mf}(A{l2}_{ty}, __builtin_bit_cast({ht}, B{w}_{k}), floatx4{{0.f, 0.f, 0.f, 0.f}}, 0, 0, 0);")
+                path(j, ks, lambda k, v: tuple(f"D{ty}_{w}_{k}[{v}]" for ty in range(3)))
+            else:
+                path(j, ks, lambda k, v: (f"U{w}_{k}", None, None))
+            # keep the accumulation here (the compiler would sink the sums below the loop body's branches and hold
+            # every path's W and u until then)
+            ops = ", ".join(f'"+v"(gx{k}_{v})' for k in ks for v in range(4))
+            A(f"    asm volatile(\"\" : {ops});")
+            if j + depth == n:
+                rec_rows()
+            if j + depth < n:
+                qload(j + depth, "", True)
+            else:
+                qload(j + depth - n, "n", False)
+        A("    const int n_own = min(e1 - (eb + 4 * eg), 4);   // this lane's edges inside the receiver's range (may be <= 0)")
+        A("    // sums over the 16 channels of the row: transpose-reduction, lane cl = 3 v + j ends with value j of edge v")
+        vals = [f"{nm}{v}" for v in range(4) for nm in ("gr", "gt", "gp")]
+        for x in vals:
+            A(f"    {x} *= gun;")
+        A("    const bool b3 = cl & 8, b2 = cl & 4, b1 = cl & 2, b0 = cl & 1;")
+        for j in range(8):
+            hi = vals[8 + j] if 8 + j < 12 else "0.f"
+            A(f"    const float s8_{j} = (b3 ? {hi} : {vals[j]}) + mm_dpp<0x140>(b3 ? {vals[j]} : {hi});")
+        for j in range(4):
+            A(f"    const float s4_{j} = (b2 ? s8_{4 + j} : s8_{j}) + mm_dpp<0x141>(b2 ? s8_{j} : s8_{4 + j});")
+        for j in range(2):
+            A(f"    const float s2_{j} = (b1 ? s4_{2 + j} : s4_{j}) + mm_dpp<0x1B>(b1 ? s4_{j} : s4_{2 + j});")
+        A("    float sum = (b0 ? s2_1 : s2_0) + mm_dpp<0xB1>(b0 ? s2_0 : s2_1);")
+        A("    const float tc = cl < 3 ? t0 : cl < 6 ? t1 : cl < 9 ? t2 : t3;")
+        A("    if (cl == 0 || cl == 3 || cl == 6 || cl == 9) sum *= mm_spline_dxdr(tc, inv_h);   // zero below the table start")
+        A("    if (cl < 12 && cl < 3 * n_own)")
+        A("      part[(size_t)cb * part_stride + (size_t)(eb + 4 * eg) * 3 + cl] = sum;")
+        if pool:
+            for v in range(4):
+                A(f"    const unsigned sl{v} = (sl4 >> {8 * v}) & 255u;")
+            A("    // the group's LDS accumulators of the senders by 32-bit compare-and-swap, all issued together and repeated only")
+            A("    // where another wave came between; edges without a slot add to gX directly")
+            A("    if (__all(n_own == 4 && !(sl0 == 255 || sl1 == 255 || sl2 == 255 || sl3 == 255))) {")
+            vk = [(v, k) for v in range(4) for k in range(nX)]
+            for v in range(4):
+                A(f"      unsigned* __restrict__ l{v} = (unsigned*)gxs + sl{v} * {16 * nX} + cl;")
+            for v, k in vk:
+                A(f"      unsigned a{k}_{v} = l{v}[{16 * k}];")
+            for v, k in vk:
+                A(f"      unsigned r{k}_{v} = atomicCAS(l{v} + {16 * k}, a{k}_{v}, "
+                  f"__float_as_uint(fmaf(gx{k}_{v}, gun, __uint_as_float(a{k}_{v}))));")
+            A("      if (" + " | ".join(f"(r{k}_{v} != a{k}_{v})" for v, k in vk) + ") {")
+            for v, k in vk:
+                A(f"        while (r{k}_{v} != a{k}_{v}) {{ a{k}_{v} = r{k}_{v}; r{k}_{v} = atomicCAS(l{v} + {16 * k}, "
+                  f"a{k}_{v}, __float_as_uint(fmaf(gx{k}_{v}, gun, __uint_as_float(a{k}_{v})))); }}")
+            A("      }")
+            A("    } else {")
+            for v in range(4):
+                A(f"      if ({v} < n_own) {{")
+                A(f"        if (sl{v} != 255) {{")
+                A(f"          mm_lds_add4_f32(gxs + sl{v} * {16 * nX} + cl, gx0_{v} * gun, gx1_{v} * gun, gx2_{v} * gun, gx3_{v} * gun);")
+                A("        } else {")
+                A(f"          float* __restrict__ gxp = gX + (size_t)__float_as_int(e_pk[eb + 4 * eg + {v}].z) * {nX * C} + cb * {16 * nX} + cl;")
+                for k in range(nX):
+                    A(f"          atomicAdd(gxp + {16 * k}, gx{k}_{v} * gun);")
+                A("        }")
+                A("      }")
+            A("    }")
+        else:
+            for v in range(4):
+                A(f"    if ({v} < n_own) {{")
+                A(f"      float* __restrict__ gxp = gX + (size_t)(eb + 4 * eg + {v}) * {nX * C} + cb * {16 * nX} + cl;")
+                for k in range(nX):
+                    A(f"      gxp[{16 * k}] = gx{k}_{v} * gun;")
+                A("    }")
+        A("  }")
+        A("  }   // edges")
+        if pool:
+            A("  __syncthreads();")
+            A(f"  for (int j = threadIdx.x; j < ns * 64; j += {64 * GROUP}) {{")
+            A("    const int sl = j >> 6, r = j & 63;   // a slot: 256 contiguous bytes [component][channel] of its sender's row")
+            A(f"    atomicAdd(gX + (size_t)ssend[sl] * {nX * C} + cb * {16 * nX} + r, gxs[j]);")
+            A("  }")
+        A("}")
+        A("")
+        A(f"extern \"C\" int {name[:-7]}(const int* rowptr, int nC, const float* e_pk, const float* e_u,")
+        A("    const float* X, int x_stride, const float* tab, int n_tab, int M, float inv_h, const float* gA,")
+        A("    float* part, long part_stride, float* gX," + (" const unsigned char* e_slot, const int* g_send, const int* g_n,"
+                                                           if pool else "") + " hipStream_t stream) {")
+        A("  MM_CHECK_ARG(nC >= 0 && M >= 2 && n_tab >= 1, \"bad sizes\");")
+        if pool:
+            A("  MM_CHECK_ARG(e_slot && g_send && g_n, \"the groups' sender slots (mm_sender_slots) are required\");")
+        A("  MM_CHECK_ARG(gX != nullptr, \"the sender-feature gradient buffer is required\");")
+        A(f"  MM_CHECK_ARG((long)n_tab * (M - 1) * {nW * 256} < (1L << 32), \"a channel block's tables exceed 4 GiB\");")
+        A("  if (nC == 0) return MM_OK;")
+        A(f"  hipLaunchKernelGGL({name}, dim3(8 * ((nC + 3) / 4)), dim3(256), 0, stream, rowptr, nC,")
+        A(f"                     (const floatx4*)e_pk, (const floatx4*)e_u, X, x_stride, (const floatx4*)tab,")
+        A(f"                     n_tab * (M - 1) * {nW * 16}, inv_h, gA, part, part_stride, gX" +
+          (", e_slot, g_send, g_n);" if pool else ");"))
+        A(f"  return mm::launch_status(\"{name[:-7]}\");")
+        A("}")
+        A("")
+    kernel("mm_conv2_bwd_vec_kernel", "pool")
+    kernel("mm_conv2_bwd_vec_det_kernel", "edge")
     return "\n".join(L) + "\n"
 
 
@@ -1525,6 +2002,7 @@ def generate(out_dir, tables):
     for n, tab in tpw_tables().items():
         files[f"tpw_{n}.hip"] = tpw_source(tab, n)
     files["conv_l0123.hip"] = conv_wide_source(tpw_tables()["l0123"], "0123")
+    files.update({"polar.h": POLAR_HEADER, "conv_l2v.hip": conv2_bwd_vec_source(tables.tp2)})
     for name, src in files.items():
         path = os.path.join(out_dir, name)
         if not os.path.exists(path) or open(path).read() != src:

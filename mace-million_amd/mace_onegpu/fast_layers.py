@@ -117,7 +117,7 @@ class FastLayers:
     def __init__(self, model, species_cols, spline_grid=512, r_lo=0.5, device="cuda", ace_layer1=True,
                  deterministic=False):
         self.dev = torch.device(device)
-        # deterministic=True: pass B sums the sender-feature gradient per sender in a fixed order (mm_conv2_bwd_det
+        # deterministic=True: pass B sums the sender-feature gradient per sender in a fixed order (mm_conv2_bwd_vec_det
         # + mm_gather_rows_csr) instead of with float atomics, so repeated evaluations are bitwise identical; it
         # costs a [edges, 512] fp32 buffer per chunk workspace and the per-chunk sender sort
         self.deterministic = bool(deterministic)
@@ -191,6 +191,9 @@ class FastLayers:
         self.n_tab = len(self.radial_sets)
         self.pair_map = torch.tensor(pm, dtype=torch.int32, device=dev)
         self.tab = [self._build_table(P, k) for k in range(2)]
+        # the layer-2 backward on the matrix cores addresses one channel block's tables with 32 bits; larger tables
+        # (more than 1.6 M knots in all) take the per-harmonic kernels
+        self.bwd_vec = self.n_tab * (self.M - 1) * self.tables.tp2["nW"] * 256 < 2 ** 32
         # -------- layer 1 in the exact density-projection (ACE) form: per-edge ht x Y outer products on MFMA,
         # one GEMM per atom with the folded weights G[l, s_recv] (up to 4 species).  It factors W = ht(r) A3 with
         # one ht for all pairs, so per-pair networks take the spline-convolution path
@@ -350,10 +353,17 @@ class FastLayers:
         f = dict(dtype=torch.float32, device=dev)
         i = dict(dtype=torch.int32, device=dev)
         ws = dict(nC=nC, nN=n_nodes, E=E)
+        # backward partials: 3 numbers per edge and channel block (layer 2), 17 per edge (layer 1; 17 per block in the
+        # per-harmonic forms)
+        n_part = max(NCB * 3, 17 if self.ace and self.bwd_vec else NCB * 17)
         ws.update(e_u=torch.empty(E, 4, **f), e_pk=torch.empty(E, 4, **f),
-                  e_recv=torch.empty(E, **i), e_dd=torch.empty(E, **f), part=torch.empty(NCB * E * 17, **f))
+                  e_recv=torch.empty(E, **i), e_dd=torch.empty(E, **f), part=torch.empty(n_part * E, **f))
+        if not self.deterministic:      # the layer-2 backward's sender slots (mm_sender_slots)
+            ng = (nC + codegen.GROUP - 1) // codegen.GROUP
+            ws.update(e_slot=torch.empty(E + 64, dtype=torch.uint8, device=dev),
+                      g_send=torch.empty(ng * codegen.SLOTS, **i), g_n=torch.empty(ng, **i))
         if self.deterministic:
-            ws["gXe"] = torch.empty(E, 4 * C, **f)       # per-edge dL/dX rows of mm_conv2_bwd_det
+            ws["gXe"] = torch.empty(E, 4 * C, **f)       # per-edge dL/dX rows of mm_conv2_bwd_vec_det
         # A (a layer's message, read by the linear after its convolution) and gA (its cotangent, written by the
         # transposed linear and read by the backward convolution) are never live together in a pass: one buffer
         A = torch.empty(nC * self.nO2 * C, **f)
@@ -370,7 +380,7 @@ class FastLayers:
     def _lin(self, plan, inp, in_stride, out, out_stride, W, rows, in_rows=None, out_rows=None, scale=None,
              scale_mode=0, species=False, accumulate=0, w_group_stride=0, count_dev=None, in_cb=0):
         """count_dev (optional device int32 [1]): the row count read by the kernel, rows only sizing the launch.
-        in_cb: input rows in 16-channel-block-major order with in_cb components (mm_conv2_bwd's dL/dX)."""
+        in_cb: input rows in 16-channel-block-major order with in_cb components (mm_conv2_bwd_vec's dL/dX)."""
         ws = self.ws
         units = (rows, plan.k_sum, plan.n_in, plan.n, accumulate, plan.n_w * (self.S if species else 1))
         if species:
@@ -520,23 +530,30 @@ class FastLayers:
                     ws["gM"], 16 * C, ws["rho"], ws["g_rho"], stream())
         self._lin(self.plan_lin2T, ws["gM"], 16 * C, ws["gA"], self.nO2 * C, self.W_lin2T, g.nC, scale=ws["rho"],
                   scale_mode=1)
+        det = "_det" if self.deterministic else ""
+        n = 3 if self.bwd_vec else 17                   # numbers per partial row
+        gX, slots = ws["gXh"], ()
+        if self.deterministic:
+            gX = ws["gXe"]
+        else:
+            K.mm_fill_f32(gX, g.n_nodes * D1, 0.0, stream())
+            if self.bwd_vec:
+                slots = (ws["e_slot"], ws["g_send"], ws["g_n"])
+                K.mm_sender_slots(g.rowptr, g.nC, g.ls, *slots, stream())
+        bwd = getattr(K, ("mm_conv2_bwd_vec" if self.bwd_vec else "mm_conv2_bwd") + det)
+        self._timed("conv2_bwd", (g.nE, g.nC, g.n_nodes), bwd, g.rowptr, g.nC, ws["e_pk"], ws["e_u"], ws["Xh"], D1,
+                    self.tab[1], self.n_tab, self.M, self.inv_h, ws["gA"], ws["part"], ws["E"] * n, gX, *slots,
+                    stream())
         if self.deterministic:
             srp, sperm = sender_csr(g)
-            self._timed("conv2_bwd", (g.nE, g.nC, g.n_nodes), K.mm_conv2_bwd_det, g.rowptr, g.nC, ws["e_pk"],
-                        ws["e_u"], ws["Xh"], D1, self.tab[1], self.n_tab, self.M, self.inv_h, ws["gA"], ws["part"],
-                        ws["E"] * 17, ws["gXe"], stream())
-            K.mm_gather_rows_csr(srp, sperm, ws["gXe"], D1, D1, ws["gXh"], D1, g.n_nodes, stream())
-        else:
-            K.mm_fill_f32(ws["gXh"], g.n_nodes * D1, 0.0, stream())
-            self._timed("conv2_bwd", (g.nE, g.nC, g.n_nodes), K.mm_conv2_bwd, g.rowptr, g.nC, ws["e_pk"], ws["e_u"],
-                        ws["Xh"], D1, self.tab[1], self.n_tab, self.M, self.inv_h, ws["gA"], ws["part"],
-                        ws["E"] * 17, ws["gXh"], stream())
+            K.mm_gather_rows_csr(srp, sperm, gX, D1, D1, ws["gXh"], D1, g.n_nodes, stream())
         pf = self._chunk_pair_forces(g, PF, forces)
-        K.mm_edge_grad(g.nE, g.E_dev, ws["part"], ws["E"] * 17, NCB, ws["g_rho"], ws["e_recv"], ws["e_dd"], ws["e_u"],
-                       pf, 0, stream())
+        grad = K.mm_edge_grad_vec if self.bwd_vec else K.mm_edge_grad
+        grad(g.nE, g.E_dev, ws["part"], ws["E"] * n, NCB, ws["g_rho"], ws["e_recv"], ws["e_dd"], ws["e_u"], pf, 0,
+             stream())
         if forces is not None:
             self._add_chunk_forces(g, pf, forces)
-        # gXh holds dL/dX in 16-channel-block-major rows (as mm_conv2_bwd / mm_conv2_bwd_det write it)
+        # gXh holds dL/dX in 16-channel-block-major rows (as mm_conv2_bwd_vec / _vec_det write it)
         self._lin(self.plan_p1, ws["gXh"], D1, G1, D1, self.W_up2T, g.n_nodes, out_rows=g.nodes, accumulate=1,
                   count_dev=g.N_dev, in_cb=4)
         self._lin(self.plan_sk1, gh2, C, G1, D1, self.W_sk1T, g.nC, out_rows=g.nodes, species=True, w_group_stride=1,
