@@ -15,30 +15,46 @@
 // Six 16x16x32 bf16 products take 96 cycles against 256 for the same K = 32 in v_mfma_f32_16x16x4f32.  The
 // weights are split once on the host; the input rows are split as they are loaded.
 //
-// Launch: grid (n_comp, ceil(rows / (256 n_blk)), n_groups), components fastest: the workgroups of one row block
-// are dispatched together, so an output row is written and an input row is read by neighbouring workgroups
-// (measured: 4-15 % less linear time than row blocks fastest).  1024 threads = 16 waves, each wave 16 rows x 128
-// columns (8 MFMA tiles) of each of its n_blk row blocks; the weight block (3 bf16 planes of 128 x 128, 96 KiB)
-// is staged in LDS in the lane order of the B operand.  16 waves of one workgroup per CU = 4 waves per SIMD.
+// Weights in registers.  A workgroup is 4 waves; each holds 32 of the 128 columns of a weight block (96 registers: 3
+// planes x 4 K-steps x 2 tiles) and streams rows past them, 32 rows (a stage) at a time.  The rows of a stage are
+// loaded coalesced by the whole workgroup, split once and written to LDS in operand order, one stage ahead of the
+// products; a stage is 96 matrix instructions per wave on four independent sums.  The weights are the first operand,
+// so that a lane ends with 4 consecutive columns of one row: 16-byte stores.
+// Bound: the bf16 products and the rows' traffic, which are near each other (40 x 40 components, 131,072 rows: 0.85 ms of
+// products at the 1.21 PFLOP/s of a large matrix product, 0.80 ms of traffic at the 4.67 TB/s of a large copy).  Before,
+// a workgroup staged the whole weight block (96 KiB) in LDS for 256 rows, and 16 waves read it again for every 16 rows:
+// LDS reads cost as much as the products, and nothing of a workgroup's start and end overlapped.  Measured (us, before
+// -> now; 16 components of 1 source, 16 of 2-3 sources, 40 of 1 source):
+//      192 rows:  12.5 -> < 9     27 -> < 10    12.6 -> < 9     (launch calls take 9 us)
+//    4,001 rows:   22 -> 20       40 -> 36       56 -> 39
+//   16,384 rows:   83 -> 56      174 -> 146     163 -> 149
+//  131,072 rows:  474 -> 452    1180 -> 1118   1167 -> 1134
+// Several sources: NS stages share each load of a source's weights, with NS stages of sums held.  4 stages from two
+// rounds of workgroups on (16 x 2 components, 131,072 rows: 849 us, 1115 us with 1 stage, 920 us with 2, 897 us with 3);
+// below that 1 stage, for more workgroups (1,024 rows: 11 us, 19 us with 4).
 // Weight blocks: plane p of block b at bf16 offset (3 b + p) 16384; element W[k][n], k = 32 t + 8 g + u,
 // n = 16 nt + i, at (((t * 8 + nt) * 4 + g) * 16 + i) * 8 + u, so that lane (i, g) reads its 8 k-values of step t
-// and tile nt as one 16-byte LDS read, the 16 lanes of a group reading 256 consecutive bytes (no bank conflicts);
-// the A operand of lane (row, g) is in[row][32 t + 8 g .. + 7], loaded coalesced and passed through 2.5 KiB of
-// LDS rows per wave (mm_lin_load_a, mm_lin_stage_a); a row past the last one reads logical row 0 and is not stored.
+// and tile nt as one 16-byte load, a wave 1 KiB.  The rows in LDS: 16-byte unit (row tile, plane, k / 8, row), the k / 8
+// groups 17 units apart: the 8-byte writes (32 lanes: one row) and the 16-byte reads (16 lanes: 16 rows) use every bank
+// once.
+// Components fastest in the grid: the workgroups of one row block run together, so an output row is written and an
+// input row read by neighbouring workgroups.
 #include "common.h"
 
-#include <algorithm>
+#include <climits>
 
 #define MM_LIN_MAX_COMP 48
 #define MM_LIN_MAX_SRC 3
-#define MM_LIN_NW 16
-#define MM_LIN_BLOCK_ROWS (16 * MM_LIN_NW)
-#define MM_LIN_AS 40   // LDS row stride (floats) of a wave's A staging rows
-// a launch keeps at least this many workgroups (4 per CU) when it groups row blocks per workgroup
-#define MM_LIN_MIN_WG 1024
+#define MM_LIN_NW 4          // waves per workgroup
+#define MM_LIN_ROWS 32       // rows of a stage
+#define MM_LIN_WG_ROWS 1024  // rows per workgroup at most
+#define MM_LIN_AS 17         // LDS distance (16 B) of the k-groups of a row tile
+#define MM_LIN_WG 512        // resident workgroups of the card (2 per CU)
+#define MM_LIN_START 2       // cost of a workgroup's start, in stages
+#define MM_LIN_NS 4          // stages per load of weights with several sources
 
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx8 __attribute__((ext_vector_type(8)));
 
 struct MMLinComp {
   int n_src;
@@ -48,7 +64,7 @@ struct MMLinComp {
 };
 
 struct MMLinArgs {
-  const float* in;
+  const float* in;        // 16-byte aligned rows
   long in_stride;
   const int* in_rows;     // nullable: in row of logical row id
   float* out;
@@ -69,165 +85,175 @@ struct MMLinArgs {
   MMLinComp comp[MM_LIN_MAX_COMP];
 };
 
-struct MMLinRows {
-  bool valid;
-  long in_row;
-};
-
-__device__ __forceinline__ void mm_lin_rows(const MMLinArgs& args, const int* list, int nrows, int row0, int wave,
-                                            int i, MMLinRows& rw) {
-  const int r = row0 + wave * 16 + i;
-  rw.valid = r < nrows;
-  const int rid = rw.valid ? (list ? list[r] : r) : 0;
-  rw.in_row = args.in_rows ? (long)args.in_rows[rid] : (long)rid;
-}
-
-// Input rows of one source, loaded coalesced: lane L reads rows L >> 3 and 8 + (L >> 3) of the wave's 16, floats
-// 32 t + 4 (L & 7) .. + 3 of the source chunk, into a[2 t] and a[2 t + 1] (t = 0..3): 8 lanes read 128 contiguous
-// bytes of a row.  (In the MFMA operand layout the 16 lanes of a row group would read 16 different rows, which the
-// texture path serves one lane per clock.)  mm_lin_stage_a passes step t through the wave's LDS rows into the
-// operand layout.
-// With channel-block-major input rows (in_cb = n components per block), chunk float q = 32 t + 4 (L & 7) of
-// component k lies at (q >> 4) 16 n + 16 k + (q & 15): every lane's 4 floats stay contiguous.
-__device__ __forceinline__ void mm_lin_load_a(const MMLinArgs& args, const MMLinRows& rw, int in_off, int lane,
-                                              floatx4 (&a)[8]) {
-  const long r0 = __shfl(rw.in_row, lane >> 3), r1 = __shfl(rw.in_row, 8 + (lane >> 3));
-  const int qb = 4 * (lane & 7);
-  const int n = args.in_cb;
-  const int base = n ? (qb >> 4) * 16 * n + 16 * (in_off >> 7) + (qb & 15) : in_off + qb;
-  const int tstep = n ? 32 * n : 32;
-  const float* __restrict__ p0 = args.in + r0 * args.in_stride + base;
-  const float* __restrict__ p1 = args.in + r1 * args.in_stride + base;
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    a[2 * t] = *(const floatx4*)(p0 + tstep * t);
-    a[2 * t + 1] = *(const floatx4*)(p1 + tstep * t);
-  }
-}
-
-// A operand of step t: lane (i, g) gets in[row i][32 t + 8 g .. + 7], through the wave's LDS rows (row stride
-// MM_LIN_AS floats: the 16-byte reads of the 16 rows fall in different banks)
-__device__ __forceinline__ floatx8 mm_lin_stage_a(const floatx4 (&a)[8], int t, int lane, int i, int g,
-                                                  float* __restrict__ as) {
-  mm_wave_lds_sync();   // the previous step's reads are done
-  *(floatx4*)(as + (lane >> 3) * MM_LIN_AS + 4 * (lane & 7)) = a[2 * t];
-  *(floatx4*)(as + (8 + (lane >> 3)) * MM_LIN_AS + 4 * (lane & 7)) = a[2 * t + 1];
-  mm_wave_lds_sync();
-  const floatx4 xa = *(const floatx4*)(as + i * MM_LIN_AS + 8 * g);
-  const floatx4 xb = *(const floatx4*)(as + i * MM_LIN_AS + 8 * g + 4);
-  return floatx8{xa.x, xa.y, xa.z, xa.w, xb.x, xb.y, xb.z, xb.w};
-}
+// 16 B stores to rows that are only known to be float-aligned
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
 
 // x = x0 + x1 + x2 (bf16, round to nearest even; both differences are exact in fp32)
-__device__ __forceinline__ void mm_split3_bf16(const floatx8& x, bf16x8& x0, bf16x8& x1, bf16x8& x2) {
-  x0 = __builtin_convertvector(x, bf16x8);
-  const floatx8 r1 = x - __builtin_convertvector(x0, floatx8);
-  x1 = __builtin_convertvector(r1, bf16x8);
-  const floatx8 r2 = r1 - __builtin_convertvector(x1, floatx8);
-  x2 = __builtin_convertvector(r2, bf16x8);
+__device__ __forceinline__ void mm_split3_bf16(const floatx4& x, bf16x4& x0, bf16x4& x1, bf16x4& x2) {
+  x0 = __builtin_convertvector(x, bf16x4);
+  const floatx4 r1 = x - __builtin_convertvector(x0, floatx4);
+  x1 = __builtin_convertvector(r1, bf16x4);
+  const floatx4 r2 = r1 - __builtin_convertvector(x1, floatx4);
+  x2 = __builtin_convertvector(r2, bf16x4);
 }
 
-// A workgroup handles n_blk consecutive row blocks of one output component.  A weight block is staged in LDS only
-// when it is not the one already there: once for all row blocks with a single source, n_src - 1 times per row block
-// after the first with several (their order alternates between row blocks).
-__global__ void __launch_bounds__(64 * MM_LIN_NW) mm_linear_kernel(MMLinArgs args, int n_blk) {
-  __shared__ uint4 Wl[3 * 2048];
-  __shared__ float As_all[MM_LIN_NW * 16 * MM_LIN_AS];   // per wave: 16 rows of one K-step
+// NS: stages (32 rows) per weight load when a component has several sources.  n_st: stages per workgroup.
+template <int NS>
+__global__ void __launch_bounds__(64 * MM_LIN_NW, 2) mm_linear_kernel(MMLinArgs args, int n_st) {
+  __shared__ uint4 Al[2][2 * 3 * 16 * MM_LIN_AS];   // [buffer][row tile][plane][k / 8][row], k-groups MM_LIN_AS apart
+  __shared__ int s_in[MM_LIN_WG_ROWS], s_out[MM_LIN_WG_ROWS];
+  __shared__ float s_sc[MM_LIN_WG_ROWS];
   const MMLinComp& cp = args.comp[blockIdx.x];   // kernel-argument memory, read with uniform indices
   const int grp = blockIdx.z;
   const int nrows = args.list_count ? min(args.list_count[grp], args.n_rows) : args.n_rows;
-  const int blk0 = blockIdx.y * n_blk;
-  if (blk0 * MM_LIN_BLOCK_ROWS >= nrows) return;
-  const int blk1 = min(blk0 + n_blk, (nrows + MM_LIN_BLOCK_ROWS - 1) / MM_LIN_BLOCK_ROWS);
-  const int* __restrict__ list = args.list ? args.list + (size_t)grp * args.list_stride : nullptr;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
-  float* __restrict__ as = As_all + wave * 16 * MM_LIN_AS;
+  const int row0 = blockIdx.y * n_st * MM_LIN_ROWS;
+  if (row0 >= nrows) return;
+  const int n = min(n_st * MM_LIN_ROWS, nrows - row0);   // rows of this workgroup
+  const int nst = (n + MM_LIN_ROWS - 1) / MM_LIN_ROWS;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, i = lane & 15, g = lane >> 4;
   const int n_src = cp.n_src;
-  int staged = -1;   // weight block held in LDS (wave-uniform)
-  MMLinRows rw;
-  mm_lin_rows(args, list, nrows, blk0 * MM_LIN_BLOCK_ROWS, wave, i, rw);
-  for (int blk = blk0; blk < blk1; ++blk) {
-    const int row0 = blk * MM_LIN_BLOCK_ROWS;
-    floatx4 acc[8];
+
+  // this thread's part of a stage: floats 4 k4 .. + 3 of rows tid >> 5, + 8, + 16, + 24
+  const int k4 = tid & 31, rw = tid >> 5;
+  const int cb = args.in_cb;
+  const int koff = cb ? (k4 >> 2) * 16 * cb + 4 * (k4 & 3) : 4 * k4;
+  floatx4 x[4];
+  auto load = [&](int st, int q) {
+    const float* __restrict__ p = args.in + (cb ? cp.in_off[q] >> 3 : cp.in_off[q]) + koff;   // 16 floats of 128
 #pragma unroll
-    for (int nt = 0; nt < 8; ++nt) acc[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    // odd row blocks take the sources in reverse order, so that the block in LDS at the end of one row block is
-    // the first one the next needs (n_src - 1 stagings per row block instead of n_src; the order depends only on
-    // the row block, so every launch partition sums a row in the same order)
-    for (int qq = 0; qq < n_src; ++qq) {
-      const int q = (blk & 1) ? n_src - 1 - qq : qq;
-      floatx4 a[8];
-      mm_lin_load_a(args, rw, cp.in_off[q], lane, a);
-      const int widx = cp.w_idx[q] + grp * args.w_group_stride;
-      if (widx != staged) {
-        const uint4* __restrict__ Wg = args.W + (size_t)widx * 6144;
-        __syncthreads();
-        for (int j = threadIdx.x; j < 6144; j += 64 * MM_LIN_NW) Wl[j] = Wg[j];
-        __syncthreads();
-        staged = widx;
+    for (int j = 0; j < 4; ++j) x[j] = *(const floatx4*)(p + s_in[st * MM_LIN_ROWS + 8 * j + rw] * args.in_stride);
+  };
+  auto put = [&](int buf) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      bf16x4 h[3];
+      mm_split3_bf16(x[j], h[0], h[1], h[2]);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        uint2* d = (uint2*)&Al[buf][(((j >> 1) * 3 + p) * 16 + (k4 >> 1)) * MM_LIN_AS + 8 * (j & 1) + rw];
+        d[k4 & 1] = __builtin_bit_cast(uint2, h[p]);
       }
+    }
+  };
+
+  bf16x8 B[4][2][3];
+  auto load_w = [&](int q) {
+    const uint4* __restrict__ Wg = args.W + (size_t)(cp.w_idx[q] + grp * args.w_group_stride) * 6144
+                                  + (2 * wave * 4 + g) * 16 + i;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const floatx8 x = mm_lin_stage_a(a, t, lane, i, g, as);
-        bf16x8 a0, a1, a2;
-        mm_split3_bf16(x, a0, a1, a2);
+    for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int nt = 0; nt < 8; ++nt) {
-          const int o = ((t * 8 + nt) * 4 + g) * 16 + i;
-          const bf16x8 b0 = __builtin_bit_cast(bf16x8, Wl[o]);
-          const bf16x8 b1 = __builtin_bit_cast(bf16x8, Wl[2048 + o]);
-          const bf16x8 b2 = __builtin_bit_cast(bf16x8, Wl[4096 + o]);
-          // smallest terms first
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2, b0, acc[nt], 0, 0, 0);
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b2, acc[nt], 0, 0, 0);
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1, acc[nt], 0, 0, 0);
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b0, acc[nt], 0, 0, 0);
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b1, acc[nt], 0, 0, 0);
-          acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0, acc[nt], 0, 0, 0);
+      for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int p = 0; p < 3; ++p) B[t][c][p] = __builtin_bit_cast(bf16x8, Wg[p * 2048 + t * 512 + c * 64]);
+  };
+
+  // row indices and scales of the workgroup's rows (rows past the last one repeat it and are not stored); the first
+  // weights are loaded behind the indices
+  for (int r0 = 0; r0 < nst * MM_LIN_ROWS; r0 += 64 * MM_LIN_NW) {
+    const int rr = row0 + min(r0 + tid, n - 1);
+    const int id = args.list ? args.list[(size_t)grp * args.list_stride + rr] : rr;
+    int ir = id, orow = id;
+    float sc = 0.f;
+    if (args.in_rows) ir = args.in_rows[id];
+    if (args.out_rows) orow = args.out_rows[id];
+    if (args.row_scale) sc = args.row_scale[id];
+    if (r0 == 0) load_w(0);
+    s_in[r0 + tid] = ir;
+    s_out[r0 + tid] = orow;
+    s_sc[r0 + tid] = !args.row_scale ? 1.f : args.scale_mode == 1 ? 1.f / (sc + 1.f) : sc;
+  }
+  __syncthreads();
+  load(0, 0);
+  put(0);
+  __syncthreads();
+  int buf = 0;
+  for (int b = 0; b < nst; b += NS) {
+    floatx4 acc[NS][2][2];
+#pragma unroll
+    for (int s = 0; s < NS; ++s)
+#pragma unroll
+      for (int r = 0; r < 2; ++r) acc[s][r][0] = acc[s][r][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int q = 0; q < n_src; ++q) {
+      if (n_src > 1 && b + q > 0) load_w(q);
+#pragma unroll
+      for (int s = 0; s < NS; ++s) {
+        if (b + s >= nst) break;
+        // the next stage of this workgroup: of this source, of the next source, of the next block of stages (after
+        // the last one this stage again: a load without a branch leaves the weights' loads countable)
+        const bool last_s = s == NS - 1 || b + s + 1 == nst, last_q = q + 1 == n_src;
+        const bool more = !(last_s && last_q && b + NS >= nst);
+        load(!more || !last_s ? b + s + (more ? 1 : 0) : last_q ? b + NS : b, !more || !last_s ? q : last_q ? 0 : q + 1);
+        bf16x8 a[2][2][3];
+        auto load_a = [&](int t) {
+#pragma unroll
+          for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+              a[t & 1][r][p] = __builtin_bit_cast(bf16x8, Al[buf][((r * 3 + p) * 16 + 4 * t + g) * MM_LIN_AS + i]);
+        };
+        load_a(0);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          if (t < 3) load_a(t + 1);
+          __builtin_amdgcn_sched_barrier(0);   // the reads of step t + 1 stay ahead of the products of step t
+          // four independent sums; per sum the smallest terms first
+#pragma unroll
+          for (int k = 0; k < 6; ++k) {
+            constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0};
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+              for (int c = 0; c < 2; ++c)
+                acc[s][r][c] =
+                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(B[t][c][pb[k]], a[t & 1][r][pa[k]], acc[s][r][c], 0, 0, 0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (more) {
+          put(buf ^ 1);
+          __syncthreads();
+          buf ^= 1;
         }
       }
     }
-    // D layout of the 16x16 tile: lane (i, g) holds rows 4 g + v (v = 0..3) of column i.  The row indices and
-    // scales of the four rows are loaded before any store, and an accumulating launch reads the eight old values
-    // of a row together (one memory round trip per row, not one per value).  A lane past the last row uses
-    // logical row 0 (there is one) for its loads and stores nothing.
-    bool ok[4];
-    int id[4];
+    // weights as the first operand: lane (i, g) holds columns 4 g .. + 3 of row i of each tile
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int rr = row0 + wave * 16 + 4 * g + v;
-      ok[v] = rr < nrows;
-      id[v] = ok[v] ? (list ? list[rr] : rr) : 0;
-    }
-    float* op[4];
-    float sc[4];
+    for (int s = 0; s < NS; ++s) {
+      floatx4u* op[2];
+      float sc[2];
+      bool ok[2];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const long orow = args.out_rows ? (long)args.out_rows[id[v]] : (long)id[v];
-      op[v] = args.out + orow * args.out_stride + cp.out_off + i;
-      sc[v] = 1.f;
-      if (args.row_scale)
-        sc[v] = args.scale_mode == 1 ? 1.f / (args.row_scale[id[v]] + 1.f) : args.row_scale[id[v]];
-    }
-    if (args.accumulate) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        if (!ok[v]) continue;
-        float old[8];
-#pragma unroll
-        for (int nt = 0; nt < 8; ++nt) old[nt] = op[v][16 * nt];
-#pragma unroll
-        for (int nt = 0; nt < 8; ++nt) op[v][16 * nt] = old[nt] + sc[v] * acc[nt][v];
+      for (int r = 0; r < 2; ++r) {
+        const int rr = (b + s) * MM_LIN_ROWS + 16 * r + i;
+        ok[r] = rr < n;
+        const int rc = ok[r] ? rr : 0;
+        op[r] = (floatx4u*)(args.out + s_out[rc] * args.out_stride + cp.out_off + 32 * wave + 4 * g);
+        sc[r] = s_sc[rc];
       }
-    } else {
+      if (args.accumulate) {
+        floatx4 old[2][2];
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        if (!ok[v]) continue;
+        for (int r = 0; r < 2; ++r)
+          if (ok[r]) {
+            old[r][0] = op[r][0];
+            old[r][1] = op[r][4];
+          }
 #pragma unroll
-        for (int nt = 0; nt < 8; ++nt) op[v][16 * nt] = sc[v] * acc[nt][v];
+        for (int r = 0; r < 2; ++r)
+          if (ok[r]) {
+            op[r][0] = old[r][0] + sc[r] * acc[s][r][0];
+            op[r][4] = old[r][1] + sc[r] * acc[s][r][1];
+          }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+          if (ok[r]) {
+            op[r][0] = sc[r] * acc[s][r][0];
+            op[r][4] = sc[r] * acc[s][r][1];
+          }
       }
     }
-    if (blk + 1 < blk1) mm_lin_rows(args, list, nrows, row0 + MM_LIN_BLOCK_ROWS, wave, i, rw);
   }
 }
 
@@ -277,11 +303,22 @@ extern "C" int mm_linear(const float* in, long in_stride, const int* in_rows, fl
     a.comp[j].out_off = comp_out_off[j];
   }
   if (n_rows_max == 0) return MM_OK;
-  // row blocks per workgroup: as many as keep at least MM_LIN_MIN_WG workgroups in the launch (at most 8)
-  const long n_blocks = (n_rows_max + MM_LIN_BLOCK_ROWS - 1) / MM_LIN_BLOCK_ROWS;
-  const long per_blk = (long)n_comp * n_groups;
-  const int n_blk = (int)std::max(1L, std::min(8L, n_blocks * per_blk / MM_LIN_MIN_WG));
-  dim3 grid(n_comp, (unsigned)((n_blocks + n_blk - 1) / n_blk), n_groups);
-  hipLaunchKernelGGL(mm_linear_kernel, grid, dim3(64 * MM_LIN_NW), 0, stream, a, n_blk);
+  bool multi = false;
+  for (int j = 0; j < n_comp; ++j) multi |= comp_nsrc[j] > 1;
+  // stages per workgroup: the least time in rounds of resident workgroups, a workgroup costing its stages and
+  // MM_LIN_START more (first indices, rows and weights).  40 components, 16,384 rows: 149 us; with the fewest
+  // workgroups (640 of 32 stages) 182-205 us, with at least 1,024 workgroups 174 us
+  const long stages = (n_rows_max + MM_LIN_ROWS - 1) / MM_LIN_ROWS;
+  const int ns = multi && stages * n_comp >= 2L * MM_LIN_WG ? MM_LIN_NS : 1;
+  long n_st = ns, best = LONG_MAX;
+  for (long k = ns; k <= MM_LIN_WG_ROWS / MM_LIN_ROWS; k += ns) {
+    const long wgs = (stages + k - 1) / k * n_comp, cost = (wgs + MM_LIN_WG - 1) / MM_LIN_WG * (k + MM_LIN_START);
+    if (cost < best) best = cost, n_st = k;
+  }
+  const dim3 grid(n_comp, (unsigned)((stages + n_st - 1) / n_st), n_groups);
+  if (ns == MM_LIN_NS)
+    hipLaunchKernelGGL(mm_linear_kernel<MM_LIN_NS>, grid, dim3(64 * MM_LIN_NW), 0, stream, a, (int)n_st);
+  else
+    hipLaunchKernelGGL(mm_linear_kernel<1>, grid, dim3(64 * MM_LIN_NW), 0, stream, a, (int)n_st);
   return mm::launch_status("mm_linear");
 }
