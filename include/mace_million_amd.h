@@ -194,6 +194,12 @@ int mm_spline_coeffs_flat(const double* samples, int M, int D, double eps, doubl
  * recv are int32, or int64 with index64 != 0; strides in elements; send and send32 may both be null. */
 int mm_edge_csr(const void* send, long send_stride, const void* recv, long recv_stride, int index64, int E, int n,
                 int n_send, int* send32, int* rowptr, int* bad, mm_stream_t stream);
+/* ThreePassMLIAP._topology (mliap_threepass.py:288-310) of receivers a..b-1 with the senders send [E] in [0, nt):
+ * nodes = a..b-1, then the senders outside [a, b) in ascending order (room for b - a + min(E, nt - b + a)); ls [E] = row
+ * of each edge's sender in nodes; status [2] (zeroed by the caller) = senders outside [0, nt) (their ls is not
+ * written), senders outside [a, b).  scratch: 2 w + ceil(w / 1024) words, w = nt / 32 + 1, zeroed by the caller. */
+int mm_chunk_topology(const int* send, int E, int a, int b, int nt, unsigned* scratch, int* nodes, int* ls, int* status,
+                      mm_stream_t stream);
 int mm_tpw_l1_fwd(const int* rowptr, int nR, const int* eid, const int* send, const float* Y, long y_stride,
                   const float* W, long w_stride, const float* X, long x_stride, float* out, long out_stride,
                   mm_stream_t stream);

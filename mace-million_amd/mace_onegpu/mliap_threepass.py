@@ -28,6 +28,7 @@ import time
 import torch
 
 from . import chunk_graphs, fast_layers
+from ._lib import K, stream
 from .receiver_chunk_mace import check_chunk, chunk_topology, make_chunk
 
 try:
@@ -85,8 +86,11 @@ def neighbour_slot_guard(nlocal, npairs, rcutfac):
 def output_guard(eat, PF, limit, call):
     """Raises instead of handing LAMMPS non-finite energies or a pair force beyond `limit` eV/A
     (MACE3P_FMAX_ABORT, mliap_threepass.py:595-601)."""
-    fmax = float(PF.abs().max()) if PF.numel() else 0.0
-    if bool(torch.isfinite(eat).all()) and fmax == fmax and fmax < limit:
+    finite = torch.isfinite(eat).all()
+    lo, hi = torch.aminmax(PF) if PF.numel() else (PF.new_zeros(()),) * 2
+    lo, hi, finite = torch.stack([lo, hi, finite.to(PF.dtype)]).tolist()       # one device-to-host read
+    fmax = max(-lo, hi) if lo == lo else lo
+    if finite and fmax == fmax and fmax < limit:
         return
     raise RuntimeError(f"ThreePassMLIAP guard: non-finite or absurd output at call {call} "
                        f"(max |pair force| = {fmax:.3e} eV/A, limit {limit:g}); aborting before LAMMPS "
@@ -114,17 +118,20 @@ class _PairBatch:
 
     LAMMPS may hand the pairs over in any order; the kernels need them grouped by receiver (pair_i).  When they
     are not already non-decreasing they are put in that order by a stable sort, and `restore` applies the inverse
-    permutation to the per-pair results.  rowptr [nlocal + 1] is the receiver CSR (its host copy is the call's
-    one device-to-host read)."""
+    permutation to the per-pair results.  rowptr [nlocal + 1] is the receiver CSR; its host copy comes with the
+    checks in one device-to-host read (two when the pairs arrive unsorted)."""
 
     def __init__(self, data, nlocal, ntotal, dev, check):
         pi = torch.as_tensor(data.pair_i).to(dev).to(torch.int32)
         pj = torch.as_tensor(data.pair_j).to(dev).to(torch.int32)
         rij = torch.as_tensor(data.rij).to(dev).to(torch.float64)
         self.perm = None
-        if pi.numel() > 1 and bool((pi[1:] < pi[:-1]).any()):
+        csr = self._csr(pi, nlocal)
+        if csr is None:
             pi, self.perm = torch.sort(pi, stable=True)
             pj, rij = pj[self.perm], rij[self.perm]
+            csr = self._csr(pi, nlocal)
+        self.rowptr, self.rowptr_host, bad = csr
         self.pair_i, self.pair_j, self.rij = pi.contiguous(), pj.contiguous(), rij.contiguous()
         if check:
             lo_i, hi_i = (int(pi.min()), int(pi.max())) if pi.numel() else (0, 0)
@@ -132,12 +139,23 @@ class _PairBatch:
             if lo_i < 0 or hi_i >= nlocal or lo_j < 0 or hi_j >= ntotal:
                 raise ValueError(f"ThreePassMLIAP: pair_i in [{lo_i}, {hi_i}] must lie in [0, {nlocal}) and "
                                  f"pair_j in [{lo_j}, {hi_j}] in [0, {ntotal})")
-        counts = torch.bincount(pi.long(), minlength=nlocal)
-        if counts.numel() != nlocal:
+        if bad:
             raise ValueError(f"ThreePassMLIAP: a pair receiver is not a local atom (nlocal = {nlocal})")
-        self.rowptr = torch.zeros(nlocal + 1, dtype=torch.int64, device=dev)
-        self.rowptr[1:] = torch.cumsum(counts, 0)
-        self.rowptr_host = self.rowptr.cpu().numpy()
+
+    @staticmethod
+    def _csr(pi, nlocal):
+        """(rowptr on the device, on the host, number of receivers outside [0, nlocal)) of the receivers pi, or None
+        when they are not non-decreasing."""
+        if pi.numel() >= 2 ** 31 or not pi.is_cuda:
+            if pi.numel() > 1 and bool((pi[1:] < pi[:-1]).any()):
+                return None
+            bad = int(((pi < 0) | (pi >= nlocal)).sum())
+            rowptr = torch.searchsorted(pi, torch.arange(nlocal + 1, dtype=torch.int32, device=pi.device))
+            return rowptr, rowptr.cpu().numpy(), bad
+        buf = torch.zeros(nlocal + 4, dtype=torch.int32, device=pi.device)
+        K.mm_edge_csr(None, 0, pi, pi.stride(0), 0, pi.numel(), nlocal, nlocal, None, buf[3:], buf, stream())
+        host = buf.cpu().numpy()
+        return None if host[2] else (buf[3:], host[3:], int(host[1]))
 
     def restore(self, per_pair):
         """Per-pair results back in the order the pairs arrived in."""
@@ -225,6 +243,9 @@ class _Runtime:
         self.fl = fast_layers.FastLayers(model, self.cols, spline_grid=plugin.spline_grid, device=dev,
                                          ace_layer1=k.ace_layer1, deterministic=k.deterministic)
         self.scale, self.shift, self.e0 = self.fl.scale, self.fl.shift, self.fl.e0
+        self.known = torch.zeros(self.cols[-1] + 3, dtype=torch.bool)       # by element + 1, False at both ends
+        self.known[torch.tensor(self.cols) + 1] = True
+        self.known = self.known.to(dev)
         self.D1 = 4 * model.spec.C
         self.chunk = k.chunk or plugin.chunk
         self.e_align = plugin.e_align
@@ -245,7 +266,9 @@ class _Runtime:
         return round(p, 3), round(self.peak, 3)
 
     def covers(self, elems):
-        return set(torch.unique(elems).tolist()) <= set(self.cols)
+        """Whether the constants were built for every element of elems."""
+        known = self.known if elems.is_cuda else self.known.cpu()
+        return bool(known[elems.clamp(-1, known.numel() - 2) + 1].all())
 
     def layer1_cache(self, nl):
         if not self.knobs.cache_layer1:

@@ -121,9 +121,21 @@ class ChunkGraph:
 def chunk_topology(a, b, e0, e1, pj, loc, flag):
     """Receivers a..b-1 first, then the senders outside [a, b) in ascending order; int32 local sender index per
     edge.  Restates ThreePassMLIAP._topology (mliap_threepass.py:288-310); loc (int32, -1) and flag (bool, False)
-    are scratch arrays over all atoms and are restored before returning."""
+    are scratch arrays over all atoms and are restored before returning.  On the GPU (int32 senders) the kernels of
+    csrc/csr.hip build it with scratch of their own (loc gives the atom count), one device-to-host read."""
     dev = pj.device
     nC = b - a
+    if pj.is_cuda and pj.dtype == torch.int32 and nC > 0:
+        nt, E, send = loc.numel(), e1 - e0, pj[e0:e1].contiguous()
+        w = nt // 32 + 1
+        scratch = torch.zeros(2 + 2 * w + (w + 1023) // 1024, dtype=torch.int32, device=dev)
+        nodes = torch.empty(nC + min(E, nt - nC), dtype=torch.int32, device=dev)
+        ls = torch.empty(E, dtype=torch.int32, device=dev)
+        K.mm_chunk_topology(send, E, a, b, nt, scratch[2:], nodes, ls, scratch, stream())
+        bad, n_new = scratch[:2].tolist()
+        if bad:
+            raise IndexError(f"{bad} senders of receivers [{a}, {b}) are not in [0, {nt})")
+        return nodes[:nC + n_new].clone(), ls
     send_g = pj[e0:e1].long()
     loc[a:b] = torch.arange(nC, device=dev, dtype=loc.dtype)
     flag[send_g] = True
