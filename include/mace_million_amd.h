@@ -194,6 +194,9 @@ int mm_spline_coeffs_flat(const double* samples, int M, int D, double eps, doubl
  * recv are int32, or int64 with index64 != 0; strides in elements; send and send32 may both be null. */
 int mm_edge_csr(const void* send, long send_stride, const void* recv, long recv_stride, int index64, int E, int n,
                 int n_send, int* send32, int* rowptr, int* bad, mm_stream_t stream);
+/* Stable sort: keys [E] in [0, n) -> keys_out [E] ascending and perm [E], the position each came from (keys equal in
+ * their original order).  keys, keys_out, perm and scratch (2 E + 256 (ceil(E / 4096) + 1) ints) do not overlap. */
+int mm_stable_sort(const int* keys, int E, int n, int* keys_out, int* perm, int* scratch, mm_stream_t stream);
 /* ThreePassMLIAP._topology (mliap_threepass.py:288-310) of receivers a..b-1 with the senders send [E] in [0, nt):
  * nodes = a..b-1, then the senders outside [a, b) in ascending order (room for b - a + min(E, nt - b + a)); ls [E] = row
  * of each edge's sender in nodes; status [2] (zeroed by the caller) = senders outside [0, nt) (their ls is not

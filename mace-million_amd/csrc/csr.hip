@@ -179,3 +179,139 @@ extern "C" int mm_chunk_topology(const int* send, int E, int a, int b, int nt, u
     hipLaunchKernelGGL(mm_topo_local_kernel, edges, dim3(256), 0, stream, send, E, a, b, nt, scratch, pre, ls);
   return mm::launch_status("mm_chunk_topology");
 }
+
+// Stable sort of E keys in [0, n) with their positions: a least-significant-digit radix sort of 8 bits a pass, as many
+// passes as n needs (2 for the 30,000 rows of a chunk).  Per pass: digit counts of tiles of 4,096 keys, a prefix sum
+// over each digit's tiles, and the scatter.  In the scatter a wave ranks 64 consecutive keys at a time among equal
+// digits with one ballot per bit, on top of counters in LDS, so equal keys stay in order.  Bound by launches (3 a pass)
+// and the scattered 8-byte writes.  The merge sort of 64-bit keys, histogram and prefix sum it replaces took 0.3 ms for
+// each of a low-memory call's ten sender lists (46,080 atoms, 0.8 M edges each): 22.3 -> 18.6 ms a call.  Unsorted pairs of
+// 12,288 atoms: 4.66 -> 4.41 ms a force call.
+#define MM_SORT_TILE 4096
+#define MM_SORT_ROUNDS (MM_SORT_TILE / 256)
+
+__global__ void __launch_bounds__(256) mm_sort_count_kernel(const int* __restrict__ keys, int E, int shift, int tiles,
+                                                            int* __restrict__ counts) {
+  __shared__ int h[256];
+  h[threadIdx.x] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < MM_SORT_ROUNDS; ++r) {
+    const long e = (long)blockIdx.x * MM_SORT_TILE + 256 * r + threadIdx.x;
+    if (e < E) atomicAdd(&h[((unsigned)keys[e] >> shift) & 255], 1);
+  }
+  __syncthreads();
+  counts[(size_t)threadIdx.x * tiles + blockIdx.x] = h[threadIdx.x];
+}
+
+// exclusive prefix sum of 256 values, one per thread; the total goes to *total
+__device__ __forceinline__ int mm_sort_scan256(int v, int* s, int* total) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int inc = v;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int u = __shfl_up(inc, d);
+    if (lane >= d) inc += u;
+  }
+  if (lane == 63) s[wave] = inc;
+  __syncthreads();
+  int before = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    if (w < wave) before += s[w];
+  }
+  *total = s[0] + s[1] + s[2] + s[3];
+  __syncthreads();
+  return before + inc - v;
+}
+
+// one workgroup per digit: exclusive prefix sum over its tiles, and its total
+__global__ void __launch_bounds__(256) mm_sort_scan_kernel(int* __restrict__ counts, int tiles,
+                                                           int* __restrict__ totals) {
+  __shared__ int s[4];
+  int* __restrict__ row = counts + (size_t)blockIdx.x * tiles;
+  int carry = 0;
+  for (int t0 = 0; t0 < tiles; t0 += 256) {
+    const int t = t0 + threadIdx.x;
+    int total;
+    const int x = mm_sort_scan256(t < tiles ? row[t] : 0, s, &total);
+    if (t < tiles) row[t] = carry + x;
+    carry += total;
+  }
+  if (threadIdx.x == 0) totals[blockIdx.x] = carry;
+}
+
+// vals null: the positions 0 .. E - 1
+__global__ void __launch_bounds__(256) mm_sort_scatter_kernel(const int* __restrict__ keys, const int* __restrict__ vals,
+                                                              int E, int shift, int tiles,
+                                                              const int* __restrict__ counts,
+                                                              const int* __restrict__ totals,
+                                                              int* __restrict__ keys_out, int* __restrict__ vals_out) {
+  __shared__ int cnt[4][256];
+  __shared__ int s[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const long e0 = (long)blockIdx.x * MM_SORT_TILE + wave * (MM_SORT_TILE / 4) + lane;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) cnt[w][tid] = 0;
+  int key[MM_SORT_ROUNDS], rank[MM_SORT_ROUNDS];
+#pragma unroll
+  for (int r = 0; r < MM_SORT_ROUNDS; ++r) key[r] = e0 + 64 * r < E ? keys[e0 + 64 * r] : 0;
+  int unused;
+  const int digit0 = mm_sort_scan256(totals[tid], s, &unused);   // its barriers also cover the cleared counters
+#pragma unroll
+  for (int r = 0; r < MM_SORT_ROUNDS; ++r) {
+    const bool ok = e0 + 64 * r < E;
+    const int d = ((unsigned)key[r] >> shift) & 255;
+    unsigned long long same = __ballot(ok);
+#pragma unroll
+    for (int b = 0; b < 8; ++b) {
+      const unsigned long long m = __ballot((d >> b) & 1);
+      same &= (d >> b) & 1 ? m : ~m;
+    }
+    const int before = __popcll(same & ((1ull << lane) - 1));
+    const int c = cnt[wave][d];
+    rank[r] = c + before;
+    mm_wave_lds_sync();
+    if (ok && before == 0) cnt[wave][d] = c + __popcll(same);
+    mm_wave_lds_sync();
+  }
+  __syncthreads();
+  int at = digit0 + counts[(size_t)tid * tiles + blockIdx.x];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const int c = cnt[w][tid];
+    cnt[w][tid] = at;
+    at += c;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < MM_SORT_ROUNDS; ++r) {
+    const long e = e0 + 64 * r;
+    if (e >= E) continue;
+    const long o = cnt[wave][((unsigned)key[r] >> shift) & 255] + rank[r];
+    keys_out[o] = key[r];
+    vals_out[o] = vals ? vals[e] : (int)e;
+  }
+}
+
+extern "C" int mm_stable_sort(const int* keys, int E, int n, int* keys_out, int* perm, int* scratch,
+                              hipStream_t stream) {
+  MM_CHECK_ARG(E >= 0 && n >= 0, "bad sizes");
+  if (E == 0) return MM_OK;
+  const int tiles = (int)(((long)E + MM_SORT_TILE - 1) / MM_SORT_TILE);
+  int *tk = scratch, *tv = scratch + E, *counts = scratch + 2 * (size_t)E, *totals = counts + 256 * (size_t)tiles;
+  int passes = 1;
+  while (passes < 4 && (unsigned)(n > 0 ? n - 1 : 0) >> (8 * passes)) ++passes;
+  const int *k = keys, *v = nullptr;
+  for (int p = 0; p < passes; ++p) {
+    const bool last = (passes - p) & 1;   // the passes alternate and end in the outputs
+    int *ko = last ? keys_out : tk, *vo = last ? perm : tv;
+    hipLaunchKernelGGL(mm_sort_count_kernel, dim3(tiles), dim3(256), 0, stream, k, E, 8 * p, tiles, counts);
+    hipLaunchKernelGGL(mm_sort_scan_kernel, dim3(256), dim3(256), 0, stream, counts, tiles, totals);
+    hipLaunchKernelGGL(mm_sort_scatter_kernel, dim3(tiles), dim3(256), 0, stream, k, v, E, 8 * p, tiles, counts, totals,
+                       ko, vo);
+    k = ko;
+    v = vo;
+  }
+  return mm::launch_status("mm_stable_sort");
+}

@@ -63,6 +63,7 @@ SIGNATURES = {
     "mm_gather_rows_csr": [P, P, P, L, I, P, L, I, P],
     "mm_edge_csr": [P, L, P, L, I, I, I, I, P, P, P, P],
     "mm_chunk_topology": [P, I, I, I, I, P, P, P, P, P],
+    "mm_stable_sort": [P, I, I, P, P, P, P],
     # explicit-weight channelwise TP (generated; FusedConvTP)
     **{f"mm_tpw_{n}_fwd": [P, I, P, P, P, L, P, L, P, L, P, L, P] for n in ("l1", "l2", "l0123")},
     **{f"mm_tpw_{n}_bwd": [P, I, P, P, P, L, P, L, P, L, P, L, P, L, P, L, P, L, P] for n in ("l1", "l2", "l0123")},

@@ -22,6 +22,7 @@ import torch
 
 from . import codegen, model as mm
 from ._lib import K, stream
+from .fused_conv import csr_of_sorted, stable_sort
 
 C = 128
 NCB = 8
@@ -101,11 +102,8 @@ def sender_csr(g):
     carries them (the graph executor's static chunk) is used as is."""
     if getattr(g, "sender_rowptr", None) is not None:
         return g.sender_rowptr, g.sender_perm
-    ls = g.ls[:g.nE].long()
-    perm = torch.argsort(ls, stable=True).to(torch.int32)
-    rp = torch.zeros(g.n_nodes + 1, dtype=torch.int32, device=ls.device)
-    rp[1:] = torch.cumsum(torch.bincount(ls, minlength=g.n_nodes), 0).to(torch.int32)
-    return rp, perm
+    keys, perm = stable_sort(g.ls[:g.nE], g.n_nodes)
+    return csr_of_sorted(keys, g.n_nodes), perm
 
 
 class FastLayers:

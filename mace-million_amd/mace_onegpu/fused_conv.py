@@ -94,6 +94,23 @@ def _parse_irreps(text):
     return out
 
 
+def stable_sort(keys, n):
+    """(sorted keys, positions they came from), int32, of GPU keys in [0, n): mm_stable_sort."""
+    E = keys.numel()
+    keys = keys.to(torch.int32).contiguous()
+    out, perm = torch.empty_like(keys), torch.empty_like(keys)
+    scratch = torch.empty(2 * E + 256 * ((E + 4095) // 4096 + 1), dtype=torch.int32, device=keys.device)
+    K.mm_stable_sort(keys, E, n, out, perm, scratch, stream())
+    return out, perm
+
+
+def csr_of_sorted(keys, n):
+    """Row pointers int32 [n + 1] of ascending int32 GPU keys in [0, n)."""
+    buf = torch.zeros(n + 4, dtype=torch.int32, device=keys.device)
+    K.mm_edge_csr(None, 0, keys, 1, 0, keys.numel(), n, n, None, buf[3:], buf, stream())
+    return buf[3:]
+
+
 def receiver_csr(edge_index, n_nodes, n_send_rows):
     """(rowptr int32 [n+1], eid int32 [E] or None when already receiver-sorted, send int32 [E]) with bounds checks
     of both index rows (one device->host read)."""
@@ -121,9 +138,9 @@ def receiver_csr(edge_index, n_nodes, n_send_rows):
         raise IndexError(f"receiver index out of range [0, {n_nodes}): min {int(recv.min())}, max {int(recv.max())}")
     if not unsorted:
         return rowptr, None, send32
-    recv, eid = torch.sort(recv.to(torch.int32), stable=True)
+    recv, eid = stable_sort(recv, n_nodes)
     K.mm_edge_csr(None, 0, recv, 1, 0, E, n_nodes, n_send_rows, None, rowptr, bad, stream())
-    return rowptr, eid.to(torch.int32), send32
+    return rowptr, eid, send32
 
 
 def _check(t, name, cols):

@@ -29,6 +29,7 @@ import torch
 
 from . import chunk_graphs, fast_layers
 from ._lib import K, stream
+from .fused_conv import stable_sort
 from .receiver_chunk_mace import check_chunk, chunk_topology, make_chunk
 
 try:
@@ -126,12 +127,11 @@ class _PairBatch:
         pj = torch.as_tensor(data.pair_j).to(dev).to(torch.int32)
         rij = torch.as_tensor(data.rij).to(dev).to(torch.float64)
         self.perm = None
-        csr = self._csr(pi, nlocal)
-        if csr is None:
-            pi, self.perm = torch.sort(pi, stable=True)
+        self.rowptr, self.rowptr_host, bad, unsorted = self._csr(pi, nlocal)
+        if unsorted and not bad:
+            pi, self.perm = self._sort(pi, nlocal)
             pj, rij = pj[self.perm], rij[self.perm]
-            csr = self._csr(pi, nlocal)
-        self.rowptr, self.rowptr_host, bad = csr
+            self.rowptr, self.rowptr_host, _, _ = self._csr(pi, nlocal)
         self.pair_i, self.pair_j, self.rij = pi.contiguous(), pj.contiguous(), rij.contiguous()
         if check:
             lo_i, hi_i = (int(pi.min()), int(pi.max())) if pi.numel() else (0, 0)
@@ -143,19 +143,26 @@ class _PairBatch:
             raise ValueError(f"ThreePassMLIAP: a pair receiver is not a local atom (nlocal = {nlocal})")
 
     @staticmethod
+    def _sort(pi, nlocal):
+        """(pi in ascending order, stable permutation), receivers in [0, nlocal)."""
+        if not pi.is_cuda or pi.numel() >= 2 ** 31:
+            return torch.sort(pi, stable=True)
+        pi, perm = stable_sort(pi, nlocal)
+        return pi, perm.long()
+
+    @staticmethod
     def _csr(pi, nlocal):
-        """(rowptr on the device, on the host, number of receivers outside [0, nlocal)) of the receivers pi, or None
-        when they are not non-decreasing."""
+        """(rowptr on the device, on the host, number of receivers outside [0, nlocal), whether some receiver is smaller
+        than its predecessor) of the receivers pi; rowptr means something when they are ascending and inside."""
         if pi.numel() >= 2 ** 31 or not pi.is_cuda:
-            if pi.numel() > 1 and bool((pi[1:] < pi[:-1]).any()):
-                return None
+            unsorted = pi.numel() > 1 and bool((pi[1:] < pi[:-1]).any())
             bad = int(((pi < 0) | (pi >= nlocal)).sum())
             rowptr = torch.searchsorted(pi, torch.arange(nlocal + 1, dtype=torch.int32, device=pi.device))
-            return rowptr, rowptr.cpu().numpy(), bad
+            return rowptr, rowptr.cpu().numpy(), bad, unsorted
         buf = torch.zeros(nlocal + 4, dtype=torch.int32, device=pi.device)
         K.mm_edge_csr(None, 0, pi, pi.stride(0), 0, pi.numel(), nlocal, nlocal, None, buf[3:], buf, stream())
         host = buf.cpu().numpy()
-        return None if host[2] else (buf[3:], host[3:], int(host[1]))
+        return buf[3:], host[3:], int(host[1]), bool(host[2])
 
     def restore(self, per_pair):
         """Per-pair results back in the order the pairs arrived in."""

@@ -444,11 +444,9 @@ def pair_to_atom_forces(sysm, PF, graphs=None):
             K.mm_chunk_forces(g.n_nodes, g.nC, g.rowptr, srp, sperm, g.nodes, PF[g.e0:g.e1], F, stream())
         return F
     if not hasattr(sysm, "_s_perm") or sysm._s_perm_E != sysm.send.numel():
-        s_perm = torch.argsort(sysm.send.long(), stable=True)
-        cnt = torch.bincount(sysm.send.long(), minlength=N)
-        s_rowptr = torch.zeros(N + 1, dtype=torch.int64, device=dev)
-        s_rowptr[1:] = torch.cumsum(cnt, 0)
-        sysm._s_perm, sysm._s_rowptr, sysm._s_perm_E = s_perm, s_rowptr, sysm.send.numel()
+        from .fused_conv import csr_of_sorted, stable_sort
+        keys, s_perm = stable_sort(sysm.send, N)
+        sysm._s_perm, sysm._s_rowptr, sysm._s_perm_E = s_perm.long(), csr_of_sorted(keys, N).long(), sysm.send.numel()
     F = torch.empty(N, 3, dtype=torch.float64, device=dev)
     K.mm_pair_forces_to_atoms(N, sysm.rowptr, sysm._s_rowptr, sysm._s_perm, PF, F, stream())
     return F
