@@ -117,70 +117,86 @@ extern "C" int mm_readout1(int n, const float* h1, long h_stride, const float* w
 
 // R2(h2) = sum_j w2_j silu_n(h2 . W1[:, j]) with W1 = r1_w1 / sqrt(C), w2 = r1_w2 / sqrt(16), silu_n = cst silu;
 // eat[i] += scale R2_i;  g_h2[i] = scale dR2/dh2.
-// Four lanes per node (hidden width H <= MM_RO2_HMAX): lane q of a node's group takes the features 4 (q + 4 j) .. + 3,
-// j = 0..7, so the group reads and writes 64 contiguous bytes per access and a lane issues its 8 loads together.
-// W1 is staged in LDS with row stride H + 1 (the 4 lanes of a group read 4 different banks).  The partial
-// pre-activations are summed over the group with two xor-shuffles, which leaves the same sum in all four lanes.
+// 16 lanes per node: lane q takes the features q + 16 j, j = 0..7 (a group reads and writes 64 contiguous bytes per
+// access), and after a reduce-scatter over the group owns the hidden units q and q + 16.  W1 is staged in LDS, padded
+// with zeros to HM = 16 or 32 columns so that the loops have no conditions; with row stride HM + 4 the 16 lanes' 16-byte
+// reads use every bank once.  Bound by the latency of one node's chain: with 4 lanes per node, each holding all hidden
+// units behind a condition per unit, it took 27 us for 192 nodes, 32 us for 16,384 and
+// 63 us for 131,072; now 7, 11 and 40 us.
 #define MM_RO2_HMAX 32
-#define MM_RO2_NODES 64   // nodes per 256-thread workgroup
+#define MM_RO2_NODES 16   // nodes per 256-thread workgroup
+template <int HM>
 __global__ void __launch_bounds__(256) mm_readout2_kernel(int n, const float* __restrict__ h2, long h_stride,
                                                           const float* __restrict__ W1, const float* __restrict__ w2,
                                                           int H, float cst, float scale, double* __restrict__ eat,
                                                           float* __restrict__ gh, long gh_stride) {
-  __shared__ float w1s[MM_C * (MM_RO2_HMAX + 1)];
-  const int ws = H + 1;
-  for (int t = threadIdx.x; t < MM_C * H; t += 256) w1s[(t / H) * ws + t % H] = W1[t];
+  constexpr int WS = HM + 4, OWN = HM / 16;
+  __shared__ float w1s[MM_C * WS];
+  const int q = threadIdx.x & 15;
+  const int node = blockIdx.x * MM_RO2_NODES + (threadIdx.x >> 4);
+  const int row = min(node, n - 1);   // groups past the last node repeat it and store nothing
+  float a[8], w[OWN];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) a[j] = h2[(size_t)row * h_stride + q + 16 * j];
+#pragma unroll
+  for (int o = 0; o < OWN; ++o) w[o] = q + 16 * o < H ? w2[q + 16 * o] : 0.f;
+  for (int t = threadIdx.x; t < MM_C * HM; t += 256) {
+    const int k = t / HM, j = t % HM;
+    w1s[k * WS + j] = j < H ? W1[k * H + j] : 0.f;
+  }
   __syncthreads();
-  const int node = blockIdx.x * MM_RO2_NODES + (threadIdx.x >> 2);
-  if (node >= n) return;   // the four lanes of a group share the node, so no shuffle partner is missing
-  const int q = threadIdx.x & 3;
-  const floatx4* __restrict__ hp = (const floatx4*)(h2 + (size_t)node * h_stride);
-  floatx4 a[8];
+  float z[HM];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) a[j] = hp[q + 4 * j];
-  float z[MM_RO2_HMAX];
-#pragma unroll
-  for (int j = 0; j < MM_RO2_HMAX; ++j) z[j] = 0.f;
+  for (int j = 0; j < HM; ++j) z[j] = 0.f;
 #pragma unroll
   for (int jj = 0; jj < 8; ++jj) {
-    const float* __restrict__ wr = w1s + 4 * (q + 4 * jj) * ws;
+    const floatx4* __restrict__ wr = (const floatx4*)(w1s + (q + 16 * jj) * WS);
 #pragma unroll
-    for (int j = 0; j < MM_RO2_HMAX; ++j) {
-      if (j < H) {
-        z[j] = fmaf(a[jj].x, wr[j], z[j]);
-        z[j] = fmaf(a[jj].y, wr[ws + j], z[j]);
-        z[j] = fmaf(a[jj].z, wr[2 * ws + j], z[j]);
-        z[j] = fmaf(a[jj].w, wr[3 * ws + j], z[j]);
+    for (int j = 0; j < HM / 4; ++j) {
+      const floatx4 x = wr[j];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) z[4 * j + c] = fmaf(a[jj], x[c], z[4 * j + c]);
+    }
+  }
+  // reduce-scatter: after the step of distance d a lane keeps the units that agree with it in that bit
+#pragma unroll
+  for (int d = 8; d; d >>= 1) {
+#pragma unroll
+    for (int o = 0; o < OWN; ++o)
+#pragma unroll
+      for (int j = 0; j < d; ++j) {
+        const float lo = z[16 * o + j], hi = z[16 * o + j + d];
+        const bool up = q & d;
+        z[16 * o + j] = (up ? hi : lo) + __shfl_xor(up ? lo : hi, d);
       }
-    }
   }
-  float e = 0.f;
+  float e = 0.f, u[OWN];
 #pragma unroll
-  for (int j = 0; j < MM_RO2_HMAX; ++j) {
-    if (j < H) {
-      z[j] += __shfl_xor(z[j], 1);
-      z[j] += __shfl_xor(z[j], 2);
-      const float sg = 1.f / (1.f + expf(-z[j]));
-      e += w2[j] * cst * z[j] * sg;
-      z[j] = scale * w2[j] * cst * sg * (1.f + z[j] * (1.f - sg));   // scale * d/dz (w2_j cst silu(z))
-    }
+  for (int o = 0; o < OWN; ++o) {
+    const float x = z[16 * o], sg = 1.f / (1.f + expf(-x));
+    const bool in = q + 16 * o < H;
+    e += in ? w[o] * cst * x * sg : 0.f;
+    u[o] = in ? scale * w[o] * cst * sg * (1.f + x * (1.f - sg)) : 0.f;   // scale * d/dz (w2_j cst silu(z))
   }
+#pragma unroll
+  for (int d = 8; d; d >>= 1) e += __shfl_xor(e, d);
+#pragma unroll
+  for (int o = 0; o < OWN; ++o)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) z[16 * o + j] = __shfl(u[o], j, 16);
+  if (node >= n) return;
   if (q == 0) eat[node] += (double)(scale * e);
-  floatx4* __restrict__ op = (floatx4*)(gh + (size_t)node * gh_stride);
 #pragma unroll
   for (int jj = 0; jj < 8; ++jj) {
-    const float* __restrict__ wr = w1s + 4 * (q + 4 * jj) * ws;
-    floatx4 g = {0.f, 0.f, 0.f, 0.f};
+    const floatx4* __restrict__ wr = (const floatx4*)(w1s + (q + 16 * jj) * WS);
+    float g = 0.f;
 #pragma unroll
-    for (int j = 0; j < MM_RO2_HMAX; ++j) {
-      if (j < H) {
-        g.x = fmaf(z[j], wr[j], g.x);
-        g.y = fmaf(z[j], wr[ws + j], g.y);
-        g.z = fmaf(z[j], wr[2 * ws + j], g.z);
-        g.w = fmaf(z[j], wr[3 * ws + j], g.w);
-      }
+    for (int j = 0; j < HM / 4; ++j) {
+      const floatx4 x = wr[j];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) g = fmaf(z[4 * j + c], x[c], g);
     }
-    op[q + 4 * jj] = g;
+    gh[(size_t)node * gh_stride + q + 16 * jj] = g;
   }
 }
 
@@ -189,8 +205,13 @@ extern "C" int mm_readout2(int n, const float* h2, long h_stride, const float* W
   MM_CHECK_ARG(n >= 0 && H >= 1 && H <= MM_RO2_HMAX, "bad sizes (1 <= H <= 32)");
   MM_CHECK_ARG(h_stride % 4 == 0 && gh_stride % 4 == 0, "row strides must be multiples of 4 floats");
   if (n == 0) return MM_OK;
-  hipLaunchKernelGGL(mm_readout2_kernel, dim3((n + MM_RO2_NODES - 1) / MM_RO2_NODES), dim3(256), 0, stream, n, h2,
-                     h_stride, W1, w2, H, cst, scale, eat, gh, gh_stride);
+  const dim3 grid((n + MM_RO2_NODES - 1) / MM_RO2_NODES);
+  if (H <= 16)
+    hipLaunchKernelGGL(mm_readout2_kernel<16>, grid, dim3(256), 0, stream, n, h2, h_stride, W1, w2, H, cst, scale, eat,
+                       gh, gh_stride);
+  else
+    hipLaunchKernelGGL(mm_readout2_kernel<32>, grid, dim3(256), 0, stream, n, h2, h_stride, W1, w2, H, cst, scale, eat,
+                       gh, gh_stride);
   return mm::launch_status("mm_readout2");
 }
 
