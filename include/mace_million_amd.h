@@ -200,7 +200,8 @@ int mm_stable_sort(const int* keys, int E, int n, int* keys_out, int* perm, int*
 /* ThreePassMLIAP._topology (mliap_threepass.py:288-310) of receivers a..b-1 with the senders send [E] in [0, nt):
  * nodes = a..b-1, then the senders outside [a, b) in ascending order (room for b - a + min(E, nt - b + a)); ls [E] = row
  * of each edge's sender in nodes; status [2] (zeroed by the caller) = senders outside [0, nt) (their ls is not
- * written), senders outside [a, b).  scratch: 2 w + ceil(w / 1024) words, w = nt / 32 + 1, zeroed by the caller. */
+ * written), senders outside [a, b).  scratch: 10 w + ceil(w / 1024) words, w = nt / 32 + 1, 16-byte aligned, the
+ * first 8 w zeroed by the caller. */
 int mm_chunk_topology(const int* send, int E, int a, int b, int nt, unsigned* scratch, int* nodes, int* ls, int* status,
                       mm_stream_t stream);
 int mm_tpw_l1_fwd(const int* rowptr, int nR, const int* eid, const int* send, const float* Y, long y_stride,

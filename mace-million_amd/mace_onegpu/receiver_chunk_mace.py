@@ -128,10 +128,10 @@ def chunk_topology(a, b, e0, e1, pj, loc, flag):
     if pj.is_cuda and pj.dtype == torch.int32 and nC > 0:
         nt, E, send = loc.numel(), e1 - e0, pj[e0:e1].contiguous()
         w = nt // 32 + 1
-        scratch = torch.zeros(2 + 2 * w + (w + 1023) // 1024, dtype=torch.int32, device=dev)
+        scratch = torch.zeros(4 + 10 * w + (w + 1023) // 1024, dtype=torch.int32, device=dev)
         nodes = torch.empty(nC + min(E, nt - nC), dtype=torch.int32, device=dev)
         ls = torch.empty(E, dtype=torch.int32, device=dev)
-        K.mm_chunk_topology(send, E, a, b, nt, scratch[2:], nodes, ls, scratch, stream())
+        K.mm_chunk_topology(send, E, a, b, nt, scratch[4:], nodes, ls, scratch, stream())
         bad, n_new = scratch[:2].tolist()
         if bad:
             raise IndexError(f"{bad} senders of receivers [{a}, {b}) are not in [0, {nt})")
