@@ -9,7 +9,8 @@
 //               dd < r_max^2 and j != i; candidate order preserved.
 // Every fp64 operation is a separately rounded IEEE operation: the file is compiled with -ffp-contract=off and
 // the arithmetic scopes carry "#pragma clang fp contract(off)" (HIP's __dmul_rn / __dadd_rn are plain * and +,
-// which clang would otherwise fuse into FMAs and so change dd at the last bit).  Output: CSR (rowptr int64 [N+1], senders int32 [E]) in the sorted index space.
+// which clang would otherwise fuse into FMAs and so change dd at the last bit).  Output: CSR (rowptr int64 [N+1],
+// senders int32 [E]) in the sorted index space.
 #include "common.h"
 #include "mic.h"
 
@@ -263,14 +264,107 @@ __global__ void __launch_bounds__(256) mm_nl_pairs_kernel(const double* __restri
   }
 }
 
-// Grid of mm_nl_pairs_kernel: a workgroup per cell (16 receivers per workgroup when brute), a cell's receivers shared
-// by up to 8 workgroups while the cells alone give the GPU fewer than 4 workgroups per CU.
-static dim3 nl_pairs_grid(long N, const int* ncell, int brute) {
-  if (brute) return dim3((unsigned)((N + 4 * MM_NL_R - 1) / (4 * MM_NL_R)));
+// The same for boxes of thinly filled cells (gases, slabs and droplets in vacuum), where a workgroup per cell has few
+// receivers to share the candidates and many cells to find empty: a wave per receiver.  Lanes 0 .. 26 look up the
+// cells, then the wave tests 64 candidates at a time from global memory.  Bound by the latency of that chain.
+// Neighbour build, a thread per receiver -> workgroup per cell -> wave per receiver, us: 100,000 atoms of which a cell
+// holds 0.1: 161 -> 1,314 -> 163; 1: 192 -> 598 -> 175; 3.7: 265 -> 320 -> 198; 6.4: 343 -> 247 -> 223; 9.4: 395 ->
+// 232 -> 258; a droplet of 20,000 atoms in 10^6 cells: 429 -> 753 -> 146.
+#define MM_NL_WAVE_WGS (1L << 20)   // workgroups of a launch at most; the waves stride over the receivers
+
+template <bool FILL>
+__global__ void __launch_bounds__(256) mm_nl_wave_kernel(const double* __restrict__ pos, const int* __restrict__ cell,
+                                                         long N, double bx, double by, double bz, int nx, int ny,
+                                                         int nz, const int* __restrict__ start,
+                                                         const int* __restrict__ count, double r2,
+                                                         int* __restrict__ NN, const long* __restrict__ rowptr,
+                                                         int* __restrict__ send,
+                                                         unsigned long long* __restrict__ masks, int cap) {
+  __shared__ int s_end[4][32], s_off[4][32];   // per cell: candidates up to its end, first atom - candidates before it
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const double hx = 0.5 * bx, hy = 0.5 * by, hz = 0.5 * bz;
+  for (long i = (long)blockIdx.x * 4 + wave; i < N; i += (long)gridDim.x * 4) {
+    const long base = FILL ? rowptr[i] : 0;
+    if (FILL && rowptr[i + 1] == base) continue;
+    int st = 0, ct = 0;
+    if (lane < 27) {
+      const int ax = (cell[3 * i] + lane / 9 - 1 + nx) % nx, ay = (cell[3 * i + 1] + (lane / 3) % 3 - 1 + ny) % ny,
+                az = (cell[3 * i + 2] + lane % 3 - 1 + nz) % nz;
+      const int q = (ax * ny + ay) * nz + az;
+      st = start[q];
+      ct = count[q];
+    }
+    const double xi = pos[3 * i], yi = pos[3 * i + 1], zi = pos[3 * i + 2];
+    int inc = ct;
+#pragma unroll
+    for (int d = 1; d < 32; d <<= 1) {
+      const int u = __shfl_up(inc, d);
+      if (lane >= d) inc += u;
+    }
+    const int T = __shfl(inc, 31);   // lanes 27 .. 31 add nothing
+    mm_wave_lds_sync();              // the previous receiver's words have been read
+    if (lane < 32) {
+      s_end[wave][lane] = inc;
+      s_off[wave][lane] = st - (inc - ct);
+    }
+    mm_wave_lds_sync();
+    const bool masked = masks != nullptr && T <= 64L * cap;
+    int n = 0;
+    for (int s = 0; 64 * s < T; ++s) {
+      const int g = 64 * s + lane;
+      const bool in = g < T;
+      int lo = 0, hi = 26;   // first cell that ends beyond g
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        if (s_end[wave][mid] > g) hi = mid;
+        else lo = mid + 1;
+      }
+      const long j = in ? g + s_off[wave][lo] : i;
+      unsigned long long b;
+      if (FILL && masked) {
+        b = masks[i * cap + s];
+      } else {
+#pragma clang fp contract(off)
+        const double dx = mm_mic(xi - pos[3 * j], bx, hx);
+        const double dy = mm_mic(yi - pos[3 * j + 1], by, hy);
+        const double dz = mm_mic(zi - pos[3 * j + 2], bz, hz);
+        const double dd = (dx * dx + dy * dy) + dz * dz;
+        b = __ballot(dd < r2 && j != i);
+        if (!FILL && masked && lane == 0) masks[i * cap + s] = b;
+      }
+      if (FILL && ((b >> lane) & 1ull))
+        send[base + n + __builtin_amdgcn_mbcnt_hi((unsigned)(b >> 32),
+                                                  __builtin_amdgcn_mbcnt_lo((unsigned)b, 0))] = (int)j;
+      n += __popcll(b);
+    }
+    if (!FILL && lane == 0) NN[i] = n;
+  }
+}
+
+// Which kernel takes a box.  brute: 16 receivers per workgroup.  A workgroup per cell where a cell holds MM_NL_MEAN
+// atoms or more on average (figures above), a cell's receivers shared by up to 8 workgroups while the cells alone give
+// the GPU fewer than 4 workgroups per CU; a wave per receiver in thinner boxes, and in boxes of so many cells that a
+// launch with a workgroup each would exceed the 2^32 threads of a launch.
+#define MM_NL_MEAN 8
+template <bool FILL>
+static void nl_pairs_launch(const double* pos, const int* cell, long N, const double* box, const int* ncell,
+                            const int* start, const int* count, double r2, int brute, int* NN, const long* rowptr,
+                            int* send, unsigned long long* masks, int cap, hipStream_t stream) {
   const long cells = (long)ncell[0] * ncell[1] * ncell[2];
-  long y = 1;
-  while (y < 8 && cells * y < 1024) y *= 2;
-  return dim3((unsigned)cells, (unsigned)y);
+  if (!brute && (N < MM_NL_MEAN * cells || cells >= (1L << 23))) {
+    hipLaunchKernelGGL(mm_nl_wave_kernel<FILL>, dim3((unsigned)min((N + 3) / 4, MM_NL_WAVE_WGS)), dim3(256), 0, stream,
+                       pos, cell, N, box[0], box[1], box[2], ncell[0], ncell[1], ncell[2], start, count, r2, NN,
+                       rowptr, send, masks, cap);
+    return;
+  }
+  dim3 grid((unsigned)((N + 4 * MM_NL_R - 1) / (4 * MM_NL_R)));
+  if (!brute) {
+    unsigned y = 1;
+    while (y < 8 && cells * y < 1024) y *= 2;
+    grid = dim3((unsigned)cells, y);
+  }
+  hipLaunchKernelGGL(mm_nl_pairs_kernel<FILL>, grid, dim3(256), 0, stream, pos, N, box[0], box[1], box[2], ncell[0],
+                     ncell[1], ncell[2], start, count, r2, brute, NN, rowptr, send, masks, cap);
 }
 
 extern "C" int mm_nl_workspace_bytes(long N, size_t* bytes) {
@@ -333,11 +427,9 @@ extern "C" int mm_nl_count_masked(const double* pos_s, const int* cell_s, long N
                                   unsigned long long* masks, int cap, hipStream_t stream) {
   MM_CHECK_ARG(N >= 0 && N < (1L << 31) && box && ncell, "bad arguments");
   MM_CHECK_ARG(cap >= 0 && (cap == 0 || masks), "cap words per atom need the mask buffer");
-  (void)cell_s;   // the cells' ranges say which atoms they hold
   if (N == 0) return MM_OK;
-  hipLaunchKernelGGL(mm_nl_pairs_kernel<false>, nl_pairs_grid(N, ncell, brute), dim3(256), 0, stream, pos_s, N, box[0],
-                     box[1], box[2], ncell[0], ncell[1], ncell[2], start, count, r2, brute, NN, (const long*)nullptr,
-                     (int*)nullptr, cap ? masks : nullptr, cap);
+  nl_pairs_launch<false>(pos_s, cell_s, N, box, ncell, start, count, r2, brute, NN, nullptr, nullptr,
+                         cap ? masks : nullptr, cap, stream);
   return mm::launch_status("mm_nl_count");
 }
 
@@ -500,11 +592,9 @@ extern "C" int mm_nl_fill_masked(const double* pos_s, const int* cell_s, long N,
                                  int* send, const unsigned long long* masks, int cap, hipStream_t stream) {
   MM_CHECK_ARG(N >= 0 && N < (1L << 31) && box && ncell, "bad arguments");
   MM_CHECK_ARG(cap >= 0 && (cap == 0 || masks), "cap words per atom need the mask buffer");
-  (void)cell_s;
   if (N == 0) return MM_OK;
-  hipLaunchKernelGGL(mm_nl_pairs_kernel<true>, nl_pairs_grid(N, ncell, brute), dim3(256), 0, stream, pos_s, N, box[0],
-                     box[1], box[2], ncell[0], ncell[1], ncell[2], start, count, r2, brute, (int*)nullptr, rowptr,
-                     send, cap ? (unsigned long long*)masks : nullptr, cap);
+  nl_pairs_launch<true>(pos_s, cell_s, N, box, ncell, start, count, r2, brute, nullptr, rowptr, send,
+                        cap ? (unsigned long long*)masks : nullptr, cap, stream);
   return mm::launch_status("mm_nl_fill");
 }
 
