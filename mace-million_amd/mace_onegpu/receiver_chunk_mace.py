@@ -71,6 +71,8 @@ class System:
         """Mask words per atom in which the count pass leaves its decisions to the fill pass: half as many again as
         the mean number of candidates needs (denser cells are tested twice).  None beyond 2 GB: there the masks would
         rival the pair list itself."""
+        if self.N == 0:
+            return 0
         T = self.N if brute else 27 * self.N / ncells
         cap = int(1.5 * T / 64) + 2
         return cap if 8 * cap * self.N <= 2 << 30 else 0

@@ -50,3 +50,11 @@ def test_bit_exact_with_the_c_oracle(name):
         assert np.array_equal(s.perm.cpu().numpy(), perm) and np.array_equal(s.pos.cpu().numpy(), pos_s)
         assert np.array_equal(s.NN.cpu().numpy(), NN) and np.array_equal(s.rowptr.cpu().numpy(), rowptr)
         assert np.array_equal(s.send.cpu().numpy(), send)
+
+
+def test_no_atoms():
+    from mace_onegpu.receiver_chunk_mace import System
+    for L in ([25.0, 19.0, 31.0], [14.0, 40.0, 33.0]):       # by cells and brute force
+        s = System(np.zeros((0, 3)), np.array(L), np.zeros(0, dtype=int), R, "cuda")
+        assert s.build_neighbors() == 0
+        assert s.rowptr.tolist() == [0] and s.send.numel() == 0 and s.NN.numel() == 0
