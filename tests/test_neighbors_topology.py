@@ -218,3 +218,24 @@ def test_reverse_map_by_sort_is_an_involution():
     recv = np.repeat(np.arange(s.N), NN)
     assert np.array_equal(rev[rev], np.arange(len(send)))
     assert np.array_equal(recv[rev], send) and np.array_equal(np.asarray(send)[rev], recv)
+
+
+@pytest.mark.parametrize("N,box,free,kept", [
+    (196608, (99.3, 99.3, 198.7), 1 << 30, True),         # water: below the pair list, whatever is free
+    (100000, (14.0, 300.0, 238.0), 8 << 30, False),       # thin slab, brute force: 1.9 GB of masks for 36 MB of pairs
+    (100000, (14.0, 300.0, 238.0), 200 << 30, True),
+    (150000, (14.0, 300.0, 357.0), 200 << 30, False),     # more than 2 GB
+    (0, (30.0, 30.0, 30.0), 200 << 30, False)])
+def test_mask_words_are_bounded(monkeypatch, N, box, free, kept):
+    """The neighbour build's temporary masks: at most the pair list's size or a sixteenth of the free memory."""
+    from types import SimpleNamespace
+
+    import torch
+    from mace_onegpu.receiver_chunk_mace import System
+    monkeypatch.setattr(torch.cuda, "mem_get_info", lambda device=None: (free, 288 << 30))
+    ncell = np.floor(np.array(box) / 6.0)
+    s = SimpleNamespace(N=N, box=np.array(box), r_max=6.0, device="cuda")
+    cap = System._mask_words(s, bool((ncell < 3).any()), int(ncell.prod()))
+    assert (cap > 0) == kept
+    pairs = N * N * 4.19 * 216 / np.prod(box)
+    assert 8 * cap * N <= min(2 << 30, max(64 << 20, 4 * pairs, free / 16))
