@@ -95,9 +95,12 @@ def _parse_irreps(text):
 
 
 def stable_sort(keys, n):
-    """(sorted keys, positions they came from), int32, of GPU keys in [0, n): mm_stable_sort."""
+    """(sorted keys, positions they came from), int32, of keys in [0, n): mm_stable_sort on the GPU."""
     E = keys.numel()
     keys = keys.to(torch.int32).contiguous()
+    if not keys.is_cuda:
+        out, perm = torch.sort(keys, stable=True)
+        return out, perm.to(torch.int32)
     out, perm = torch.empty_like(keys), torch.empty_like(keys)
     scratch = torch.empty(2 * E + 256 * ((E + 4095) // 4096 + 1), dtype=torch.int32, device=keys.device)
     K.mm_stable_sort(keys, E, n, out, perm, scratch, stream())
@@ -105,7 +108,9 @@ def stable_sort(keys, n):
 
 
 def csr_of_sorted(keys, n):
-    """Row pointers int32 [n + 1] of ascending int32 GPU keys in [0, n)."""
+    """Row pointers int32 [n + 1] of ascending int32 keys in [0, n)."""
+    if not keys.is_cuda:
+        return torch.searchsorted(keys, torch.arange(n + 1, dtype=keys.dtype)).to(torch.int32)
     buf = torch.zeros(n + 4, dtype=torch.int32, device=keys.device)
     K.mm_edge_csr(None, 0, keys, 1, 0, keys.numel(), n, n, None, buf[3:], buf, stream())
     return buf[3:]
@@ -126,16 +131,23 @@ def receiver_csr(edge_index, n_nodes, n_send_rows):
     if edge_index.dtype not in (torch.int32, torch.int64):
         edge_index = edge_index.long()
     send, recv = edge_index[0], edge_index[1]
-    out = torch.empty(E + n_nodes + 1, dtype=torch.int32, device=dev)
-    send32, rowptr = out[:E], out[E:]
-    bad = torch.zeros(3, dtype=torch.int32, device=dev)
-    K.mm_edge_csr(send, send.stride(0), recv, recv.stride(0), recv.dtype == torch.int64, E, n_nodes, n_send_rows,
-                  send32, rowptr, bad, stream())
-    bad_send, bad_recv, unsorted = bad.tolist()
+    if edge_index.is_cuda:
+        out = torch.empty(E + n_nodes + 1, dtype=torch.int32, device=dev)
+        send32, rowptr = out[:E], out[E:]
+        bad = torch.zeros(3, dtype=torch.int32, device=dev)
+        K.mm_edge_csr(send, send.stride(0), recv, recv.stride(0), recv.dtype == torch.int64, E, n_nodes, n_send_rows,
+                      send32, rowptr, bad, stream())
+        bad_send, bad_recv, unsorted = bad.tolist()
+    else:
+        bad_send, bad_recv = (int(((t < 0) | (t >= m)).sum()) for t, m in ((send, n_send_rows), (recv, n_nodes)))
+        unsorted = bool((recv[1:] < recv[:-1]).any())
     if bad_send:
         raise IndexError(f"sender index out of range [0, {n_send_rows}): min {int(send.min())}, max {int(send.max())}")
     if bad_recv:
         raise IndexError(f"receiver index out of range [0, {n_nodes}): min {int(recv.min())}, max {int(recv.max())}")
+    if not edge_index.is_cuda:
+        recv, eid = stable_sort(recv, n_nodes)
+        return csr_of_sorted(recv, n_nodes), eid if unsorted else None, send.to(torch.int32).contiguous()
     if not unsorted:
         return rowptr, None, send32
     recv, eid = stable_sort(recv, n_nodes)

@@ -40,6 +40,41 @@ def test_module_api_errors():
     assert "built on first use" in repr(ChannelwiseTP([0, 2]))
 
 
+@pytest.mark.parametrize("layout", ["sorted", "unsorted", "int32", "int16", "columns"])
+def test_index_preparation_on_the_cpu(layout):
+    """receiver_csr and sender_csr take CPU tensors (the kernels need the GPU, the index preparation does not)."""
+    from types import SimpleNamespace
+
+    from mace_onegpu.fast_layers import sender_csr
+    from mace_onegpu.fused_conv import receiver_csr
+    rng = np.random.default_rng(0)
+    n, E = 30, 200
+    recv, send = np.sort(rng.integers(3, n - 4, E)), rng.integers(0, n, E)
+    if layout == "unsorted":
+        recv = rng.permutation(recv)
+    ei = torch.from_numpy(np.stack([send, recv]))
+    if layout.startswith("int"):
+        ei = ei.to(getattr(torch, layout))
+    if layout == "columns":
+        ei = ei.t().contiguous().t()
+    rowptr, eid, s32 = receiver_csr(ei, n, n)
+    assert rowptr.dtype == s32.dtype == torch.int32 and np.array_equal(s32.numpy(), send)
+    assert np.array_equal(rowptr.numpy(), np.searchsorted(np.sort(recv), np.arange(n + 1)))
+    if layout == "unsorted":
+        assert eid.dtype == torch.int32 and np.array_equal(eid.numpy(), np.argsort(recv, kind="stable"))
+    else:
+        assert eid is None
+    for row, name in ((0, "sender"), (1, "receiver")):
+        for value in (-1, n):
+            bad = ei.clone()
+            bad[row, 7] = value
+            with pytest.raises(IndexError, match=name):
+                receiver_csr(bad, n, n)
+    srp, perm = sender_csr(SimpleNamespace(ls=s32, nE=E, n_nodes=n))
+    assert np.array_equal(srp.numpy(), np.searchsorted(np.sort(send), np.arange(n + 1)))
+    assert np.array_equal(perm.numpy(), np.argsort(send, kind="stable"))
+
+
 def test_descriptor_from_irreps_strings():
     """The irreps strings of a MACE interaction block (what the reference's path_table reads) give the same
     descriptor as the l lists; multiplicities other than the kernels' and pseudo-parities are refused."""
