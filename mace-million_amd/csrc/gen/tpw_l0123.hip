@@ -5057,7 +5057,8 @@ extern "C" int mm_tpw_l0123_fwd_n(long E, const int* rowptr, int nR, const int* 
   if (nR == 0) return MM_OK;
   const long waves = (long)nR * 2;
   // E < 0: unknown, shared where the receivers alone leave most of the chip idle
-  const bool shared = E < 0 ? waves <= 2048 : true && E >= 18L * nR;
+  // (a launch takes fewer than 2^32 threads)
+  const bool shared = E < 0 ? waves <= 2048 : true && waves < (1L << 24) && E >= 18L * nR;
   dim3 grid((unsigned)(shared ? waves : (waves + 3) / 4)), block(256);
   hipLaunchKernelGGL(shared ? mm_tpw_l0123_fwd_shared_kernel : mm_tpw_l0123_fwd_kernel, grid, block, 0, stream, rowptr, nR, eid, send, Y, y_stride, W,
                      w_stride, X, x_stride, out, out_stride);
@@ -5081,7 +5082,8 @@ extern "C" int mm_tpw_l0123_bwd_n(long E, const int* rowptr, int nR, const int* 
   if (nR == 0) return MM_OK;
   const long waves = (long)nR * 6;
   // E < 0: unknown, shared where the receivers alone leave most of the chip idle
-  const bool shared = E < 0 ? waves <= 2048 : waves <= 8192 && E >= 18L * nR;
+  // (a launch takes fewer than 2^32 threads)
+  const bool shared = E < 0 ? waves <= 2048 : waves <= 8192 && waves < (1L << 24) && E >= 18L * nR;
   dim3 grid((unsigned)(shared ? waves : (waves + 3) / 4)), block(256);
   hipLaunchKernelGGL(shared ? mm_tpw_l0123_bwd_shared_kernel : mm_tpw_l0123_bwd_kernel, grid, block, 0, stream, rowptr, nR, eid, send, Y, y_stride, W,
                      w_stride, X, x_stride, gO, g_stride, gW, gw_stride, gYp, gy_cb_stride, gX, gx_stride);

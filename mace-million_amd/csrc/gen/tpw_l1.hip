@@ -1379,7 +1379,8 @@ extern "C" int mm_tpw_l1_fwd_n(long E, const int* rowptr, int nR, const int* eid
   if (nR == 0) return MM_OK;
   const long waves = (long)nR * 1;
   // E < 0: unknown, shared where the receivers alone leave most of the chip idle
-  const bool shared = E < 0 ? waves <= 2048 : true && E >= 4L * nR;
+  // (a launch takes fewer than 2^32 threads)
+  const bool shared = E < 0 ? waves <= 2048 : true && waves < (1L << 24) && E >= 4L * nR;
   dim3 grid((unsigned)(shared ? waves : (waves + 3) / 4)), block(256);
   hipLaunchKernelGGL(shared ? mm_tpw_l1_fwd_shared_kernel : mm_tpw_l1_fwd_kernel, grid, block, 0, stream, rowptr, nR, eid, send, Y, y_stride, W,
                      w_stride, X, x_stride, out, out_stride);
@@ -1403,7 +1404,8 @@ extern "C" int mm_tpw_l1_bwd_n(long E, const int* rowptr, int nR, const int* eid
   if (nR == 0) return MM_OK;
   const long waves = (long)nR * 1;
   // E < 0: unknown, shared where the receivers alone leave most of the chip idle
-  const bool shared = E < 0 ? waves <= 2048 : true && E >= 4L * nR;
+  // (a launch takes fewer than 2^32 threads)
+  const bool shared = E < 0 ? waves <= 2048 : true && waves < (1L << 24) && E >= 4L * nR;
   dim3 grid((unsigned)(shared ? waves : (waves + 3) / 4)), block(256);
   hipLaunchKernelGGL(shared ? mm_tpw_l1_bwd_shared_kernel : mm_tpw_l1_bwd_kernel, grid, block, 0, stream, rowptr, nR, eid, send, Y, y_stride, W,
                      w_stride, X, x_stride, gO, g_stride, gW, gw_stride, gYp, gy_cb_stride, gX, gx_stride);

@@ -1453,7 +1453,8 @@ def tpw_source(tab, name):
         A("  if (nR == 0) return MM_OK;")
         A(f"  const long waves = (long)nR * {nh_k};")
         A("  // E < 0: unknown, shared where the receivers alone leave most of the chip idle")
-        A(f"  const bool shared = E < 0 ? waves <= 2048 : {few} && E >= {_share_edges(state)}L * nR;")
+        A("  // (a launch takes fewer than 2^32 threads)")
+        A(f"  const bool shared = E < 0 ? waves <= 2048 : {few} && waves < (1L << 24) && E >= {_share_edges(state)}L * nR;")
         A("  dim3 grid((unsigned)(shared ? waves : (waves + 3) / 4)), block(256);")
         if kind == "fwd":
             A(f"  hipLaunchKernelGGL(shared ? mm_{kn}_fwd_shared_kernel : mm_{kn}_fwd_kernel, grid, block, 0, stream, rowptr, nR, eid, send, Y, y_stride, W,")

@@ -75,3 +75,22 @@ def test_indices_out_of_range(row, value):
     ei[row, 1] = value
     with pytest.raises(IndexError, match="sender" if row == 0 else "receiver"):
         receiver_csr(ei, 7, 7)
+
+
+def test_more_receivers_than_one_launch_takes_workgroups():
+    """2^24 receivers of 4 edges (a mean degree at which a workgroup shares a receiver's edges): a workgroup each would
+    be 2^32 threads, more than a launch takes.  All edges read one row of each operand, so every output row is the
+    same; four equal fp32 products, the bar is an ulp of their sum for each of the 3 roundings."""
+    from mace_onegpu._lib import stream
+    d = ChannelwiseTP([0], 0, (0,))
+    fwd, _ = d.kernels(edge_count=True)
+    n = 2 ** 24
+    g = torch.Generator().manual_seed(0)
+    X, W, Y = (torch.randn(1, k, generator=g) for k in (C, C, 16))
+    i32 = dict(dtype=torch.int32, device="cuda")
+    rowptr, zeros = torch.arange(0, 4 * n + 1, 4, **i32), torch.zeros(4 * n, **i32)
+    out = torch.empty(n, C, device="cuda")
+    fwd(4 * n, rowptr, n, zeros, zeros, Y.cuda(), 16, W.cuda(), C, X.cuda(), C, out, C, stream())
+    ref = 4 * d.table["terms"][0][4] * (X * W * Y[:, :1]).double()
+    assert bool((out == out[0]).all())
+    assert float(((out[:1].double().cpu() - ref) / ref).abs().max()) <= 3 * 2.0 ** -23
