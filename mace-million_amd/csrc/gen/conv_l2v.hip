@@ -2,21 +2,10 @@
 #include "../common.h"
 #include "polar.h"
 
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
-typedef float float2v __attribute__((ext_vector_type(2)));
 typedef unsigned uint2v __attribute__((ext_vector_type(2)));
 typedef unsigned uint4v __attribute__((ext_vector_type(4)));
-
-// x = h0 + h1 (fp16, round to nearest even; the difference is exact in fp32): |x - h0 - h1| <= 2^-24 |x| for the
-// scaled operands below.  Two values at a time.
-__device__ __forceinline__ void mm_split2_f16(float x, float y, unsigned& h0, unsigned& h1) {
-  const half2v a = __builtin_convertvector(float2v{x, y}, half2v);
-  const float2v r = float2v{x, y} - __builtin_convertvector(a, float2v);
-  h0 = __builtin_bit_cast(unsigned, a);
-  h1 = __builtin_bit_cast(unsigned, __builtin_convertvector(r, half2v));
-}
 
 __device__ __forceinline__ unsigned mm_load_u32(const unsigned char* p) {
   unsigned v;
@@ -146,11 +135,11 @@ mm_conv2_bwd_vec_kernel(const int* __restrict__ rowptr, int nC, const floatx4* _
   const float mx4 = fmaxf(fmaxf(fabsf(g38), fabsf(g39)), fmaxf(fmaxf(fabsf(g36), fabsf(g37)), fmaxf(fmaxf(fabsf(g34), fabsf(g35)), fmaxf(fmaxf(fabsf(g32), fabsf(g33)), mx3))));
   const int gex = max(__float_as_int(mx4) >> 23, 40);
   const float gsc = __int_as_float((265 - gex) << 23);
-  const float gun = __int_as_float((gex - 11) << 23);   // 1 / gsc
-  const float U0_0 = g0 * gsc;   // l2 = 0: u does not depend on the edge
-  const float U3_1 = g5 * gsc;   // l2 = 0: u does not depend on the edge
-  const float U3_2 = g6 * gsc;   // l2 = 0: u does not depend on the edge
-  const float U3_3 = g7 * gsc;   // l2 = 0: u does not depend on the edge
+  const float gun = __int_as_float((gex - 24) << 23);   // 1 / (gsc MM_POLAR_SCALE)
+  const float U0_0 = g0 * gsc * MM_POLAR_SCALE;   // l2 = 0: the same u for every edge
+  const float U3_1 = g5 * gsc * MM_POLAR_SCALE;   // l2 = 0: the same u for every edge
+  const float U3_2 = g6 * gsc * MM_POLAR_SCALE;   // l2 = 0: the same u for every edge
+  const float U3_3 = g7 * gsc * MM_POLAR_SCALE;   // l2 = 0: the same u for every edge
   g0 *= gsc;
   g1 *= gsc;
   g2 *= gsc;
@@ -191,84 +180,84 @@ mm_conv2_bwd_vec_kernel(const int* __restrict__ rowptr, int nC, const floatx4* _
   g37 *= gsc;
   g38 *= gsc;
   g39 *= gsc;
-  // B operands: lane (channel cl, k-group eg) holds fp16 piece eg & 1 of its channel's constants
-  const bool pb = eg & 1;
+  // B operands: lane (channel cl, k-group eg) holds fp16 piece 1 - (eg & 1) of its channel's constants
+  const bool pb = !(eg & 1);
   uint4v B7_1;
-  { unsigned h0, h1; mm_split2_f16(1.2499999999999998f * g25, 2.4999999999999996f * g24, h0, h1); B7_1[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(fmaf(0.24999999999999997f, g25, 0.8660254037844387f * g23), -0.5f * g22, h0, h1); B7_1[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.25000000000000006f * g21, -2.4999999999999996f * g22, h0, h1); B7_1[2] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-1.25f * g21, 0.f, h0, h1); B7_1[3] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.2499999999999998f, 2.4999999999999996f}, float2v{g25, g24}, h0, h1); B7_1[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(0.24999999999999997f, g25, 0.8660254037844387f * g23), -0.5f}, float2v{1.f, g22}, h0, h1); B7_1[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.25000000000000006f, -2.4999999999999996f}, float2v{g21, g22}, h0, h1); B7_1[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.25f, 0.f}, float2v{g21, 1.f}, h0, h1); B7_1[3] = pb ? h1 : h0; }
   uint4v B7_2;
-  { unsigned h0, h1; mm_split2_f16(0.f, 2.4999999999999996f * g21, h0, h1); B7_2[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(g22, 0.8660254037844387f * g23, h0, h1); B7_2[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(g24, 2.4999999999999996f * g25, h0, h1); B7_2[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{0.f, 2.4999999999999996f}, float2v{1.f, g21}, h0, h1); B7_2[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.0f, 0.8660254037844387f}, float2v{g22, g23}, h0, h1); B7_2[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.0000000000000004f, 2.4999999999999996f}, float2v{g24, g25}, h0, h1); B7_2[2] = pb ? h1 : h0; }
   B7_2[3] = 0;
   uint4v B7_3;
-  { unsigned h0, h1; mm_split2_f16(1.2499999999999998f * g21, 2.4999999999999996f * g22, h0, h1); B7_3[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.24999999999999997f * g21, -0.5f * g24, h0, h1); B7_3[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(fmaf(-0.25000000000000006f, g25, 0.866025403784439f * g23), 2.4999999999999996f * g24, h0, h1); B7_3[2] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.25f * g25, 0.f, h0, h1); B7_3[3] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.2499999999999998f, 2.4999999999999996f}, float2v{g21, g22}, h0, h1); B7_3[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.24999999999999997f, -0.5f}, float2v{g21, g24}, h0, h1); B7_3[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(-0.25000000000000006f, g25, 0.866025403784439f * g23), 2.4999999999999996f}, float2v{1.f, g24}, h0, h1); B7_3[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.25f, 0.f}, float2v{g25, 1.f}, h0, h1); B7_3[3] = pb ? h1 : h0; }
   uint4v B8_0;
-  { unsigned h0, h1; mm_split2_f16(2.091650066335189f * g26, 5.123475382979799f * g27, h0, h1); B8_0[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.620185174601965f * g28, 1.3228756555322956f * g29, h0, h1); B8_0[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.6201851746019658f * g30, 5.123475382979799f * g31, h0, h1); B8_0[2] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(2.0916500663351894f * g32, 0.f, h0, h1); B8_0[3] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{2.091650066335189f, 5.123475382979799f}, float2v{g26, g27}, h0, h1); B8_0[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.620185174601965f, 1.3228756555322956f}, float2v{g28, g29}, h0, h1); B8_0[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.6201851746019658f, 5.123475382979799f}, float2v{g30, g31}, h0, h1); B8_0[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{2.0916500663351894f, 0.f}, float2v{g32, 1.f}, h0, h1); B8_0[3] = pb ? h1 : h0; }
   uint4v B4_1;
-  { unsigned h0, h1; mm_split2_f16(1.0606601717798207f * g10, 2.121320343559642f * g9, h0, h1); B4_1[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.35355339059327384f * g8, 0.f, h0, h1); B4_1[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-1.060660171779821f * g8, 0.f, h0, h1); B4_1[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.0606601717798207f, 2.121320343559642f}, float2v{g10, g9}, h0, h1); B4_1[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.35355339059327384f, 0.f}, float2v{g8, 1.f}, h0, h1); B4_1[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.060660171779821f, 0.f}, float2v{g8, 1.f}, h0, h1); B4_1[2] = pb ? h1 : h0; }
   B4_1[3] = 0;
   uint4v B4_2;
-  { unsigned h0, h1; mm_split2_f16(0.f, 2.121320343559642f * g8, h0, h1); B4_2[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(0.7071067811865478f * g9, 2.121320343559642f * g10, h0, h1); B4_2[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{0.f, 2.121320343559642f}, float2v{1.f, g8}, h0, h1); B4_2[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{0.7071067811865478f, 2.121320343559642f}, float2v{g9, g10}, h0, h1); B4_2[1] = pb ? h1 : h0; }
   B4_2[2] = 0;
   B4_2[3] = 0;
   uint4v B4_3;
-  { unsigned h0, h1; mm_split2_f16(1.0606601717798207f * g8, 0.f, h0, h1); B4_3[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.35355339059327384f * g10, 2.121320343559642f * g9, h0, h1); B4_3[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.060660171779821f * g10, 0.f, h0, h1); B4_3[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.0606601717798207f, 0.f}, float2v{g8, 1.f}, h0, h1); B4_3[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.35355339059327384f, 2.121320343559642f}, float2v{g10, g9}, h0, h1); B4_3[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.060660171779821f, 0.f}, float2v{g10, 1.f}, h0, h1); B4_3[2] = pb ? h1 : h0; }
   B4_3[3] = 0;
   uint4v B5_0;
-  { unsigned h0, h1; mm_split2_f16(1.936491673103708f * g11, 3.8729833462074166f * g12, h0, h1); B5_0[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.1180339887498953f * g13, 3.872983346207417f * g14, h0, h1); B5_0[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.9364916731037083f * g15, 0.f, h0, h1); B5_0[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.936491673103708f, 3.8729833462074166f}, float2v{g11, g12}, h0, h1); B5_0[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.1180339887498953f, 3.872983346207417f}, float2v{g13, g14}, h0, h1); B5_0[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.9364916731037083f, 0.f}, float2v{g15, 1.f}, h0, h1); B5_0[2] = pb ? h1 : h0; }
   B5_0[3] = 0;
   uint4v B9_1;
-  { unsigned h0, h1; mm_split2_f16(fmaf(1.369306393762915f, g39, 0.35355339059327373f * g37), fmaf(2.236067977499789f, g38, 1.7320508075688774f * g36), h0, h1); B9_1[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.7071067811865478f * g35, -2.2360679774997894f * g34, h0, h1); B9_1[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(fmaf(-0.3535533905932738f, g35, -1.3693063937629153f * g33), 0.f, h0, h1); B9_1[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(1.369306393762915f, g39, 0.35355339059327373f * g37), fmaf(2.236067977499789f, g38, 1.7320508075688774f * g36)}, float2v{1.f, 1.f}, h0, h1); B9_1[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.7071067811865478f, -2.2360679774997894f}, float2v{g35, g34}, h0, h1); B9_1[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(-0.3535533905932738f, g35, -1.3693063937629153f * g33), 0.f}, float2v{1.f, 1.f}, h0, h1); B9_1[2] = pb ? h1 : h0; }
   B9_1[3] = 0;
   uint4v B9_2;
-  { unsigned h0, h1; mm_split2_f16(-1.1180339887498947f * g34, -2.8284271247461903f * g35, h0, h1); B9_2[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.8660254037844392f * g36, -2.8284271247461903f * g37, h0, h1); B9_2[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-1.118033988749895f * g38, 0.f, h0, h1); B9_2[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.1180339887498947f, -2.8284271247461903f}, float2v{g34, g35}, h0, h1); B9_2[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.8660254037844392f, -2.8284271247461903f}, float2v{g36, g37}, h0, h1); B9_2[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.118033988749895f, 0.f}, float2v{g38, 1.f}, h0, h1); B9_2[2] = pb ? h1 : h0; }
   B9_2[3] = 0;
   uint4v B9_3;
-  { unsigned h0, h1; mm_split2_f16(fmaf(0.35355339059327373f, g35, -1.369306393762915f * g33), -2.236067977499789f * g34, h0, h1); B9_3[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.7071067811865478f * g37, fmaf(-2.2360679774997894f, g38, 1.7320508075688774f * g36), h0, h1); B9_3[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(fmaf(-1.3693063937629153f, g39, 0.3535533905932738f * g37), 0.f, h0, h1); B9_3[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(0.35355339059327373f, g35, -1.369306393762915f * g33), -2.236067977499789f}, float2v{1.f, g34}, h0, h1); B9_3[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.7071067811865478f, fmaf(-2.2360679774997894f, g38, 1.7320508075688774f * g36)}, float2v{g37, 1.f}, h0, h1); B9_3[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(-1.3693063937629153f, g39, 0.3535533905932738f * g37), 0.f}, float2v{1.f, 1.f}, h0, h1); B9_3[2] = pb ? h1 : h0; }
   B9_3[3] = 0;
   uint2v B1_1;
-  { unsigned h0, h1; mm_split2_f16(g1, 0.f, h0, h1); B1_1[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{0.9999999999999999f, 0.f}, float2v{g1, 1.f}, h0, h1); B1_1[0] = pb ? h1 : h0; }
   B1_1[1] = 0;
   uint2v B1_2;
-  { unsigned h0, h1; mm_split2_f16(0.f, g1, h0, h1); B1_2[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{0.f, 1.0f}, float2v{1.f, g1}, h0, h1); B1_2[0] = pb ? h1 : h0; }
   B1_2[1] = 0;
   uint2v B1_3;
   B1_3[0] = 0;
-  { unsigned h0, h1; mm_split2_f16(g1, 0.f, h0, h1); B1_3[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{0.9999999999999999f, 0.f}, float2v{g1, 1.f}, h0, h1); B1_3[1] = pb ? h1 : h0; }
   uint2v B2_0;
-  { unsigned h0, h1; mm_split2_f16(1.732050807568877f * g2, 1.7320508075688772f * g3, h0, h1); B2_0[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.732050807568877f * g4, 0.f, h0, h1); B2_0[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.732050807568877f, 1.7320508075688772f}, float2v{g2, g3}, h0, h1); B2_0[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.732050807568877f, 0.f}, float2v{g4, 1.f}, h0, h1); B2_0[1] = pb ? h1 : h0; }
   uint2v B6_1;
-  { unsigned h0, h1; mm_split2_f16(fmaf(1.224744871391589f, g20, 0.7071067811865475f * g18), -1.2247448713915892f * g17, h0, h1); B6_1[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-1.224744871391589f * g16, 0.f, h0, h1); B6_1[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(1.224744871391589f, g20, 0.7071067811865475f * g18), -1.2247448713915892f}, float2v{1.f, g17}, h0, h1); B6_1[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.224744871391589f, 0.f}, float2v{g16, 1.f}, h0, h1); B6_1[1] = pb ? h1 : h0; }
   uint2v B6_2;
-  { unsigned h0, h1; mm_split2_f16(-1.2247448713915892f * g17, -1.4142135623730951f * g18, h0, h1); B6_2[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-1.2247448713915892f * g19, 0.f, h0, h1); B6_2[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.2247448713915892f, -1.4142135623730951f}, float2v{g17, g18}, h0, h1); B6_2[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.2247448713915892f, 0.f}, float2v{g19, 1.f}, h0, h1); B6_2[1] = pb ? h1 : h0; }
   uint2v B6_3;
-  { unsigned h0, h1; mm_split2_f16(-1.224744871391589f * g16, -1.2247448713915892f * g19, h0, h1); B6_3[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(fmaf(-1.224744871391589f, g20, 0.7071067811865475f * g18), 0.f, h0, h1); B6_3[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.224744871391589f, -1.2247448713915892f}, float2v{g16, g19}, h0, h1); B6_3[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(-1.224744871391589f, g20, 0.7071067811865475f * g18), 0.f}, float2v{1.f, 1.f}, h0, h1); B6_3[1] = pb ? h1 : h0; }
   if ((int)threadIdx.x < ns) ssend[threadIdx.x] = g_send[(size_t)grp * 208 + threadIdx.x];
   for (int j = threadIdx.x; j < ns * 16; j += 256) gxs4[j] = floatx4{0.f, 0.f, 0.f, 0.f};
   __syncthreads();
@@ -331,27 +320,27 @@ mm_conv2_bwd_vec_kernel(const int* __restrict__ rowptr, int nC, const floatx4* _
     const unsigned sl4 = mm_load_u32(e_slot + eb + 4 * eg);   // slots of four edges (the array is padded)
     // A operands of edge eb + cl: lane group 0 the harmonics, 1 and 2 their two derivatives
     {
-      float P[16], s, cp, sp;
+      float F[16], A[16], s, cp, sp;
       mm_polar(ua.x, ua.y, s, cp, sp);
-      mm_polar_operands(ua.z, s, cp, sp, eg, P);
+      mm_polar_operands(ua.x, ua.y, ua.z, s, cp, sp, eg, F, A);
       mm_wave_lds_sync();   // the previous tile's operands have been read
       if (eg < 3) {
         { uint4v a = {}, b = {};
-          { unsigned h0, h1; mm_split2_f16(P[9], P[10], h0, h1); a[0] = h0; b[0] = h1; }
-          { unsigned h0, h1; mm_split2_f16(P[11], P[12], h0, h1); a[1] = h0; b[1] = h1; }
-          { unsigned h0, h1; mm_split2_f16(P[13], P[14], h0, h1); a[2] = h0; b[2] = h1; }
-          { unsigned h0, h1; mm_split2_f16(P[15], 0.f, h0, h1); a[3] = h0; b[3] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[9], F[10]}, float2v{A[9], A[10]}, h0, h1); a[0] = h0; b[0] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[11], F[12]}, float2v{A[11], A[12]}, h0, h1); a[1] = h0; b[1] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[13], F[14]}, float2v{A[13], A[14]}, h0, h1); a[2] = h0; b[2] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[15], 0.f}, float2v{A[15], 0.f}, h0, h1); a[3] = h0; b[3] = h1; }
           uint4v* __restrict__ d = ya + ((eg * 3 + 0) * 16 + cl) * 2;
           d[0] = a; d[1] = b; }
         { uint4v a = {}, b = {};
-          { unsigned h0, h1; mm_split2_f16(P[4], P[5], h0, h1); a[0] = h0; b[0] = h1; }
-          { unsigned h0, h1; mm_split2_f16(P[6], P[7], h0, h1); a[1] = h0; b[1] = h1; }
-          { unsigned h0, h1; mm_split2_f16(P[8], 0.f, h0, h1); a[2] = h0; b[2] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[4], F[5]}, float2v{A[4], A[5]}, h0, h1); a[0] = h0; b[0] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[6], F[7]}, float2v{A[6], A[7]}, h0, h1); a[1] = h0; b[1] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[8], 0.f}, float2v{A[8], 0.f}, h0, h1); a[2] = h0; b[2] = h1; }
           uint4v* __restrict__ d = ya + ((eg * 3 + 1) * 16 + cl) * 2;
           d[0] = a; d[1] = b; }
         { uint4v a = {}, b = {};
-          { unsigned h0, h1; mm_split2_f16(P[1], P[2], h0, h1); a[0] = h0; b[0] = h1; }
-          { unsigned h0, h1; mm_split2_f16(P[3], 0.f, h0, h1); a[1] = h0; b[1] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[1], F[2]}, float2v{A[1], A[2]}, h0, h1); a[0] = h0; b[0] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[3], 0.f}, float2v{A[3], 0.f}, h0, h1); a[1] = h0; b[1] = h1; }
           uint4v* __restrict__ d = ya + ((eg * 3 + 2) * 16 + cl) * 2;
           d[0] = a; d[1] = b; }
       }
@@ -377,9 +366,9 @@ mm_conv2_bwd_vec_kernel(const int* __restrict__ rowptr, int nC, const floatx4* _
     float gx1_3 = 0.f;
     float gx2_3 = 0.f;
     float gx3_3 = 0.f;
-    const half8v A3_0 = __builtin_bit_cast(half8v, ya[((0) * 16 + cl) * 2 + (eg >> 1)]);
-    const half8v A3_1 = __builtin_bit_cast(half8v, ya[((3) * 16 + cl) * 2 + (eg >> 1)]);
-    const half8v A3_2 = __builtin_bit_cast(half8v, ya[((6) * 16 + cl) * 2 + (eg >> 1)]);
+    const half8v A3_0 = __builtin_bit_cast(half8v, ya[((0) * 16 + cl) * 2 + 1 - (eg >> 1)]);
+    const half8v A3_1 = __builtin_bit_cast(half8v, ya[((3) * 16 + cl) * 2 + 1 - (eg >> 1)]);
+    const half8v A3_2 = __builtin_bit_cast(half8v, ya[((6) * 16 + cl) * 2 + 1 - (eg >> 1)]);
     const floatx4 D0_7_1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A3_0, __builtin_bit_cast(half8v, B7_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     const floatx4 D1_7_1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A3_1, __builtin_bit_cast(half8v, B7_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     const floatx4 D2_7_1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A3_2, __builtin_bit_cast(half8v, B7_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
@@ -498,9 +487,9 @@ mm_conv2_bwd_vec_kernel(const int* __restrict__ rowptr, int nC, const floatx4* _
     floatx4 q3_1 = *(const floatx4*)(tcb + o1 + 1280);
     floatx4 q3_2 = *(const floatx4*)(tcb + o2 + 1280);
     floatx4 q3_3 = *(const floatx4*)(tcb + o3 + 1280);
-    const half8v A2_0 = __builtin_bit_cast(half8v, ya[((1) * 16 + cl) * 2 + (eg >> 1)]);
-    const half8v A2_1 = __builtin_bit_cast(half8v, ya[((4) * 16 + cl) * 2 + (eg >> 1)]);
-    const half8v A2_2 = __builtin_bit_cast(half8v, ya[((7) * 16 + cl) * 2 + (eg >> 1)]);
+    const half8v A2_0 = __builtin_bit_cast(half8v, ya[((1) * 16 + cl) * 2 + 1 - (eg >> 1)]);
+    const half8v A2_1 = __builtin_bit_cast(half8v, ya[((4) * 16 + cl) * 2 + 1 - (eg >> 1)]);
+    const half8v A2_2 = __builtin_bit_cast(half8v, ya[((7) * 16 + cl) * 2 + 1 - (eg >> 1)]);
     const floatx4 D0_4_1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A2_0, __builtin_bit_cast(half8v, B4_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     const floatx4 D1_4_1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A2_1, __builtin_bit_cast(half8v, B4_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     const floatx4 D2_4_1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A2_2, __builtin_bit_cast(half8v, B4_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
@@ -685,9 +674,9 @@ mm_conv2_bwd_vec_kernel(const int* __restrict__ rowptr, int nC, const floatx4* _
     floatx4 q6_1 = *(const floatx4*)(tcb + o1 + 512);
     floatx4 q6_2 = *(const floatx4*)(tcb + o2 + 512);
     floatx4 q6_3 = *(const floatx4*)(tcb + o3 + 512);
-    const half4v A1_0 = __builtin_bit_cast(half4v, *(const uint2v*)&ya[((2) * 16 + cl) * 2 + (eg >> 1)]);
-    const half4v A1_1 = __builtin_bit_cast(half4v, *(const uint2v*)&ya[((5) * 16 + cl) * 2 + (eg >> 1)]);
-    const half4v A1_2 = __builtin_bit_cast(half4v, *(const uint2v*)&ya[((8) * 16 + cl) * 2 + (eg >> 1)]);
+    const half4v A1_0 = __builtin_bit_cast(half4v, *(const uint2v*)&ya[((2) * 16 + cl) * 2 + 1 - (eg >> 1)]);
+    const half4v A1_1 = __builtin_bit_cast(half4v, *(const uint2v*)&ya[((5) * 16 + cl) * 2 + 1 - (eg >> 1)]);
+    const half4v A1_2 = __builtin_bit_cast(half4v, *(const uint2v*)&ya[((8) * 16 + cl) * 2 + 1 - (eg >> 1)]);
     const floatx4 D0_1_1 = __builtin_amdgcn_mfma_f32_16x16x16f16(A1_0, __builtin_bit_cast(half4v, B1_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     const floatx4 D1_1_1 = __builtin_amdgcn_mfma_f32_16x16x16f16(A1_1, __builtin_bit_cast(half4v, B1_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     const floatx4 D2_1_1 = __builtin_amdgcn_mfma_f32_16x16x16f16(A1_2, __builtin_bit_cast(half4v, B1_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
@@ -1194,11 +1183,11 @@ mm_conv2_bwd_vec_det_kernel(const int* __restrict__ rowptr, int nC, const floatx
   const float mx4 = fmaxf(fmaxf(fabsf(g38), fabsf(g39)), fmaxf(fmaxf(fabsf(g36), fabsf(g37)), fmaxf(fmaxf(fabsf(g34), fabsf(g35)), fmaxf(fmaxf(fabsf(g32), fabsf(g33)), mx3))));
   const int gex = max(__float_as_int(mx4) >> 23, 40);
   const float gsc = __int_as_float((265 - gex) << 23);
-  const float gun = __int_as_float((gex - 11) << 23);   // 1 / gsc
-  const float U0_0 = g0 * gsc;   // l2 = 0: u does not depend on the edge
-  const float U3_1 = g5 * gsc;   // l2 = 0: u does not depend on the edge
-  const float U3_2 = g6 * gsc;   // l2 = 0: u does not depend on the edge
-  const float U3_3 = g7 * gsc;   // l2 = 0: u does not depend on the edge
+  const float gun = __int_as_float((gex - 24) << 23);   // 1 / (gsc MM_POLAR_SCALE)
+  const float U0_0 = g0 * gsc * MM_POLAR_SCALE;   // l2 = 0: the same u for every edge
+  const float U3_1 = g5 * gsc * MM_POLAR_SCALE;   // l2 = 0: the same u for every edge
+  const float U3_2 = g6 * gsc * MM_POLAR_SCALE;   // l2 = 0: the same u for every edge
+  const float U3_3 = g7 * gsc * MM_POLAR_SCALE;   // l2 = 0: the same u for every edge
   g0 *= gsc;
   g1 *= gsc;
   g2 *= gsc;
@@ -1239,84 +1228,84 @@ mm_conv2_bwd_vec_det_kernel(const int* __restrict__ rowptr, int nC, const floatx
   g37 *= gsc;
   g38 *= gsc;
   g39 *= gsc;
-  // B operands: lane (channel cl, k-group eg) holds fp16 piece eg & 1 of its channel's constants
-  const bool pb = eg & 1;
+  // B operands: lane (channel cl, k-group eg) holds fp16 piece 1 - (eg & 1) of its channel's constants
+  const bool pb = !(eg & 1);
   uint4v B7_1;
-  { unsigned h0, h1; mm_split2_f16(1.2499999999999998f * g25, 2.4999999999999996f * g24, h0, h1); B7_1[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(fmaf(0.24999999999999997f, g25, 0.8660254037844387f * g23), -0.5f * g22, h0, h1); B7_1[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.25000000000000006f * g21, -2.4999999999999996f * g22, h0, h1); B7_1[2] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-1.25f * g21, 0.f, h0, h1); B7_1[3] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.2499999999999998f, 2.4999999999999996f}, float2v{g25, g24}, h0, h1); B7_1[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(0.24999999999999997f, g25, 0.8660254037844387f * g23), -0.5f}, float2v{1.f, g22}, h0, h1); B7_1[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.25000000000000006f, -2.4999999999999996f}, float2v{g21, g22}, h0, h1); B7_1[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.25f, 0.f}, float2v{g21, 1.f}, h0, h1); B7_1[3] = pb ? h1 : h0; }
   uint4v B7_2;
-  { unsigned h0, h1; mm_split2_f16(0.f, 2.4999999999999996f * g21, h0, h1); B7_2[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(g22, 0.8660254037844387f * g23, h0, h1); B7_2[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(g24, 2.4999999999999996f * g25, h0, h1); B7_2[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{0.f, 2.4999999999999996f}, float2v{1.f, g21}, h0, h1); B7_2[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.0f, 0.8660254037844387f}, float2v{g22, g23}, h0, h1); B7_2[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.0000000000000004f, 2.4999999999999996f}, float2v{g24, g25}, h0, h1); B7_2[2] = pb ? h1 : h0; }
   B7_2[3] = 0;
   uint4v B7_3;
-  { unsigned h0, h1; mm_split2_f16(1.2499999999999998f * g21, 2.4999999999999996f * g22, h0, h1); B7_3[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.24999999999999997f * g21, -0.5f * g24, h0, h1); B7_3[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(fmaf(-0.25000000000000006f, g25, 0.866025403784439f * g23), 2.4999999999999996f * g24, h0, h1); B7_3[2] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.25f * g25, 0.f, h0, h1); B7_3[3] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.2499999999999998f, 2.4999999999999996f}, float2v{g21, g22}, h0, h1); B7_3[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.24999999999999997f, -0.5f}, float2v{g21, g24}, h0, h1); B7_3[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(-0.25000000000000006f, g25, 0.866025403784439f * g23), 2.4999999999999996f}, float2v{1.f, g24}, h0, h1); B7_3[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.25f, 0.f}, float2v{g25, 1.f}, h0, h1); B7_3[3] = pb ? h1 : h0; }
   uint4v B8_0;
-  { unsigned h0, h1; mm_split2_f16(2.091650066335189f * g26, 5.123475382979799f * g27, h0, h1); B8_0[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.620185174601965f * g28, 1.3228756555322956f * g29, h0, h1); B8_0[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.6201851746019658f * g30, 5.123475382979799f * g31, h0, h1); B8_0[2] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(2.0916500663351894f * g32, 0.f, h0, h1); B8_0[3] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{2.091650066335189f, 5.123475382979799f}, float2v{g26, g27}, h0, h1); B8_0[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.620185174601965f, 1.3228756555322956f}, float2v{g28, g29}, h0, h1); B8_0[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.6201851746019658f, 5.123475382979799f}, float2v{g30, g31}, h0, h1); B8_0[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{2.0916500663351894f, 0.f}, float2v{g32, 1.f}, h0, h1); B8_0[3] = pb ? h1 : h0; }
   uint4v B4_1;
-  { unsigned h0, h1; mm_split2_f16(1.0606601717798207f * g10, 2.121320343559642f * g9, h0, h1); B4_1[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.35355339059327384f * g8, 0.f, h0, h1); B4_1[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-1.060660171779821f * g8, 0.f, h0, h1); B4_1[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.0606601717798207f, 2.121320343559642f}, float2v{g10, g9}, h0, h1); B4_1[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.35355339059327384f, 0.f}, float2v{g8, 1.f}, h0, h1); B4_1[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.060660171779821f, 0.f}, float2v{g8, 1.f}, h0, h1); B4_1[2] = pb ? h1 : h0; }
   B4_1[3] = 0;
   uint4v B4_2;
-  { unsigned h0, h1; mm_split2_f16(0.f, 2.121320343559642f * g8, h0, h1); B4_2[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(0.7071067811865478f * g9, 2.121320343559642f * g10, h0, h1); B4_2[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{0.f, 2.121320343559642f}, float2v{1.f, g8}, h0, h1); B4_2[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{0.7071067811865478f, 2.121320343559642f}, float2v{g9, g10}, h0, h1); B4_2[1] = pb ? h1 : h0; }
   B4_2[2] = 0;
   B4_2[3] = 0;
   uint4v B4_3;
-  { unsigned h0, h1; mm_split2_f16(1.0606601717798207f * g8, 0.f, h0, h1); B4_3[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.35355339059327384f * g10, 2.121320343559642f * g9, h0, h1); B4_3[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.060660171779821f * g10, 0.f, h0, h1); B4_3[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.0606601717798207f, 0.f}, float2v{g8, 1.f}, h0, h1); B4_3[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.35355339059327384f, 2.121320343559642f}, float2v{g10, g9}, h0, h1); B4_3[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.060660171779821f, 0.f}, float2v{g10, 1.f}, h0, h1); B4_3[2] = pb ? h1 : h0; }
   B4_3[3] = 0;
   uint4v B5_0;
-  { unsigned h0, h1; mm_split2_f16(1.936491673103708f * g11, 3.8729833462074166f * g12, h0, h1); B5_0[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.1180339887498953f * g13, 3.872983346207417f * g14, h0, h1); B5_0[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.9364916731037083f * g15, 0.f, h0, h1); B5_0[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.936491673103708f, 3.8729833462074166f}, float2v{g11, g12}, h0, h1); B5_0[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.1180339887498953f, 3.872983346207417f}, float2v{g13, g14}, h0, h1); B5_0[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.9364916731037083f, 0.f}, float2v{g15, 1.f}, h0, h1); B5_0[2] = pb ? h1 : h0; }
   B5_0[3] = 0;
   uint4v B9_1;
-  { unsigned h0, h1; mm_split2_f16(fmaf(1.369306393762915f, g39, 0.35355339059327373f * g37), fmaf(2.236067977499789f, g38, 1.7320508075688774f * g36), h0, h1); B9_1[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.7071067811865478f * g35, -2.2360679774997894f * g34, h0, h1); B9_1[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(fmaf(-0.3535533905932738f, g35, -1.3693063937629153f * g33), 0.f, h0, h1); B9_1[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(1.369306393762915f, g39, 0.35355339059327373f * g37), fmaf(2.236067977499789f, g38, 1.7320508075688774f * g36)}, float2v{1.f, 1.f}, h0, h1); B9_1[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.7071067811865478f, -2.2360679774997894f}, float2v{g35, g34}, h0, h1); B9_1[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(-0.3535533905932738f, g35, -1.3693063937629153f * g33), 0.f}, float2v{1.f, 1.f}, h0, h1); B9_1[2] = pb ? h1 : h0; }
   B9_1[3] = 0;
   uint4v B9_2;
-  { unsigned h0, h1; mm_split2_f16(-1.1180339887498947f * g34, -2.8284271247461903f * g35, h0, h1); B9_2[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.8660254037844392f * g36, -2.8284271247461903f * g37, h0, h1); B9_2[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-1.118033988749895f * g38, 0.f, h0, h1); B9_2[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.1180339887498947f, -2.8284271247461903f}, float2v{g34, g35}, h0, h1); B9_2[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.8660254037844392f, -2.8284271247461903f}, float2v{g36, g37}, h0, h1); B9_2[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.118033988749895f, 0.f}, float2v{g38, 1.f}, h0, h1); B9_2[2] = pb ? h1 : h0; }
   B9_2[3] = 0;
   uint4v B9_3;
-  { unsigned h0, h1; mm_split2_f16(fmaf(0.35355339059327373f, g35, -1.369306393762915f * g33), -2.236067977499789f * g34, h0, h1); B9_3[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-0.7071067811865478f * g37, fmaf(-2.2360679774997894f, g38, 1.7320508075688774f * g36), h0, h1); B9_3[1] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(fmaf(-1.3693063937629153f, g39, 0.3535533905932738f * g37), 0.f, h0, h1); B9_3[2] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(0.35355339059327373f, g35, -1.369306393762915f * g33), -2.236067977499789f}, float2v{1.f, g34}, h0, h1); B9_3[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-0.7071067811865478f, fmaf(-2.2360679774997894f, g38, 1.7320508075688774f * g36)}, float2v{g37, 1.f}, h0, h1); B9_3[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(-1.3693063937629153f, g39, 0.3535533905932738f * g37), 0.f}, float2v{1.f, 1.f}, h0, h1); B9_3[2] = pb ? h1 : h0; }
   B9_3[3] = 0;
   uint2v B1_1;
-  { unsigned h0, h1; mm_split2_f16(g1, 0.f, h0, h1); B1_1[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{0.9999999999999999f, 0.f}, float2v{g1, 1.f}, h0, h1); B1_1[0] = pb ? h1 : h0; }
   B1_1[1] = 0;
   uint2v B1_2;
-  { unsigned h0, h1; mm_split2_f16(0.f, g1, h0, h1); B1_2[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{0.f, 1.0f}, float2v{1.f, g1}, h0, h1); B1_2[0] = pb ? h1 : h0; }
   B1_2[1] = 0;
   uint2v B1_3;
   B1_3[0] = 0;
-  { unsigned h0, h1; mm_split2_f16(g1, 0.f, h0, h1); B1_3[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{0.9999999999999999f, 0.f}, float2v{g1, 1.f}, h0, h1); B1_3[1] = pb ? h1 : h0; }
   uint2v B2_0;
-  { unsigned h0, h1; mm_split2_f16(1.732050807568877f * g2, 1.7320508075688772f * g3, h0, h1); B2_0[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(1.732050807568877f * g4, 0.f, h0, h1); B2_0[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.732050807568877f, 1.7320508075688772f}, float2v{g2, g3}, h0, h1); B2_0[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{1.732050807568877f, 0.f}, float2v{g4, 1.f}, h0, h1); B2_0[1] = pb ? h1 : h0; }
   uint2v B6_1;
-  { unsigned h0, h1; mm_split2_f16(fmaf(1.224744871391589f, g20, 0.7071067811865475f * g18), -1.2247448713915892f * g17, h0, h1); B6_1[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-1.224744871391589f * g16, 0.f, h0, h1); B6_1[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(1.224744871391589f, g20, 0.7071067811865475f * g18), -1.2247448713915892f}, float2v{1.f, g17}, h0, h1); B6_1[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.224744871391589f, 0.f}, float2v{g16, 1.f}, h0, h1); B6_1[1] = pb ? h1 : h0; }
   uint2v B6_2;
-  { unsigned h0, h1; mm_split2_f16(-1.2247448713915892f * g17, -1.4142135623730951f * g18, h0, h1); B6_2[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(-1.2247448713915892f * g19, 0.f, h0, h1); B6_2[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.2247448713915892f, -1.4142135623730951f}, float2v{g17, g18}, h0, h1); B6_2[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.2247448713915892f, 0.f}, float2v{g19, 1.f}, h0, h1); B6_2[1] = pb ? h1 : h0; }
   uint2v B6_3;
-  { unsigned h0, h1; mm_split2_f16(-1.224744871391589f * g16, -1.2247448713915892f * g19, h0, h1); B6_3[0] = pb ? h1 : h0; }
-  { unsigned h0, h1; mm_split2_f16(fmaf(-1.224744871391589f, g20, 0.7071067811865475f * g18), 0.f, h0, h1); B6_3[1] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{-1.224744871391589f, -1.2247448713915892f}, float2v{g16, g19}, h0, h1); B6_3[0] = pb ? h1 : h0; }
+  { unsigned h0, h1; mm_split2_f16(float2v{fmaf(-1.224744871391589f, g20, 0.7071067811865475f * g18), 0.f}, float2v{1.f, 1.f}, h0, h1); B6_3[1] = pb ? h1 : h0; }
   if (e0 < e1) {
   floatx4 pkn0, pkn1, pkn2, pkn3, un;   // records and edge vector of the next tile
   unsigned on0, on1, on2, on3;           // its table rows
@@ -1375,27 +1364,27 @@ mm_conv2_bwd_vec_det_kernel(const int* __restrict__ rowptr, int nC, const floatx
     un = e_u[min(eb + 16 + cl, e1 - 1)];
     // A operands of edge eb + cl: lane group 0 the harmonics, 1 and 2 their two derivatives
     {
-      float P[16], s, cp, sp;
+      float F[16], A[16], s, cp, sp;
       mm_polar(ua.x, ua.y, s, cp, sp);
-      mm_polar_operands(ua.z, s, cp, sp, eg, P);
+      mm_polar_operands(ua.x, ua.y, ua.z, s, cp, sp, eg, F, A);
       mm_wave_lds_sync();   // the previous tile's operands have been read
       if (eg < 3) {
         { uint4v a = {}, b = {};
-          { unsigned h0, h1; mm_split2_f16(P[9], P[10], h0, h1); a[0] = h0; b[0] = h1; }
-          { unsigned h0, h1; mm_split2_f16(P[11], P[12], h0, h1); a[1] = h0; b[1] = h1; }
-          { unsigned h0, h1; mm_split2_f16(P[13], P[14], h0, h1); a[2] = h0; b[2] = h1; }
-          { unsigned h0, h1; mm_split2_f16(P[15], 0.f, h0, h1); a[3] = h0; b[3] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[9], F[10]}, float2v{A[9], A[10]}, h0, h1); a[0] = h0; b[0] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[11], F[12]}, float2v{A[11], A[12]}, h0, h1); a[1] = h0; b[1] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[13], F[14]}, float2v{A[13], A[14]}, h0, h1); a[2] = h0; b[2] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[15], 0.f}, float2v{A[15], 0.f}, h0, h1); a[3] = h0; b[3] = h1; }
           uint4v* __restrict__ d = ya + ((eg * 3 + 0) * 16 + cl) * 2;
           d[0] = a; d[1] = b; }
         { uint4v a = {}, b = {};
-          { unsigned h0, h1; mm_split2_f16(P[4], P[5], h0, h1); a[0] = h0; b[0] = h1; }
-          { unsigned h0, h1; mm_split2_f16(P[6], P[7], h0, h1); a[1] = h0; b[1] = h1; }
-          { unsigned h0, h1; mm_split2_f16(P[8], 0.f, h0, h1); a[2] = h0; b[2] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[4], F[5]}, float2v{A[4], A[5]}, h0, h1); a[0] = h0; b[0] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[6], F[7]}, float2v{A[6], A[7]}, h0, h1); a[1] = h0; b[1] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[8], 0.f}, float2v{A[8], 0.f}, h0, h1); a[2] = h0; b[2] = h1; }
           uint4v* __restrict__ d = ya + ((eg * 3 + 1) * 16 + cl) * 2;
           d[0] = a; d[1] = b; }
         { uint4v a = {}, b = {};
-          { unsigned h0, h1; mm_split2_f16(P[1], P[2], h0, h1); a[0] = h0; b[0] = h1; }
-          { unsigned h0, h1; mm_split2_f16(P[3], 0.f, h0, h1); a[1] = h0; b[1] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[1], F[2]}, float2v{A[1], A[2]}, h0, h1); a[0] = h0; b[0] = h1; }
+          { unsigned h0, h1; mm_split2_f16(float2v{F[3], 0.f}, float2v{A[3], 0.f}, h0, h1); a[1] = h0; b[1] = h1; }
           uint4v* __restrict__ d = ya + ((eg * 3 + 2) * 16 + cl) * 2;
           d[0] = a; d[1] = b; }
       }
@@ -1421,9 +1410,9 @@ mm_conv2_bwd_vec_det_kernel(const int* __restrict__ rowptr, int nC, const floatx
     float gx1_3 = 0.f;
     float gx2_3 = 0.f;
     float gx3_3 = 0.f;
-    const half8v A3_0 = __builtin_bit_cast(half8v, ya[((0) * 16 + cl) * 2 + (eg >> 1)]);
-    const half8v A3_1 = __builtin_bit_cast(half8v, ya[((3) * 16 + cl) * 2 + (eg >> 1)]);
-    const half8v A3_2 = __builtin_bit_cast(half8v, ya[((6) * 16 + cl) * 2 + (eg >> 1)]);
+    const half8v A3_0 = __builtin_bit_cast(half8v, ya[((0) * 16 + cl) * 2 + 1 - (eg >> 1)]);
+    const half8v A3_1 = __builtin_bit_cast(half8v, ya[((3) * 16 + cl) * 2 + 1 - (eg >> 1)]);
+    const half8v A3_2 = __builtin_bit_cast(half8v, ya[((6) * 16 + cl) * 2 + 1 - (eg >> 1)]);
     const floatx4 D0_7_1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A3_0, __builtin_bit_cast(half8v, B7_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     const floatx4 D1_7_1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A3_1, __builtin_bit_cast(half8v, B7_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     const floatx4 D2_7_1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A3_2, __builtin_bit_cast(half8v, B7_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
@@ -1542,9 +1531,9 @@ mm_conv2_bwd_vec_det_kernel(const int* __restrict__ rowptr, int nC, const floatx
     floatx4 q3_1 = *(const floatx4*)(tcb + o1 + 1280);
     floatx4 q3_2 = *(const floatx4*)(tcb + o2 + 1280);
     floatx4 q3_3 = *(const floatx4*)(tcb + o3 + 1280);
-    const half8v A2_0 = __builtin_bit_cast(half8v, ya[((1) * 16 + cl) * 2 + (eg >> 1)]);
-    const half8v A2_1 = __builtin_bit_cast(half8v, ya[((4) * 16 + cl) * 2 + (eg >> 1)]);
-    const half8v A2_2 = __builtin_bit_cast(half8v, ya[((7) * 16 + cl) * 2 + (eg >> 1)]);
+    const half8v A2_0 = __builtin_bit_cast(half8v, ya[((1) * 16 + cl) * 2 + 1 - (eg >> 1)]);
+    const half8v A2_1 = __builtin_bit_cast(half8v, ya[((4) * 16 + cl) * 2 + 1 - (eg >> 1)]);
+    const half8v A2_2 = __builtin_bit_cast(half8v, ya[((7) * 16 + cl) * 2 + 1 - (eg >> 1)]);
     const floatx4 D0_4_1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A2_0, __builtin_bit_cast(half8v, B4_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     const floatx4 D1_4_1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A2_1, __builtin_bit_cast(half8v, B4_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     const floatx4 D2_4_1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(A2_2, __builtin_bit_cast(half8v, B4_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
@@ -1729,9 +1718,9 @@ mm_conv2_bwd_vec_det_kernel(const int* __restrict__ rowptr, int nC, const floatx
     floatx4 q6_1 = *(const floatx4*)(tcb + o1 + 512);
     floatx4 q6_2 = *(const floatx4*)(tcb + o2 + 512);
     floatx4 q6_3 = *(const floatx4*)(tcb + o3 + 512);
-    const half4v A1_0 = __builtin_bit_cast(half4v, *(const uint2v*)&ya[((2) * 16 + cl) * 2 + (eg >> 1)]);
-    const half4v A1_1 = __builtin_bit_cast(half4v, *(const uint2v*)&ya[((5) * 16 + cl) * 2 + (eg >> 1)]);
-    const half4v A1_2 = __builtin_bit_cast(half4v, *(const uint2v*)&ya[((8) * 16 + cl) * 2 + (eg >> 1)]);
+    const half4v A1_0 = __builtin_bit_cast(half4v, *(const uint2v*)&ya[((2) * 16 + cl) * 2 + 1 - (eg >> 1)]);
+    const half4v A1_1 = __builtin_bit_cast(half4v, *(const uint2v*)&ya[((5) * 16 + cl) * 2 + 1 - (eg >> 1)]);
+    const half4v A1_2 = __builtin_bit_cast(half4v, *(const uint2v*)&ya[((8) * 16 + cl) * 2 + 1 - (eg >> 1)]);
     const floatx4 D0_1_1 = __builtin_amdgcn_mfma_f32_16x16x16f16(A1_0, __builtin_bit_cast(half4v, B1_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     const floatx4 D1_1_1 = __builtin_amdgcn_mfma_f32_16x16x16f16(A1_1, __builtin_bit_cast(half4v, B1_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     const floatx4 D2_1_1 = __builtin_amdgcn_mfma_f32_16x16x16f16(A1_2, __builtin_bit_cast(half4v, B1_1), floatx4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);

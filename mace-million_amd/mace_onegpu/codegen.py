@@ -592,13 +592,20 @@ def conv_source(tab, layer, need_gx, opts=None):
 # follows: the kernel returns three numbers per edge (dL/dr and two tangential derivatives) where the per-harmonic form
 # returns 17.
 #
-# Products at fp32 accuracy from fp16 matrix instructions: each operand is the sum of two fp16 values (h0 = fp16(x), h1 =
-# fp16(x - h0), |x - h0 - h1| <= 2^-24 |x|; G is scaled per channel into the fp16 range by a power of two, the harmonics are
-# below 6), and all four piece products are taken, side by side along the inner index: k-group 2 a + b of the instruction
-# holds piece a of Y and piece b of G.
+# Products from fp16 matrix instructions: each operand is the sum of two fp16 values, the second from the exact residual
+# (mm_split2_f16), and all four piece products are taken, side by side along the inner index: k-group 3 - 2 a - b of the
+# instruction holds piece a of Y and piece b of G.  (The instruction adds its k-groups in order: the small ones first give
+# a rounding error of 3.4e-8 of the sum's rms, the other way round 5.2e-8; one rounding is 2.5e-8.)  Two pieces hold 23
+# bits, an error of up to 2^-23 of the operand where fp32 has 2^-24, as long as the operand is in the upper part of the
+# fp16 range; both are scaled there by powers of two.  G, per channel, to below 2^15: 23 bits down to 2^-17 of the channel's
+# largest, 2^-40 of it below.  The harmonics: see mm_polar_operands.
+# What that costs is won back where the harmonics are evaluated and the products rounded.  Errors of the kernel alone
+# against 64 bits, same fp32 inputs, per-harmonic form -> here, water and four-species alloy: forces 1.50e-7 -> 1.42e-7
+# and 1.49e-7 -> 1.43e-7, dL/dX 1.24e-7 -> 1.25e-7 and 1.20e-7 -> 1.23e-7.  Of the whole layer-2 pass (24 chunks of 785 to
+# 16,857 receivers): pair forces 5.93e-7 -> 5.92e-7, dL/dh1 4.02e-7 -> 4.02e-7.
 #
-# Measured (16,384 receivers x 90 edges, 1.47 M edges): 2.42 -> 2.20 ms, the edge gradient that reads its partials 0.149 ->
-# 0.028 ms, mm_sender_slots 9 us; the layer-2 pass of that chunk 4.50 -> 4.18 ms.  Errors against 64 bits 5.3e-7 -> 5.2e-7.
+# Measured (16,384 receivers x 90 edges, 1.47 M edges): 2.42 -> 2.20 ms, the edge gradient that reads its partials
+# 0.149 -> 0.028 ms, mm_sender_slots 9 us; the layer-2 pass of that chunk 4.50 -> 4.18 ms.
 # Bound by VALU issue (the spline evaluation, the two products with X and W, the operand split) at 2 waves per SIMD:
 # about 0.2 ms of the matrix time is exposed, 0.25 ms goes into each receiver's operand B, 0.15 ms into the LDS adds.
 # Why this form: fp32 matrix instructions (16x16x1) hold the SIMD's vector ALU while they run (2.64 ms), the fp16 ones
@@ -639,21 +646,10 @@ BWD_VEC_HEADER = """// generated by mace_onegpu/codegen.py -- layer-2 edge convo
 #include "../common.h"
 #include "polar.h"
 
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
 typedef _Float16 half8v __attribute__((ext_vector_type(8)));
-typedef float float2v __attribute__((ext_vector_type(2)));
 typedef unsigned uint2v __attribute__((ext_vector_type(2)));
 typedef unsigned uint4v __attribute__((ext_vector_type(4)));
-
-// x = h0 + h1 (fp16, round to nearest even; the difference is exact in fp32): |x - h0 - h1| <= 2^-24 |x| for the
-// scaled operands below.  Two values at a time.
-__device__ __forceinline__ void mm_split2_f16(float x, float y, unsigned& h0, unsigned& h1) {
-  const half2v a = __builtin_convertvector(float2v{x, y}, half2v);
-  const float2v r = float2v{x, y} - __builtin_convertvector(a, float2v);
-  h0 = __builtin_bit_cast(unsigned, a);
-  h1 = __builtin_bit_cast(unsigned, __builtin_convertvector(r, half2v));
-}
 
 __device__ __forceinline__ unsigned mm_load_u32(const unsigned char* p) {
   unsigned v;
@@ -715,8 +711,22 @@ extern "C" int mm_sender_slots(const int* rowptr, int nC, const int* send, unsig
 }
 """
 
-POLAR_HEADER = """// generated by mace_onegpu/codegen.py -- harmonics of an edge direction and their tangential derivatives
+POLAR_HEADER = """// generated by mace_onegpu/codegen.py -- harmonics of an edge direction and their tangential derivatives, and the
+// split of fp32 operands for fp16 matrix instructions
 #pragma once
+
+typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float float2v __attribute__((ext_vector_type(2)));
+
+// a b = h0 + h1 + error, fp16 values rounded to nearest even, h1 from the exact residual of the product (one rounding):
+// |error| <= 2^-23 |a b| where |a b| >= 2^-2, and <= 2^-25 below.  Two products at a time.
+__device__ __forceinline__ void mm_split2_f16(float2v a, float2v b, unsigned& h0, unsigned& h1) {
+  const half2v h = __builtin_convertvector(a * b, half2v);
+  const float2v f = __builtin_convertvector(h, float2v);
+  h0 = __builtin_bit_cast(unsigned, h);
+  const float2v r = {fmaf(a.x, b.x, -f.x), fmaf(a.y, b.y, -f.y)};
+  h1 = __builtin_bit_cast(unsigned, __builtin_convertvector(r, half2v));
+}
 
 // Polar frame of a unit vector (x, y, z): s = sin(theta), (cp, sp) = (cos, sin)(phi).  At the poles phi = 0.
 __device__ __forceinline__ void mm_polar(float x, float y, float& s, float& cp, float& sp) {
@@ -729,35 +739,40 @@ __device__ __forceinline__ void mm_polar(float x, float y, float& s, float& cp, 
   sp = pole ? 0.f : y * r;
 }
 
-// A-operand values of one edge: P[m], m = 1..15, of the basis B_lm = F_lm(z, s) {cos, sin}(|m| phi) (Y_m = c_m B_m, the
-// c_m folded into the other operand): type 0 the value, type 1 d/dtheta, type 2 (1 / sin(theta)) d/dphi.  The three
-// types differ in one scalar factor per (l, |m|) and in the azimuthal pair, so a lane evaluates its own type only.
-__device__ __forceinline__ void mm_polar_operands(float z, float s, float cp, float sp, int type, float (&P)[16]) {
-  const bool t0 = type == 0, t1 = type == 1;
-  const float z2 = z * z, s2 = s * s, zs = z * s;
-  const float f5 = fmaf(5.f, z2, -1.f);
-  // F_lm | dF_lm/dtheta | |m| F_lm / s
-  const float f10 = t0 ? z : t1 ? -s : 0.f;
-  const float f11 = t0 ? s : t1 ? z : 1.f;
-  const float f20 = t0 ? fmaf(3.f, z2, -1.f) : t1 ? -6.f * zs : 0.f;
-  const float f21 = t0 ? zs : t1 ? z2 - s2 : z;
-  const float f22 = t0 ? s2 : t1 ? 2.f * zs : 2.f * s;
-  const float f30 = t0 ? z * fmaf(5.f, z2, -3.f) : t1 ? -s * fmaf(15.f, z2, -3.f) : 0.f;
-  const float f31 = t0 ? s * f5 : t1 ? z * fmaf(-10.f, s2, f5) : f5;
-  const float f32 = t0 ? z * s2 : t1 ? s * fmaf(2.f, z2, -s2) : 2.f * zs;
-  const float f33 = t0 ? s * s2 : t1 ? 3.f * z * s2 : 3.f * s2;
-  const float c2 = fmaf(cp, cp, -sp * sp), q2 = 2.f * cp * sp;
-  const float c3 = fmaf(cp, c2, -sp * q2), q3 = fmaf(sp, c2, cp * q2);
-  const bool t2 = type == 2;
-  // azimuthal pair (cos, sin)(m phi), or its derivative / m: (-sin, cos)
-  const float a1 = t2 ? -sp : cp, b1 = t2 ? cp : sp;
-  const float a2 = t2 ? -q2 : c2, b2 = t2 ? c2 : q2;
-  const float a3 = t2 ? -q3 : c3, b3 = t2 ? c3 : q3;
-  P[0] = t0 ? 1.f : 0.f;
-  P[1] = f11 * b1; P[2] = f10; P[3] = f11 * a1;
-  P[4] = f22 * b2; P[5] = f21 * b1; P[6] = f20; P[7] = f21 * a1; P[8] = f22 * a2;
-  P[9] = f33 * b3; P[10] = f32 * b2; P[11] = f31 * b1; P[12] = f30; P[13] = f31 * a1; P[14] = f32 * a2;
-  P[15] = f33 * a3;
+// A-operand values of one edge: F[m] A[m], m = 1..15, of the basis B_lm = F_l|m|(z) s^|m| {cos, sin}(|m| phi)
+// (Y_m = c_m B_m, the c_m folded into the other operand): type 0 the value, type 1 d/dtheta, type 2 (1 / s) d/dphi, all
+// times MM_POLAR_SCALE.  They stay below 4.2, so the scaled ones fill the upper end of the fp16 range: two pieces hold
+// a product to 2^-23 of its value down to 2^-15, and to 2^-38 below.  The types differ in one factor per (l, |m|) and
+// in where the azimuthal pairs begin, so a lane evaluates its own type only.  The pairs are turned on by x + i y, which
+// is exact: rms errors of 4e-8 to 7e-8 with the split, half those of products of s, cos(m phi) and sin(m phi).
+#define MM_POLAR_SCALE 8192.f
+__device__ __forceinline__ void mm_polar_operands(float x, float y, float z, float s, float cp, float sp, int type,
+                                                  float (&F)[16], float (&A)[16]) {
+  const bool t0 = type == 0, t1 = type == 1, t2 = type == 2;
+  const float z2 = z * z, s2 = fmaf(x, x, y * y), zk = MM_POLAR_SCALE * z, sk = MM_POLAR_SCALE * s, zz = z + z;
+  const float f5 = fmaf(zz, zz, fmaf(z, z, -1.f));   // 5 z^2 - 1 from exact products
+  // s^|m| {cos, sin}(|m| phi) (type 0), s^(|m| - 1) {cos, sin} (type 1), s^(|m| - 1) {-sin, cos} (type 2)
+  const float c1 = MM_POLAR_SCALE * (t0 ? x : cp), d1 = MM_POLAR_SCALE * (t0 ? y : sp);
+  const float c2 = fmaf(c1, x, -(d1 * y)), d2 = fmaf(c1, y, d1 * x);
+  const float c3 = fmaf(c2, x, -(d2 * y)), d3 = fmaf(c2, y, d2 * x);
+  A[1] = A[5] = A[11] = t2 ? c1 : d1;
+  A[3] = A[7] = A[13] = t2 ? -d1 : c1;
+  A[4] = A[10] = t2 ? c2 : d2;
+  A[8] = A[14] = t2 ? -d2 : c2;
+  A[9] = t2 ? c3 : d3;
+  A[15] = t2 ? -d3 : c3;
+  A[0] = A[2] = A[6] = A[12] = 1.f;
+  // F_lm | |m| z F_lm - s^2 F'_lm (m = 0: -s F'_l0) | |m| F_lm
+  F[0] = t0 ? MM_POLAR_SCALE : 0.f;
+  F[2] = t0 ? zk : t1 ? -sk : 0.f;
+  F[1] = F[3] = t1 ? z : 1.f;
+  F[6] = t0 ? fmaf(zk, zz, fmaf(zk, z, -MM_POLAR_SCALE)) : t1 ? -6.f * z * sk : 0.f;
+  F[5] = F[7] = t1 ? z2 - s2 : z;
+  F[4] = F[8] = t0 ? 1.f : t1 ? zz : 2.f;
+  F[12] = t0 ? zk * (f5 - 2.f) : t1 ? -3.f * sk * f5 : 0.f;
+  F[11] = F[13] = t1 ? z * fmaf(-10.f, s2, f5) : f5;
+  F[10] = F[14] = t0 ? z : t1 ? fmaf(2.f, z2, -s2) : zz;
+  F[9] = F[15] = t0 ? 1.f : t1 ? 3.f * z : 3.f;
 }
 """
 
@@ -797,6 +812,11 @@ def conv2_bwd_vec_source(tab, depth=2):
                 e = f"fmaf({_f(cc)}, g{o}, {e})"
         return e or "0.f"
 
+    def gfactors(w, k, m):
+        """The two factors of an entry (a sum of several terms: the sum and 1)."""
+        lst = G.get((w, k, m), [])
+        return (_f(lst[0][1]), f"g{lst[0][0]}") if len(lst) == 1 else (gexpr(w, k, m), "1.f")
+
     def kernel(name, mode):
         pool = mode == "pool"
         A(f"extern \"C\" __global__ void __launch_bounds__({64 * GROUP}, 2)")
@@ -835,15 +855,15 @@ def conv2_bwd_vec_source(tab, depth=2):
                 mx = f"mx{o // 8}"
         A(f"  const int gex = max(__float_as_int({mx}) >> 23, 40);")
         A(f"  const float gsc = __int_as_float(({127 + 127 + b_exp} - gex) << 23);")
-        A(f"  const float gun = __int_as_float((gex - {b_exp}) << 23);   // 1 / gsc")
+        A(f"  const float gun = __int_as_float((gex - {b_exp + 13}) << 23);   // 1 / (gsc MM_POLAR_SCALE)")
         for w, l2, ks in paths:
             if l2 == 0:
                 for k in ks:
-                    A(f"  const float U{w}_{k} = {gexpr(w, k, 0)} * gsc;   // l2 = 0: u does not depend on the edge")
+                    A(f"  const float U{w}_{k} = {gexpr(w, k, 0)} * gsc * MM_POLAR_SCALE;   // l2 = 0: the same u for every edge")
         for o in range(nO):
             A(f"  g{o} *= gsc;")
-        A("  // B operands: lane (channel cl, k-group eg) holds fp16 piece eg & 1 of its channel's constants")
-        A("  const bool pb = eg & 1;")
+        A("  // B operands: lane (channel cl, k-group eg) holds fp16 piece 1 - (eg & 1) of its channel's constants")
+        A("  const bool pb = !(eg & 1);")
         for w, l2, ks in steps:
             if not l2:
                 continue
@@ -853,11 +873,12 @@ def conv2_bwd_vec_source(tab, depth=2):
                 A(f"  uint{nr}v B{w}_{k};")
                 for j in range(nr):
                     ms = [l2 * l2 + 2 * j + q for q in (0, 1)]
-                    ex = [gexpr(w, k, m) if m < l2 * l2 + nm else "0.f" for m in ms]
-                    if ex == ["0.f", "0.f"]:
+                    ex = [gfactors(w, k, m) if m < l2 * l2 + nm else ("0.f", "1.f") for m in ms]
+                    if all(e[0] == "0.f" for e in ex):
                         A(f"  B{w}_{k}[{j}] = 0;")
                     else:
-                        A(f"  {{ unsigned h0, h1; mm_split2_f16({ex[0]}, {ex[1]}, h0, h1); B{w}_{k}[{j}] = pb ? h1 : h0; }}")
+                        A(f"  {{ unsigned h0, h1; mm_split2_f16(float2v{{{ex[0][0]}, {ex[1][0]}}}, float2v{{{ex[0][1]}, {ex[1][1]}}}, h0, h1); "
+                          f"B{w}_{k}[{j}] = pb ? h1 : h0; }}")
 
         def rec_load(eb):
             """Records of this lane's four edges of the tile at eb (clamped to the receiver's last edge)."""
@@ -898,17 +919,18 @@ def conv2_bwd_vec_source(tab, depth=2):
             A("    const unsigned sl4 = mm_load_u32(e_slot + eb + 4 * eg);   // slots of four edges (the array is padded)")
         A("    // A operands of edge eb + cl: lane group 0 the harmonics, 1 and 2 their two derivatives")
         A("    {")
-        A("      float P[16], s, cp, sp;")
+        A("      float F[16], A[16], s, cp, sp;")
         A("      mm_polar(ua.x, ua.y, s, cp, sp);")
-        A("      mm_polar_operands(ua.z, s, cp, sp, eg, P);")
+        A("      mm_polar_operands(ua.x, ua.y, ua.z, s, cp, sp, eg, F, A);")
         A("      mm_wave_lds_sync();   // the previous tile's operands have been read")
         A("      if (eg < 3) {")
         for d, l2 in enumerate(degrees):
             nm = 2 * l2 + 1
             A(f"        {{ uint4v a = {{}}, b = {{}};")
             for j in range((nm + 1) // 2):
-                v = [f"P[{l2 * l2 + 2 * j + q}]" if 2 * j + q < nm else "0.f" for q in (0, 1)]
-                A(f"          {{ unsigned h0, h1; mm_split2_f16({v[0]}, {v[1]}, h0, h1); a[{j}] = h0; b[{j}] = h1; }}")
+                m = [l2 * l2 + 2 * j + q for q in (0, 1)]
+                v = [", ".join(f"{nm}[{q}]" if q < l2 * l2 + nm2 else "0.f" for q in m) for nm, nm2 in (("F", nm), ("A", nm))]
+                A(f"          {{ unsigned h0, h1; mm_split2_f16(float2v{{{v[0]}}}, float2v{{{v[1]}}}, h0, h1); a[{j}] = h0; b[{j}] = h1; }}")
             A(f"          uint4v* __restrict__ d = ya + ((eg * {len(degrees)} + {d}) * 16 + cl) * 2;")
             A("          d[0] = a; d[1] = b; }")
         A("      }")
@@ -947,7 +969,7 @@ def conv2_bwd_vec_source(tab, depth=2):
                 if l2 != last:
                     d = degrees.index(l2)
                     for ty in range(3):
-                        row = f"ya[(({ty * len(degrees) + d}) * 16 + cl) * 2 + (eg >> 1)]"
+                        row = f"ya[(({ty * len(degrees) + d}) * 16 + cl) * 2 + 1 - (eg >> 1)]"
                         if l2 == 1:
                             A(f"    const half4v A{l2}_{ty} = __builtin_bit_cast(half4v, *(const uint2v*)&{row});")
                         else:

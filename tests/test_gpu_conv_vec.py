@@ -4,7 +4,9 @@ ones and a short last group, more distinct senders than LDS slots, more edges th
 and next to the poles of the polar frame, cotangents from 1e-30 to 1e20 with channels of zeros, lengths below the table
 start; and non-finite cotangents, which must stay visible.
 
-Bars: sums of up to a few thousand products against fp64, 1e-5 of the largest value, as for the per-harmonic kernels."""
+Bars: sums of up to a few thousand products against fp64, 1e-5 of the largest value, as for the per-harmonic kernels; and
+5e-7 in the 2-norm, where the independent errors of a value's factors (operands of 2^-23, some ten fp32 roundings of 2^-24
+at most, a third of that rms) add up to about 2e-7."""
 import numpy as np
 import pytest
 import torch
@@ -114,6 +116,9 @@ def test_against_fp64_autograd(name, scale):
             got = got.double().cpu()
             assert torch.isfinite(got).all()
             assert float((got - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
+            rel = float((got - ref).norm() / ref.norm())
+            print(f"  det {det}: relative error {rel:.2e}", flush=True)
+            assert rel <= 5e-7
 
 
 @pytest.mark.parametrize("bad", [float("nan"), float("inf")])
