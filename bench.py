@@ -689,7 +689,7 @@ def run_conv(a):
     part = torch.empty(8 * E * 17, device="cuda")
     gX = torch.zeros(nN, 4 * C, device="cuda")
     st = stream()
-    slots = (ws["e_slot"], ws["g_send"], ws["g_n"])
+    slots = fl.sender_slots()
     K.mm_sender_slots(g.rowptr, nC, g.ls, *slots, st)
     calls = {
         "conv1_fwd": (lambda: K.mm_conv1_fwd(g.rowptr, nC, pk1, eu1, fl.Xs1, C, fl.tab[0], fl.n_tab, fl.M, out1, rho,

@@ -271,6 +271,8 @@ class ChunkGraphExec:
         fl.ws, fl.ktimer = self.ws, None
         try:
             fl.workspace(self.C, self.n_cap, self.e_cap)
+            if fl.bwd_vec and not fl.deterministic:
+                fl.sender_slots()       # allocated here, on the stream that the replays run on
             self.ws = fl.ws
             bodies = (("A", self._body_A), ("B", self._body_B), ("C", self._body_C))
             side = torch.cuda.Stream()

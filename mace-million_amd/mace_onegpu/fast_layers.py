@@ -345,8 +345,11 @@ class FastLayers:
         nC = max(nC, ws["nC"] if ws else 0)
         n_nodes = max(n_nodes, ws["nN"] if ws else 0)
         E = max(E, ws["E"] if ws else 0)
-        self.ws = None
-        torch.cuda.empty_cache()
+        if ws is not None:
+            # the old buffers go back to the device before the larger ones are taken (1.3 to 5 ms: a first workspace,
+            # which replaces nothing, does without)
+            self.ws = ws = None
+            torch.cuda.empty_cache()
         dev = self.dev
         f = dict(dtype=torch.float32, device=dev)
         i = dict(dtype=torch.int32, device=dev)
@@ -356,10 +359,6 @@ class FastLayers:
         n_part = max(NCB * 3, 17 if self.ace and self.bwd_vec else NCB * 17)
         ws.update(e_u=torch.empty(E, 4, **f), e_pk=torch.empty(E, 4, **f),
                   e_recv=torch.empty(E, **i), e_dd=torch.empty(E, **f), part=torch.empty(n_part * E, **f))
-        if not self.deterministic:      # the layer-2 backward's sender slots (mm_sender_slots)
-            ng = (nC + codegen.GROUP - 1) // codegen.GROUP
-            ws.update(e_slot=torch.empty(E + 64, dtype=torch.uint8, device=dev),
-                      g_send=torch.empty(ng * codegen.SLOTS, **i), g_n=torch.empty(ng, **i))
         if self.deterministic:
             ws["gXe"] = torch.empty(E, 4 * C, **f)       # per-edge dL/dX rows of mm_conv2_bwd_vec_det
         # A (a layer's message, read by the linear after its convolution) and gA (its cotangent, written by the
@@ -373,6 +372,17 @@ class FastLayers:
                   Xh=torch.empty(n_nodes * 4 * C, **f), gXh=torch.empty(n_nodes * 4 * C, **f))
         self.ws = ws
         return ws
+
+    def sender_slots(self):
+        """The workspace's buffers for the layer-2 backward's sender slots (arguments of mm_sender_slots), allocated
+        when pass B first asks for them."""
+        ws = self.ws
+        if "e_slot" not in ws:
+            ng = (ws["nC"] + codegen.GROUP - 1) // codegen.GROUP
+            i = dict(dtype=torch.int32, device=self.dev)
+            ws.update(e_slot=torch.empty(ws["E"] + 64, dtype=torch.uint8, device=self.dev),
+                      g_send=torch.empty(ng * codegen.SLOTS, **i), g_n=torch.empty(ng, **i))
+        return ws["e_slot"], ws["g_send"], ws["g_n"]
 
     # ------------------------------------------------------------------ helpers
     def _lin(self, plan, inp, in_stride, out, out_stride, W, rows, in_rows=None, out_rows=None, scale=None,
@@ -536,7 +546,7 @@ class FastLayers:
         else:
             K.mm_fill_f32(gX, g.n_nodes * D1, 0.0, stream())
             if self.bwd_vec:
-                slots = (ws["e_slot"], ws["g_send"], ws["g_n"])
+                slots = self.sender_slots()
                 K.mm_sender_slots(g.rowptr, g.nC, g.ls, *slots, stream())
         bwd = getattr(K, ("mm_conv2_bwd_vec" if self.bwd_vec else "mm_conv2_bwd") + det)
         self._timed("conv2_bwd", (g.nE, g.nC, g.n_nodes), bwd, g.rowptr, g.nC, ws["e_pk"], ws["e_u"], ws["Xh"], D1,
