@@ -41,3 +41,34 @@ def test_first_workspace_keeps_the_cache_and_layer_1_takes_no_sender_slots(model
     fl.workspace(g.nC + 1, g.n_nodes, g.nE)
     assert len(emptied) == 1 and fl.ws is not old and "e_slot" not in fl.ws
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("deterministic", [False, True])
+def test_pass_b_with_tables_beyond_32_bits(model, chunk, deterministic):
+    """pass_b takes the per-harmonic kernels where one channel block's tables exceed 32-bit addresses (bwd_vec False): 17
+    numbers per partial row instead of 3, and a workspace that holds them.  Both forms agree to 2e-6 in the 2-norm (an
+    error of 7e-7 each against 64 bits) and write nothing behind the chunk's pair forces."""
+    s, g, cols = chunk
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    H1 = torch.randn(s.N, 512, generator=gen, device="cuda")
+    out = {}
+    for vec in (True, False):
+        fl = _layers(model, cols, deterministic=deterministic)
+        assert fl.bwd_vec
+        fl.bwd_vec = vec
+        ws = fl.prepare(g)
+        assert ws["part"].numel() >= 8 * ws["E"] * (3 if vec else 17)
+        # a guard behind the partials: the buffer is replaced by the front of a longer one
+        n = ws["part"].numel()
+        room = torch.full((n + 1024,), 7.0, device="cuda")
+        ws["part"] = room[:n]
+        PF = torch.full((g.nE + 64, 3), 5.0, device="cuda")
+        G1, eat = torch.zeros(s.N, 512, device="cuda"), torch.zeros(s.N, dtype=torch.float64, device="cuda")
+        print(f"case bwd_vec {vec} deterministic {deterministic}: {g.nE} edges", flush=True)
+        fl.pass_b(g, H1, G1, PF, eat)
+        torch.cuda.synchronize()
+        assert bool((room[n:] == 7.0).all()) and bool((PF[g.nE:] == 5.0).all())
+        out[vec] = (PF[:g.nE].double(), G1.double(), eat)
+    assert torch.equal(out[True][2], out[False][2])
+    for a, b in zip(out[True][:2], out[False][:2]):
+        assert float((a - b).norm() / b.norm()) <= 2e-6
