@@ -105,3 +105,12 @@ def test_build_counts_symc_ops_from_assembly():
         for d in ("fwd", "bwd"):
             assert 0.6 * src[d] <= asm[d] <= src[d], (layer, d, asm[d], src[d])
     assert all(v["packed"] == 0 for v in json.load(open(ops)).values())
+
+
+def test_layer_2_backward_is_not_rated_as_a_vector_kernel():
+    """Part of its counted operations run on matrix instructions: its rate is no fraction of the vector ALUs' roof."""
+    k = {n: bench.summarize(n, 1, 2.0, 3e9, 1.1e11, 1) for n in ("conv2_bwd", "conv2_fwd")}
+    assert "valu_frac" not in k["conv2_bwd"] and k["conv2_bwd"]["engine"] == "valu+mfma_f16"
+    assert "valu_frac" in k["conv2_fwd"] and "fp32_equiv_frac" not in k["conv2_fwd"]
+    r = bench.roofline_of({"conv2_bwd": k["conv2_bwd"]})
+    assert "valu_frac" not in r and abs(r["frac"] - r["fp32_equiv_frac"]) < 1e-4 and "matrix" in r["note"]
