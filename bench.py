@@ -3,12 +3,12 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--config 5|4|3|2|1] [--no-cpu] [--graphs]
 
-Prints ONE JSON line.  Default: configuration 5, the metric's "1M-atom water" -- 343,000 rigid H2O molecules
-(1,029,000 atoms) at 1.0 g/cm^3, random-init MPA-0-medium architecture, fp32 kernels, velocity-Verlet MD (dt 0.5 fs,
-300 K Maxwell-Boltzmann start, neighbour skin 2 A, rebuild when an atom moved > 1 A).  One step = one MD step
-(per-step pair filter, energy + forces by the three passes with every full receiver chunk replayed from its HIP
-graphs, integration, rebuilds when due; --no-graphs runs every chunk eagerly).  W untimed steps after the initial
-force call, then K timed steps between synchronisations.
+Prints ONE JSON line on stdout (the full record of the default run goes to stderr).  Default: configuration 5, the
+metric's "1M-atom water" -- 343,000 rigid H2O molecules (1,029,000 atoms) at 1.0 g/cm^3, random-init MPA-0-medium
+architecture, fp32 kernels, velocity-Verlet MD (dt 0.5 fs, 300 K Maxwell-Boltzmann start, neighbour skin 2 A, rebuild
+when an atom moved > 1 A).  One step = one MD step (per-step pair filter, energy + forces by the three passes with every
+full receiver chunk replayed from its HIP graphs, integration, rebuilds when due; --no-graphs runs every chunk eagerly).
+W untimed steps after the initial force call, then K timed steps between synchronisations.
   --config 3 : 98,304-atom water, one energy + force evaluation per step (ReceiverChunkMACE, chunk 16384, full chunks
                replayed from HIP graphs), topology of the chunks rebuilt every call
   --config 4 : 500,000-atom FCC Fe/Ni/Cr/Co alloy (a = 3.6 A, sigma 0.05 A), one energy + force evaluation per step
@@ -20,10 +20,10 @@ force call, then K timed steps between synchronisations.
 Objects beside the contract fields:
   roofline     : the dominant kernel, algorithmic bytes (or FLOPs) per launch / mean launch time measured with HIP
                  events on the launch stream (during the timed steps; with graphs, in one eager step after them).
-                 bound: "valu" for the edge convolutions (fp32 v_fma_f32 on the vector ALUs, roof 157.3 TFLOP/s: gfx950
-                 dual-issues VALU instructions of two waves; the layer-2 backward has part of its operations on fp16
-                 MFMA), "mfma" for the matrix-core kernels, "hbm" below the ridge; traffic = measured HBM bytes per launch
-                 from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE passes of this workload (or null)
+                 bound: "valu" for the edge convolutions (fp32 v_fma_f32 on the vector ALUs, roof 157.3 TFLOP/s:
+                 gfx950 dual-issues VALU instructions of two waves; the layer-2 backward has part of its operations
+                 on fp16 MFMA), "mfma" for the matrix-core kernels, "hbm" below the ridge; traffic = measured HBM
+                 bytes per launch from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE passes of this workload (or null)
   node_kernels : the linears (bf16 MFMA: mfma_frac = 6 F / t / 2.5 PFLOP/s; fp32_equiv_frac = F / t / 157.3) and the
                  symmetric contractions (HBM roof; FLOPs = the operations the generated kernels execute) timed with
                  HIP events in one extra step after the timed ones
@@ -35,8 +35,9 @@ Objects beside the contract fields:
                  restatement's layer-2 convolution forward and backward on 2,048 receivers of the chunk with the GPU
                  run's inputs, scaled to the chunk (and the GPU kernels' outputs checked against it); config 1: the
                  fp64 restatement on the whole box, median of 3
-  configs      : (default run) configurations 3, 4, 2 and 1 measured in the same process after configuration 5, each
-                 with its value, dominant-kernel roofline, per-kernel table and CPU baseline
+  configs      : (default run) configurations 3, 4, 2 and 1 measured in the same process after configuration 5:
+                 metric, value and time; in the full record on stderr ("# full record: {...}") also their rooflines,
+                 per-kernel tables and CPU baselines, and configuration 5's tables
 """
 import argparse
 import json
@@ -262,8 +263,8 @@ def roofline_of(kernels, workload=None):
     kernel = f"mm_{KERNEL_NAMES.get(dom, dom)}_kernel"
     out = {"kernel": kernel}
     if compute:
-        out.update({"bound": "valu" if eng.startswith("valu") else "mfma", "achieved": round(k["TFLOPs"], 3), "peak": peak,
-                    "unit": "TFLOP/s", "frac": round(k["TFLOPs"] / peak, 4),
+        out.update({"bound": "valu" if eng.startswith("valu") else "mfma", "achieved": round(k["TFLOPs"], 3),
+                    "peak": peak, "unit": "TFLOP/s", "frac": round(k["TFLOPs"] / peak, 4),
                     "frac_of_fp32_chip_peak": round(k["TFLOPs"] / FP32_CHIP_PEAK_TFLOPS, 4)})
     else:
         out.update({"bound": "hbm", "achieved": round(k["GBps"], 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
@@ -276,9 +277,9 @@ def roofline_of(kernels, workload=None):
                 "bytes_per_launch": int(k["bytes_per_launch"]), "flops_per_launch": int(k["flops_per_launch"]),
                 "ms_per_launch": round(k["ms_per_launch"], 4), "launches": k["launches"]})
     if compute and eng == "valu+mfma_f16":
-        out["note"] = ("achieved and frac count the model's fp32 operations over the chip's fp32 figure; the contraction "
-                       "over the harmonics, part of them, runs on fp16 matrix instructions, and the kernel is bound by "
-                       "the issue of the rest on the vector ALUs: frac is no fraction of the vector ALUs' roof")
+        out["note"] = ("achieved and frac count the model's fp32 operations over the chip's fp32 figure; part of them "
+                       "(the contraction over the harmonics) runs on fp16 matrix instructions, and the kernel is bound "
+                       "by the issue of the rest on the vector ALUs: frac is no fraction of the vector ALUs' roof")
     elif compute and eng == "valu":
         out["note"] = ("the kernel runs on the vector ALUs (v_fma_f32, no packed FP32): 157.3 TFLOP/s needs two VALU "
                        "instructions from two waves per SIMD issued per quad-cycle (gfx950 dual issue; 151.6 TFLOP/s "
@@ -847,6 +848,20 @@ def sub_line(line):
     return {k: line[k] for k in keep if k in line}
 
 
+# what the default run's line leaves to the full record: per-kernel tables and the step's own roofline
+TABLES = ("kernels", "node_kernels", "step_roofline", "roofline_note")
+
+
+def brief(line):
+    """The default run's line: the contract fields, roofline and CPU baseline of configuration 5, and of each other
+    configuration its metric, value and time.  (With every table, some 25 kB, a reader that keeps the last few
+    kilobytes of the output loses the head of the line.)"""
+    out = {k: v for k, v in line.items() if k not in TABLES + ("configs",)}
+    out["configs"] = {c: {k: r[k] for k in ("metric", "value", "unit", "steps", "ms_per_step") if k in r}
+                      for c, r in line["configs"].items()}
+    return out
+
+
 def free_gpu():
     import gc
 
@@ -1041,6 +1056,8 @@ def main():
             run = {1: run_config1, 2: run_conv, 3: run_ef, 4: run_ef}[c]
             extras[f"config{c}"] = sub_line(run(b))
         line["configs"] = extras
+        print("# full record: " + json.dumps(line), file=sys.stderr, flush=True)
+        line = brief(line)
     print(json.dumps(line), flush=True)
 
 

@@ -114,3 +114,25 @@ def test_layer_2_backward_is_not_rated_as_a_vector_kernel():
     assert "valu_frac" in k["conv2_fwd"] and "fp32_equiv_frac" not in k["conv2_fwd"]
     r = bench.roofline_of({"conv2_bwd": k["conv2_bwd"]})
     assert "valu_frac" not in r and abs(r["frac"] - r["fp32_equiv_frac"]) < 1e-4 and "matrix" in r["note"]
+
+
+def test_default_line_is_short():
+    """The default run's line stays below 4 kB, with the contract's fields, whatever the tables hold."""
+    kernels = {f"kernel_{j}": bench.summarize("conv2_fwd", 8, 2.0, 3e9, 1.1e11, 1) for j in range(12)}
+    roof = dict(bench.roofline_of({"conv2_bwd": bench.summarize("conv2_bwd", 8, 2.0, 3e9, 1.1e11, 1)}))
+    cpu = {"value": 1.0, "unit": "atom-steps/s", "note": "x" * 600}
+
+    class A:
+        steps, warmup = 20, 5
+    line = bench.base_line(A, "atom-steps/s (E+F, 1M-atom water, fp32, 1 GPU)", 3.4e6, 300.1, "atom-steps/s",
+                           "synthetic (seeded water generator, random-init weights)", {"workload": "w" * 300}, roof,
+                           kernels, cpu)
+    line.update(node_kernels=kernels, step_roofline={"note": "y" * 600}, roofline_note="z" * 200)
+    line["configs"] = {f"config{c}": bench.sub_line(dict(line)) for c in (3, 4, 2, 1)}
+    out = bench.brief(line)
+    assert len(json.dumps(line)) > 20000 and len(json.dumps(out)) < 4096
+    for k in ("metric", "value", "unit", "n_gpus", "steps", "warmup", "ms_per_step", "higher_is_better", "scaling",
+              "vs_baseline", "dtype", "data", "config", "roofline", "cpu_baseline"):
+        assert out[k] == line[k]
+    assert set(out["configs"]) == {"config1", "config2", "config3", "config4"}
+    assert all(set(v) == {"metric", "value", "unit", "steps", "ms_per_step"} for v in out["configs"].values())
