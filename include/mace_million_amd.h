@@ -198,8 +198,8 @@ int mm_edge_csr(const void* send, long send_stride, const void* recv, long recv_
  * their original order).  keys, keys_out, perm and scratch (2 E + 256 (ceil(E / 4096) + 1) ints) do not overlap. */
 int mm_stable_sort(const int* keys, int E, int n, int* keys_out, int* perm, int* scratch, mm_stream_t stream);
 /* ThreePassMLIAP._topology (mliap_threepass.py:288-310) of receivers a..b-1 with the senders send [E] in [0, nt):
- * nodes = a..b-1, then the senders outside [a, b) in ascending order (room for b - a + min(E, nt - b + a)); ls [E] = row
- * of each edge's sender in nodes; status [2] (zeroed by the caller) = senders outside [0, nt) (their ls is not
+ * nodes = a..b-1, then the senders outside [a, b) in ascending order (room for b - a + min(E, nt - b + a)); ls [E] =
+ * row of each edge's sender in nodes; status [2] (zeroed by the caller) = senders outside [0, nt) (their ls is not
  * written), senders outside [a, b).  scratch: 10 w + ceil(w / 1024) words, w = nt / 32 + 1, 16-byte aligned, the
  * first 8 w zeroed by the caller. */
 int mm_chunk_topology(const int* send, int E, int a, int b, int nt, unsigned* scratch, int* nodes, int* ls, int* status,

@@ -1,6 +1,6 @@
-// Receiver CSR of an edge list for the explicit-weight convolution and of ML-IAP pairs: index checks, int32 senders and the row pointers in
-// one launch instead of a chain of elementwise, reduction and histogram launches (the chain took 0.1 ms, more than
-// the convolution of a small graph).
+// Receiver CSR of an edge list for the explicit-weight convolution and of ML-IAP pairs: index checks, int32 senders and
+// the row pointers in one launch instead of a chain of elementwise, reduction and histogram launches (the chain took
+// 0.1 ms, more than the convolution of a small graph).
 #include "common.h"
 
 // Workgroups below n_edge_wg: four edges per thread, send32[e] and the violation counts (adds of the few that occur;
@@ -62,11 +62,11 @@ extern "C" int mm_edge_csr(const void* send, long send_stride, const void* recv,
 
 // Topology of one receiver chunk [a, b): the node list (the receivers, then the senders outside [a, b) in ascending
 // order) and the local sender index of every edge.  A byte per atom marks the outside senders (plain stores of 1: with
-// atomics on bits the marks of 1.5 M edges took 121 us, of 192 atoms 16 us); a prefix sum over words of 32 marks gives each
-// its place, so nothing is sorted.  Bound by launches
-// for a small chunk and by the edges' senders, read twice, for a large one.  Four launches take the place of 18 tensor
-// operations: together with mm_edge_csr for the pairs' receivers and fewer device-to-host reads, a force call on 192 atoms
-// goes from 1000 to 720 us, on 12,288 atoms in one chunk from 5.07 to 4.66 ms.
+// atomics on bits the marks of 1.5 M edges took 121 us, of 192 atoms 16 us); a prefix sum over words of 32 marks gives
+// each its place, so nothing is sorted.  Bound by launches for a small chunk and by the edges' senders, read twice, for
+// a large one.  Four launches take the place of 18 tensor operations: together with mm_edge_csr for the pairs'
+// receivers and fewer device-to-host reads, a force call on 192 atoms goes from 1000 to 720 us, on 12,288 atoms in one
+// chunk from 5.07 to 4.66 ms.
 #define MM_TOPO_WORDS 1024   // bit words per workgroup of the prefix sum
 
 __global__ void __launch_bounds__(256) mm_topo_mark_kernel(const int* __restrict__ send, int E, int a, int b, int nt,
@@ -198,8 +198,8 @@ extern "C" int mm_chunk_topology(const int* send, int E, int a, int b, int nt, u
 // over each digit's tiles, and the scatter.  In the scatter a wave ranks 64 consecutive keys at a time among equal
 // digits with one ballot per bit, on top of counters in LDS, so equal keys stay in order.  Bound by launches (3 a pass)
 // and the scattered 8-byte writes.  The merge sort of 64-bit keys, histogram and prefix sum it replaces took 0.3 ms for
-// each of a low-memory call's ten sender lists (46,080 atoms, 0.8 M edges each): 22.3 -> 18.6 ms a call.  Unsorted pairs of
-// 12,288 atoms: 4.66 -> 4.41 ms a force call.
+// each of a low-memory call's ten sender lists (46,080 atoms, 0.8 M edges each): 22.3 -> 18.6 ms a call.  Unsorted
+// pairs of 12,288 atoms: 4.66 -> 4.41 ms a force call.
 #define MM_SORT_TILE 4096
 #define MM_SORT_ROUNDS (MM_SORT_TILE / 256)
 
@@ -255,8 +255,8 @@ __global__ void __launch_bounds__(256) mm_sort_scan_kernel(int* __restrict__ cou
 }
 
 // vals null: the positions 0 .. E - 1
-__global__ void __launch_bounds__(256) mm_sort_scatter_kernel(const int* __restrict__ keys, const int* __restrict__ vals,
-                                                              int E, int shift, int tiles,
+__global__ void __launch_bounds__(256) mm_sort_scatter_kernel(const int* __restrict__ keys,
+                                                              const int* __restrict__ vals, int E, int shift, int tiles,
                                                               const int* __restrict__ counts,
                                                               const int* __restrict__ totals,
                                                               int* __restrict__ keys_out, int* __restrict__ vals_out) {

@@ -14,8 +14,8 @@ __device__ __forceinline__ unsigned mm_load_u32(const unsigned char* p) {
 }
 
 // Slots of the distinct senders of each group of 4 consecutive receivers (spatially close in the Morton order, so
-// they share most senders): e_slot[e] = the slot of edge e's sender in its group (255: none, the sender found no slot or
-// the edge lies beyond the group's first 1024), g_send[group][slot] = the sender, g_n[group] = slots in use.
+// they share most senders): e_slot[e] = the slot of edge e's sender in its group (255: none, the sender found no slot
+// or the edge lies beyond the group's first 1024), g_send[group][slot] = the sender, g_n[group] = slots in use.
 // Once per chunk, for the 8 channel blocks of the backward (which hashed the senders 8 times before).
 #define MM_SLOT_HASH 2048
 extern "C" __global__ void __launch_bounds__(256)

@@ -1,5 +1,5 @@
-// generated by mace_onegpu/codegen.py -- harmonics of an edge direction and their tangential derivatives, and the
-// split of fp32 operands for fp16 matrix instructions
+// generated by mace_onegpu/codegen.py -- harmonics of an edge direction with their tangential
+// derivatives, and the split of fp32 operands for fp16 matrix instructions
 #pragma once
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));

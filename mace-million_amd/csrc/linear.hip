@@ -20,23 +20,23 @@
 // loaded coalesced by the whole workgroup, split once and written to LDS in operand order, one stage ahead of the
 // products; a stage is 96 matrix instructions per wave on four independent sums.  The weights are the first operand,
 // so that a lane ends with 4 consecutive columns of one row: 16-byte stores.
-// Bound: the bf16 products and the rows' traffic, which are near each other (40 x 40 components, 131,072 rows: 0.85 ms of
-// products at the 1.21 PFLOP/s of a large matrix product, 0.80 ms of traffic at the 4.67 TB/s of a large copy).  Before,
-// a workgroup staged the whole weight block (96 KiB) in LDS for 256 rows, and 16 waves read it again for every 16 rows:
-// LDS reads cost as much as the products, and nothing of a workgroup's start and end overlapped.  Measured (us, before
+// Bound: the bf16 products and the rows' traffic, which are near each other (40 x 40 components, 131,072 rows: 0.85 ms
+// of products at the 1.21 PFLOP/s of a large matrix product, 0.80 ms of traffic at the 4.67 TB/s of a large copy).
+// Before, a workgroup staged the whole weight block (96 KiB) in LDS for 256 rows, and 16 waves read it again for every
+// 16 rows: LDS reads cost as much as the products, and nothing of a workgroup's start and end overlapped.  Measured
+// (us, before
 // -> now; 16 components of 1 source, 16 of 2-3 sources, 40 of 1 source):
 //      192 rows:  12.5 -> < 9     27 -> < 10    12.6 -> < 9     (launch calls take 9 us)
 //    4,001 rows:   22 -> 20       40 -> 36       56 -> 39
 //   16,384 rows:   83 -> 56      174 -> 146     163 -> 149
 //  131,072 rows:  474 -> 452    1180 -> 1118   1167 -> 1134
 // Several sources: NS stages share each load of a source's weights, with NS stages of sums held.  4 stages from two
-// rounds of workgroups on (16 x 2 components, 131,072 rows: 849 us, 1115 us with 1 stage, 920 us with 2, 897 us with 3);
-// below that 1 stage, for more workgroups (1,024 rows: 11 us, 19 us with 4).
-// Weight blocks: plane p of block b at bf16 offset (3 b + p) 16384; element W[k][n], k = 32 t + 8 g + u,
-// n = 16 nt + i, at (((t * 8 + nt) * 4 + g) * 16 + i) * 8 + u, so that lane (i, g) reads its 8 k-values of step t
-// and tile nt as one 16-byte load, a wave 1 KiB.  The rows in LDS: 16-byte unit (row tile, plane, k / 8, row), the k / 8
-// groups 17 units apart: the 8-byte writes (32 lanes: one row) and the 16-byte reads (16 lanes: 16 rows) use every bank
-// once.
+// rounds of workgroups on (16 x 2 components, 131,072 rows: 849 us, 1115 us with 1 stage, 920 us with 2, 897 us with
+// 3); below that 1 stage, for more workgroups (1,024 rows: 11 us, 19 us with 4).
+// Weight blocks: plane p of block b at bf16 offset (3 b + p) 16384; element W[k][n], k = 32 t + 8 g + u, n = 16 nt + i,
+// at (((t * 8 + nt) * 4 + g) * 16 + i) * 8 + u, so that lane (i, g) reads its 8 k-values of step t and tile nt as one
+// 16-byte load, a wave 1 KiB.  The rows in LDS: 16-byte unit (row tile, plane, k / 8, row), the k / 8 groups 17 units
+// apart: the 8-byte writes (32 lanes: one row) and the 16-byte reads (16 lanes: 16 rows) use every bank once.
 // Components fastest in the grid: the workgroups of one row block run together, so an output row is written and an
 // input row read by neighbouring workgroups.
 #include "common.h"
@@ -183,7 +183,8 @@ __global__ void __launch_bounds__(64 * MM_LIN_NW, 2) mm_linear_kernel(MMLinArgs 
         // the last one this stage again: a load without a branch leaves the weights' loads countable)
         const bool last_s = s == NS - 1 || b + s + 1 == nst, last_q = q + 1 == n_src;
         const bool more = !(last_s && last_q && b + NS >= nst);
-        load(!more || !last_s ? b + s + (more ? 1 : 0) : last_q ? b + NS : b, !more || !last_s ? q : last_q ? 0 : q + 1);
+        load(!more || !last_s ? b + s + (more ? 1 : 0) : last_q ? b + NS : b,
+             !more || !last_s ? q : last_q ? 0 : q + 1);
         bf16x8 a[2][2][3];
         auto load_a = [&](int t) {
 #pragma unroll

@@ -44,9 +44,9 @@ extern "C" int mm_fill_i32(int* p, long n, int v, hipStream_t stream) {
 
 // ------------------------------------------------------------------------------------------------ species lists
 // Stable partition of rows 0..n-1 by species: lists[s * stride + j] = j-th row of species s, counts[s].
-// One workgroup per species, which takes its rows of tiles of 4,096 in order (4 consecutive rows per thread, a prefix sum
-// over the threads' counts).  Bound by the latency of a tile, 32 of them for a chunk of 131,072 receivers: 62 us, where
-// one workgroup with a segment of rows per thread, uncoalesced, took 264 us (9,216 receivers: 6 us, was 13).
+// One workgroup per species, which takes its rows of tiles of 4,096 in order (4 consecutive rows per thread, a prefix
+// sum over the threads' counts).  Bound by the latency of a tile, 32 of them for a chunk of 131,072 receivers: 62 us,
+// where one workgroup with a segment of rows per thread, uncoalesced, took 264 us (9,216 receivers: 6 us, was 13).
 #define MM_MAX_SPECIES 16
 __global__ void __launch_bounds__(1024) mm_species_lists_kernel(const int* __restrict__ spec, int n,
                                                                 int* __restrict__ lists, long stride,
@@ -132,10 +132,10 @@ extern "C" int mm_readout1(int n, const float* h1, long h_stride, const float* w
 // eat[i] += scale R2_i;  g_h2[i] = scale dR2/dh2.
 // 16 lanes per node: lane q takes the features q + 16 j, j = 0..7 (a group reads and writes 64 contiguous bytes per
 // access), and after a reduce-scatter over the group owns the hidden units q and q + 16.  W1 is staged in LDS, padded
-// with zeros to HM = 16 or 32 columns so that the loops have no conditions; with row stride HM + 4 the 16 lanes' 16-byte
-// reads use every bank once.  Bound by the latency of one node's chain: with 4 lanes per node, each holding all hidden
-// units behind a condition per unit, it took 27 us for 192 nodes, 32 us for 16,384 and
-// 63 us for 131,072; now 7, 11 and 40 us.
+// with zeros to HM = 16 or 32 columns so that the loops have no conditions; with row stride HM + 4 the 16 lanes'
+// 16-byte reads use every bank once.  Bound by the latency of one node's chain: with 4 lanes per node, each holding all
+// hidden units behind a condition per unit, it took 27 us for 192 nodes, 32 us for 16,384 and 63 us for 131,072; now 7,
+// 11 and 40 us.
 #define MM_RO2_HMAX 32
 #define MM_RO2_NODES 16   // nodes per 256-thread workgroup
 template <int HM>

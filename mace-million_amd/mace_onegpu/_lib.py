@@ -68,7 +68,8 @@ SIGNATURES = {
     **{f"mm_tpw_{n}_fwd": [P, I, P, P, P, L, P, L, P, L, P, L, P] for n in ("l1", "l2", "l0123")},
     **{f"mm_tpw_{n}_bwd": [P, I, P, P, P, L, P, L, P, L, P, L, P, L, P, L, P, L, P] for n in ("l1", "l2", "l0123")},
     **{f"mm_tpw_{n}_fwd_n": [L, P, I, P, P, P, L, P, L, P, L, P, L, P] for n in ("l1", "l2", "l0123")},
-    **{f"mm_tpw_{n}_bwd_n": [L, P, I, P, P, P, L, P, L, P, L, P, L, P, L, P, L, P, L, P] for n in ("l1", "l2", "l0123")},
+    **{f"mm_tpw_{n}_bwd_n": [L, P, I, P, P, P, L, P, L, P, L, P, L, P, L, P, L, P, L, P]
+       for n in ("l1", "l2", "l0123")},
     # symmetric contraction (generated)
     "mm_symc1_fwd": [I, P, L, P, P, P, L, P],
     "mm_symc2_fwd": [I, P, L, P, P, P, L, P],

@@ -594,15 +594,15 @@ def conv_source(tab, layer, need_gx, opts=None):
 #
 # Products from fp16 matrix instructions: each operand is the sum of two fp16 values, the second from the exact residual
 # (mm_split2_f16), and all four piece products are taken, side by side along the inner index: k-group 3 - 2 a - b of the
-# instruction holds piece a of Y and piece b of G.  (The instruction adds its k-groups in order: the small ones first give
-# a rounding error of 3.4e-8 of the sum's rms, the other way round 5.2e-8; one rounding is 2.5e-8.)  Two pieces hold 23
-# bits, an error of up to 2^-23 of the operand where fp32 has 2^-24, as long as the operand is in the upper part of the
-# fp16 range; both are scaled there by powers of two.  G, per channel, to below 2^15: 23 bits down to 2^-17 of the channel's
-# largest, 2^-40 of it below.  The harmonics: see mm_polar_operands.
+# instruction holds piece a of Y and piece b of G.  (The instruction adds its k-groups in order: the small ones first
+# give a rounding error of 3.4e-8 of the sum's rms, the other way round 5.2e-8; one rounding is 2.5e-8.)  Two pieces
+# hold 23 bits, an error of up to 2^-23 of the operand where fp32 has 2^-24, as long as the operand is in the upper part
+# of the fp16 range; both are scaled there by powers of two.  G, per channel, to below 2^15: 23 bits down to 2^-17 of
+# the channel's largest, 2^-40 of it below.  The harmonics: see mm_polar_operands.
 # What that costs is won back where the harmonics are evaluated and the products rounded.  Errors of the kernel alone
 # against 64 bits, same fp32 inputs, per-harmonic form -> here, water and four-species alloy: forces 1.50e-7 -> 1.42e-7
-# and 1.49e-7 -> 1.43e-7, dL/dX 1.24e-7 -> 1.25e-7 and 1.20e-7 -> 1.23e-7.  Of the whole layer-2 pass (24 chunks of 785 to
-# 16,857 receivers): pair forces 5.93e-7 -> 5.92e-7, dL/dh1 4.02e-7 -> 4.02e-7.
+# and 1.49e-7 -> 1.43e-7, dL/dX 1.24e-7 -> 1.25e-7 and 1.20e-7 -> 1.23e-7.  Of the whole layer-2 pass (24 chunks of 785
+# to 16,857 receivers): pair forces 5.93e-7 -> 5.92e-7, dL/dh1 4.02e-7 -> 4.02e-7.
 #
 # Measured (16,384 receivers x 90 edges, 1.47 M edges): 2.42 -> 2.20 ms, the edge gradient that reads its partials
 # 0.149 -> 0.028 ms, mm_sender_slots 9 us; the layer-2 pass of that chunk 4.50 -> 4.18 ms.
@@ -610,8 +610,8 @@ def conv_source(tab, layer, need_gx, opts=None):
 # about 0.2 ms of the matrix time is exposed, 0.25 ms goes into each receiver's operand B, 0.15 ms into the LDS adds.
 # Why this form: fp32 matrix instructions (16x16x1) hold the SIMD's vector ALU while they run (2.64 ms), the fp16 ones
 # run beside it; a tile of 16 edges x 16 channels is one instruction's rows and columns, so lane (edge group, channel)
-# holds four edges of its channel and reads X, W and G rows of 64 contiguous bytes; a third wave per SIMD does not fit (252
-# registers, of which 64 hold B), deeper prefetch spills.
+# holds four edges of its channel and reads X, W and G rows of 64 contiguous bytes; a third wave per SIMD does not fit
+# (252 registers, of which 64 hold B), deeper prefetch spills.
 def _polar_basis(u):
     """[n, 16] B_m of unit vectors: z-polynomial x sin^|m| theta x {cos, sin}(|m| phi), the functions that
     mm_polar_operands evaluates (value type)."""
@@ -658,8 +658,8 @@ __device__ __forceinline__ unsigned mm_load_u32(const unsigned char* p) {
 }
 
 // Slots of the distinct senders of each group of GROUP consecutive receivers (spatially close in the Morton order, so
-// they share most senders): e_slot[e] = the slot of edge e's sender in its group (255: none, the sender found no slot or
-// the edge lies beyond the group's first SLOT_EDGES), g_send[group][slot] = the sender, g_n[group] = slots in use.
+// they share most senders): e_slot[e] = the slot of edge e's sender in its group (255: none, the sender found no slot
+// or the edge lies beyond the group's first SLOT_EDGES), g_send[group][slot] = the sender, g_n[group] = slots in use.
 // Once per chunk, for the 8 channel blocks of the backward (which hashed the senders 8 times before).
 #define MM_SLOT_HASH 2048
 extern "C" __global__ void __launch_bounds__(256)
@@ -711,8 +711,8 @@ extern "C" int mm_sender_slots(const int* rowptr, int nC, const int* send, unsig
 }
 """
 
-POLAR_HEADER = """// generated by mace_onegpu/codegen.py -- harmonics of an edge direction and their tangential derivatives, and the
-// split of fp32 operands for fp16 matrix instructions
+POLAR_HEADER = """// generated by mace_onegpu/codegen.py -- harmonics of an edge direction with their tangential
+// derivatives, and the split of fp32 operands for fp16 matrix instructions
 #pragma once
 
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
@@ -1087,12 +1087,12 @@ TPW_TABLES = o3.COMPILED_TP_TABLES
 # receiver each.  With few receivers it is the parallelism that pays (501 receivers of 37 edges, shared against not:
 # forward l1 34 -> 14 us, l2 68 -> 26; backward l1 83 -> 27, l2 106 -> 62); with many, a wave streams contiguous rows of
 # W next to its neighbours' (16,384 receivers of 90 edges: forward l2 1,651 -> 1,559 us, backward 4,121 -> 4,015), but
-# each pays for its part of the reduction or its own receiver constants, so short receivers stay whole.
-# Mean edges per receiver from which they are shared, by the accumulators (forward) or constants (backward) per lane:
-# at 16,384 receivers forward l1 (32) 3 edges 39 -> 39 us, 7 83 -> 72; l2 (80) 7 199 -> 198, 13 306 -> 287; l0123 (99) 13
-# 718 -> 732, 20 1,037 -> 1,019; backward l1 (32) 3 85 -> 83, l2 (76) 7 407 -> 417, 13 689 -> 680.  A backward in path
-# groups (l0123) has several waves per receiver already: shared up to SHARE_WAVES of them (37 edges: 1,500 waves 139 ->
-# 94 us, 9,000 633 -> 619, 12,000 799 -> 817).
+# each pays for its part of the reduction or its own receiver constants, so short receivers stay whole. Mean edges per
+# receiver from which they are shared, by the accumulators (forward) or constants (backward) per lane: at 16,384
+# receivers forward l1 (32) 3 edges 39 -> 39 us, 7 83 -> 72; l2 (80) 7 199 -> 198, 13 306 -> 287; l0123 (99) 13 718 ->
+# 732, 20 1,037 -> 1,019; backward l1 (32) 3 85 -> 83, l2 (76) 7 407 -> 417, 13 689 -> 680.  A backward in path groups
+# (l0123) has several waves per receiver already: shared up to SHARE_WAVES of them (37 edges: 1,500 waves 139 -> 94 us,
+# 9,000 633 -> 619, 12,000 799 -> 817).
 SHARE_WAVES = 8192
 
 

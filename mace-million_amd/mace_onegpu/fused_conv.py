@@ -203,7 +203,10 @@ class _FusedConvFn(torch.autograd.Function):
                     W.stride(0), gYp, E * 16, gX, X.stride(0), stream())
         gY = None
         if ny:
-            gY = (gYp.sum(0) if desc.gy_parts > 1 else gYp[0])[:, :desc.nY] if E else torch.zeros(0, desc.nY, dtype=Y.dtype, device=Y.device)
+            if E:
+                gY = (gYp.sum(0) if desc.gy_parts > 1 else gYp[0])[:, :desc.nY]
+            else:
+                gY = torch.zeros(0, desc.nY, dtype=Y.dtype, device=Y.device)
         if nw and not E:
             gW = torch.zeros_like(W)
         return gX, gY, gW, None, None

@@ -1,5 +1,5 @@
-"""mm_chunk_topology against the tensor form of chunk_topology (run on the CPU): node list and local senders of chunks at
-the edges of its 32-atom words and 32,768-atom blocks, without edges, with every atom a sender, and bad senders."""
+"""mm_chunk_topology against the tensor form of chunk_topology (run on the CPU): node list and local senders of chunks
+at the edges of its 32-atom words and 32,768-atom blocks, without edges, with every atom a sender, and bad senders."""
 import pytest
 import torch
 

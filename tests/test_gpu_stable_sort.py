@@ -1,5 +1,5 @@
-"""mm_stable_sort and the CSR of its keys against torch's stable sort: sizes around a wave, a tile and one, two and three
-digits, keys that are all equal and keys that miss most of the range; exact."""
+"""mm_stable_sort and the CSR of its keys against torch's stable sort: sizes around a wave, a tile and one, two and
+three digits, keys that are all equal and keys that miss most of the range; exact."""
 import pytest
 import torch
 
