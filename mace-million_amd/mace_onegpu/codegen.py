@@ -604,10 +604,11 @@ def conv_source(tab, layer, need_gx, opts=None):
 # and 1.49e-7 -> 1.43e-7, dL/dX 1.24e-7 -> 1.25e-7 and 1.20e-7 -> 1.23e-7.  Of the whole layer-2 pass (24 chunks of 785
 # to 16,857 receivers): pair forces 5.93e-7 -> 5.92e-7, dL/dh1 4.02e-7 -> 4.02e-7.
 #
-# Measured (16,384 receivers x 90 edges, 1.47 M edges): 2.42 -> 2.20 ms, the edge gradient that reads its partials
-# 0.149 -> 0.028 ms, mm_sender_slots 9 us; the layer-2 pass of that chunk 4.50 -> 4.18 ms.
+# Measured (16,384 receivers x 90 edges, 1.47 M edges): 2.42 -> 2.17 ms, the edge gradient that reads its partials
+# 0.149 -> 0.028 ms, mm_sender_slots 9 us; the layer-2 pass of that chunk 4.39 -> 3.97 ms.
 # Bound by VALU issue (the spline evaluation, the two products with X and W, the operand split) at 2 waves per SIMD:
-# about 0.2 ms of the matrix time is exposed, 0.25 ms goes into each receiver's operand B, 0.15 ms into the LDS adds.
+# 0.65 of the cycles issue a VALU instruction.  Left out in timing probes: the matrix instructions 0.23 ms, the LDS adds
+# 0.17 ms, evaluating and splitting each receiver's operand B 0.07 ms.
 # Why this form: fp32 matrix instructions (16x16x1) hold the SIMD's vector ALU while they run (2.64 ms), the fp16 ones
 # run beside it; a tile of 16 edges x 16 channels is one instruction's rows and columns, so lane (edge group, channel)
 # holds four edges of its channel and reads X, W and G rows of 64 contiguous bytes; a third wave per SIMD does not fit
