@@ -70,16 +70,17 @@ class System:
     def _mask_words(self, brute, ncells):
         """Mask words per atom in which the count pass leaves its decisions to the fill pass: half as many again as
         the mean number of candidates needs (denser cells are tested twice).  0 (every candidate is tested twice)
-        where the masks would take more than the pair list of an even box and more than a sixteenth of the free
+        where the masks would take more than 64 MB, than the pair list of an even box and than a sixteenth of the free
         memory, or more than 2 GB."""
         if self.N == 0:
             return 0
         T = self.N if brute else 27 * self.N / ncells
         cap = int(1.5 * T / 64) + 2
         size = 8 * cap * self.N
-        pairs = self.N * 4.19 * self.r_max ** 3 * self.N / float(np.prod(self.box))
-        if size > 2 << 30 or size > max(4 * pairs, 64 << 20) and 16 * size > torch.cuda.mem_get_info(self.device)[0]:
-            return 0
+        if size > 64 << 20:
+            pairs = self.N * 4.19 * self.r_max ** 3 * self.N / float(np.prod(self.box))
+            if size > 2 << 30 or size > 4 * pairs and 16 * size > torch.cuda.mem_get_info(self.device)[0]:
+                return 0
         return cap
 
     def build_neighbors(self, r_cut=None):
